@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/swr.h"
+#include "swr_raster_launch.hpp"
 #include "swr_srgb.hpp"
 #include "swr_kernels.hip"
 #include "swr_batch.hip"
@@ -864,44 +865,6 @@ void enqueue_radix_pass(const uint32_t *kIn, const uint32_t *vIn, const uint32_t
   }
 }
 
-// Arguments of one raster launch over tiles [tLo, tHi) of draws [lo, hi).
-struct RasterArgs {
-  const DrawParams *params;
-  const uint32_t *tileBase;
-  int lo, hi;
-  uint32_t tLo, tHi;
-  uint32_t *counter;
-  const TriRecord *rec;
-  const int *poly;
-  const uint32_t *bin;  // NULL: the unbinned pass
-  const uint32_t *ts, *te;
-  const uint32_t *split;
-  uint32_t segT;
-  int tail;  // with bin: each tile also walks the slots from *split on
-};
-
-template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL>
-void launch_raster_batch(dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
-  hipLaunchKernelGGL((raster_batch_kernel<MS, FCOL, FTEX, XF, LEVEL>), grid, block, 0, s, a.params, a.tileBase, a.lo,
-                     a.hi, a.tLo, a.tHi, a.counter, a.rec, a.poly, a.bin, a.ts, a.te, a.split, a.segT,
-                     a.tail);
-}
-
-// The raster kernel of variant v (variant_of).
-template <bool XF, int LEVEL>
-void launch_raster_variant(int v, dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
-  switch (v & 7) {
-    case 0: launch_raster_batch<1, false, false, XF, LEVEL>(grid, block, s, a); break;
-    case 1: launch_raster_batch<1, false, true, XF, LEVEL>(grid, block, s, a); break;
-    case 2: launch_raster_batch<1, true, false, XF, LEVEL>(grid, block, s, a); break;
-    case 3: launch_raster_batch<1, true, true, XF, LEVEL>(grid, block, s, a); break;
-    case 4: launch_raster_batch<4, false, false, XF, LEVEL>(grid, block, s, a); break;
-    case 5: launch_raster_batch<4, false, true, XF, LEVEL>(grid, block, s, a); break;
-    case 6: launch_raster_batch<4, true, false, XF, LEVEL>(grid, block, s, a); break;
-    default: launch_raster_batch<4, true, true, XF, LEVEL>(grid, block, s, a); break;
-  }
-}
-
 // Setup and tile-count prefix sum of one segment (off[T] = pair count).
 // With a pair capacity `cap` > 0 the scan also builds the emission index for
 // it (enqueue_back is then told so); `zeroed`: cnt[T] is already zero.
@@ -999,13 +962,8 @@ int enqueue_back(DeviceCtx *c, Pipeline &pipe, const BatchLayout &L, const Batch
       a.split = split;
       a.segT = sg.T;
       const int var = variant_of(L.P[sg.first + lo]);
-      switch (var & 8 ? -1 : var >> 4) {
-        case -1: launch_raster_variant<true, 0>(var, dim3(wgs), block, s, a); break;
-        case 3: launch_raster_variant<false, 3>(var, dim3(wgs), block, s, a); break;
-        case 2: launch_raster_variant<false, 2>(var, dim3(wgs), block, s, a); break;
-        case 1: launch_raster_variant<false, 1>(var, dim3(wgs), block, s, a); break;
-        default: launch_raster_variant<false, 0>(var, dim3(wgs), block, s, a); break;
-      }
+      if (var >> 4 && !(var & 8)) launch_raster_common(var, dim3(wgs), block, s, a);
+      else launch_raster_general(var, dim3(wgs), block, s, a);
     }
   } else if (es) {
     SWR_HIP_CHECK(hipEventRecord(es->ev[EV_BIN], s));

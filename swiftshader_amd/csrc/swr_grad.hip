@@ -28,6 +28,7 @@
 
 #include "swr_device.hpp"
 #include "swr_params.hpp"
+#include "swr_shade.hpp"
 
 namespace swr {
 

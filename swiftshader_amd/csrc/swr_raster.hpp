@@ -1,0 +1,737 @@
+// swr_raster.hpp -- the tile rasteriser (gfx950).
+//
+//   raster_batch_kernel  one workgroup per screen tile, one wave per 8x8
+//                    block, one pixel per lane (a 2x2 quad in lanes
+//                    4k..4k+3); the block's depth / stencil / colour live in
+//                    registers while the wave walks the tile's primitive
+//                    list in order: coverage, stencil, depth, shading, blend.
+//
+// The kernel's variants are compiled in translation units of their own
+// (swr_raster_common.hip, swr_raster_general.hip), in parallel with the rest.
+//
+// Reference semantics: src/Device/QuadRasterizer.cpp,
+// src/Pipeline/PixelRoutine.cpp, src/Pipeline/PixelProgram.cpp,
+// src/Pipeline/SamplerCore.cpp.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "swr_device.hpp"
+#include "swr_params.hpp"
+#include "swr_raster_launch.hpp"
+#include "swr_shade.hpp"
+#include "swr_srgb.hpp"
+
+namespace swr {
+
+// Standard 4x sample locations relative to the pixel centre
+// (Constants.hpp:26-47) and their 28.4 offsets Xf/Yf (Constants.cpp:291-297).
+__device__ __constant__ const float kSampleX[4] = {-0.125f, 0.375f, -0.375f, 0.125f};
+__device__ __constant__ const float kSampleY[4] = {-0.375f, -0.125f, 0.125f, 0.375f};
+__device__ __constant__ const int kXf[4] = {-2, 6, -6, 2};
+__device__ __constant__ const int kYf[4] = {-6, -2, 2, 6};
+
+// D16 compares and stores Min(Max(Round(z * 0xFFFF), 0), 0xFFFF) of the
+// clamped depth (PixelRoutine.cpp:506-510, 686-711; Round is to nearest even).
+__device__ __forceinline__ float d16_value(float z) {
+  return rr_min(rr_max(__builtin_rintf(z * 65535.0f), 0.0f), 65535.0f);
+}
+
+// B8G8R8A8 keeps R and B exchanged in memory (PixelRoutine.cpp:1091-1110,
+// 2130-2143): the tile holds R8G8B8A8 order.
+__device__ __forceinline__ uint32_t bgra_swap(int bgra, uint32_t v) {
+  return bgra ? (v & 0xFF00FF00u) | ((v >> 16) & 0xFFu) | ((v & 0xFFu) << 16) : v;
+}
+
+// ---------------------------------------------------------------------------
+// Tile rasteriser
+// ---------------------------------------------------------------------------
+// Work decomposition: one workgroup per 16x16 bin, one wavefront per 8x8
+// block of the bin, one pixel per lane (lanes 4k..4k+3 form a 2x2 quad).
+// Each wave walks the bin's triangle list in API order, 64 entries at a
+// time: every lane computes the exact 8x8 coverage mask of one triangle
+// (triangle-parallel), a ballot compacts the triangles that cover the
+// block, and the wave then applies them one by one (pixel-parallel) to the
+// block's depth / stencil / colour, which stay in registers throughout.
+//
+// Coverage is the reference's span rule evaluated per sample point.  The
+// reference walks each edge with an exact integer DDA that stores
+// x = ceil(Xe(y) / 16) for rows [ceil(Y1/16), ceil(Y2/16)) into the left or
+// right span, later edges overwriting earlier ones (SetupRoutine.cpp:
+// 550-621), and a sample is covered iff left <= x < right
+// (QuadRasterizer.cpp:181-206).  With
+//   E(x, y) = DY * (16 x - X1) - DX * (16 y - Y1),   DY = Y2 - Y1 > 0,
+// "ceil(Xe/16) <= x" is exactly E >= 0 and "x < ceil(Xe/16)" is exactly
+// E < 0, so the span test becomes two integer sign tests per sample.  E at
+// the block origin is formed in 64 bits and clamped to +-2^30: beyond that
+// its sign cannot change inside the block, and the 32-bit steps are exact.
+
+struct LaneEdge {
+  int e;      // E at the block origin (clamped)
+  int ex;     // dE / dx (16 DY > 0)
+  int ey;     // dE / dy (-16 DX)
+  int y1, y2; // rows the edge spans
+  int right;  // writes the right span
+};
+
+__device__ __forceinline__ LaneEdge lane_edge(int Xa, int Ya, int Xb, int Yb, int ox, int oy) {
+  LaneEdge E;
+  const bool swap = Yb < Ya;
+  const int X1 = swap ? Xb : Xa, X2 = swap ? Xa : Xb;
+  const int Y1 = swap ? Yb : Ya, Y2 = swap ? Ya : Yb;
+  const int DX = X2 - X1, DY = Y2 - Y1;
+  E.y1 = (Y1 + 15) >> 4;  // a horizontal edge gets y1 == y2 and spans no row
+  E.y2 = (Y2 + 15) >> 4;
+  long long v = (long long)DY * (long long)(16 * ox - X1) - (long long)DX * (long long)(16 * oy - Y1);
+  const long long lim = 1ll << 30;
+  E.e = (int)(v > lim ? lim : (v < -lim ? -lim : v));
+  E.ex = 16 * DY;
+  E.ey = -16 * DX;
+  E.right = swap ? 1 : 0;
+  return E;
+}
+
+// Coverage mask (bit r*8+c = pixel (ox+c, oy+r)) of polygon (X, Y, n) for
+// the sample at 28.4 offset (xo, yo), before the scissor mask is applied.
+template <typename VFetch>
+__device__ __forceinline__ uint64_t block_coverage(const VFetch &vtx, int n, int d, int xo, int yo, int ox, int oy) {
+  int Lv[8], Lx[8], Rv[8], Rx[8];
+#pragma unroll
+  for (int r = 0; r < 8; r++) { Lv[r] = -1; Lx[r] = 0; Rv[r] = 0; Rx[r] = 0; }
+  for (int i = 0; i < n; i++) {
+    int ia = i + 1 - d, ib = i + d;
+    ia = ia >= n ? ia - n : ia;
+    ib = ib >= n ? ib - n : ib;
+    int Xa, Ya, Xb, Yb;
+    vtx(ia, Xa, Ya);
+    vtx(ib, Xb, Yb);
+    const LaneEdge E = lane_edge(Xa - xo, Ya - yo, Xb - xo, Yb - yo, ox, oy);
+    // Rows of the block the edge spans, as a bit mask, routed to the left or
+    // right span; each row then takes (E, dE/dx) under a select mask
+    // (bitfield insert), so the update has no branches.
+    const int r1 = min(max(E.y1 - oy, 0), 8), r2 = min(max(E.y2 - oy, 0), 8);
+    const uint32_t rows = (0xFFu << r1) & ~(0xFFu << r2) & 0xFFu;
+    const uint32_t rowsR = E.right ? rows : 0u, rowsL = rows ^ rowsR;
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+      const int v = E.e + E.ey * r;
+      const uint32_t ml = 0u - ((rowsL >> r) & 1u), mr = 0u - ((rowsR >> r) & 1u);
+      Lv[r] = (int)(((uint32_t)v & ml) | ((uint32_t)Lv[r] & ~ml));
+      Lx[r] = (int)(((uint32_t)E.ex & ml) | ((uint32_t)Lx[r] & ~ml));
+      Rv[r] = (int)(((uint32_t)v & mr) | ((uint32_t)Rv[r] & ~mr));
+      Rx[r] = (int)(((uint32_t)E.ex & mr) | ((uint32_t)Rx[r] & ~mr));
+    }
+  }
+  uint64_t mask = 0;
+#pragma unroll
+  for (int r = 0; r < 8; r++) {
+    // Covered iff lv >= 0 && rv < 0, i.e. the sign bit of (rv & ~lv).
+    int lv = Lv[r] + 7 * Lx[r], rv = Rv[r] + 7 * Rx[r];
+    uint32_t bits = 0;
+#pragma unroll
+    for (int c = 7; c >= 0; c--) {
+      bits = (bits << 1) | ((uint32_t)(rv & ~lv) >> 31);
+      lv -= Lx[r];
+      rv -= Rx[r];
+    }
+    mask |= (uint64_t)bits << (8 * r);
+  }
+  return mask;
+}
+
+template <int MS, bool FCOL>
+struct PixelState {
+  float zb[MS];
+  uint32_t sb[MS];
+  uint32_t cb[FCOL ? 1 : MS];
+  float4 cf[FCOL ? MS : 1];
+  uint32_t id[FCOL ? MS : 1];  // primitive_id record (float targets only)
+};
+
+// Pixel of lane `l` inside its 8x8 block: lanes 4k..4k+3 form the 2x2 quad
+// k, quads in row-major order over the block.
+__device__ __forceinline__ int lane_cx(int l) { return 2 * ((l >> 2) & 3) + (l & 1); }
+__device__ __forceinline__ int lane_cy(int l) { return 2 * (l >> 4) + ((l >> 1) & 1); }
+
+// Blend a shaded colour into the samples of this lane's pixel selected by
+// xMask, then write (PixelRoutine.cpp:1617-2936).
+// FAST: blending, when on, is SRC_ALPHA, ONE_MINUS_SRC_ALPHA, ADD.
+template <int MS, bool FCOL, bool XF, bool FAST = false>
+__device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, FCOL> &S, float4 s, int xMask,
+                                            uint32_t tri) {
+#pragma unroll
+  for (int q = 0; q < MS; q++) {
+    if (!((xMask >> q) & 1)) continue;
+    float4 dst;
+    if (FCOL) {
+      dst = S.cf[FCOL ? q : 0];
+    } else {
+      const uint32_t p = S.cb[FCOL ? 0 : q];
+      dst = make_float4(unorm8_to_float(p & 0xFFu), unorm8_to_float((p >> 8) & 0xFFu),
+                        unorm8_to_float((p >> 16) & 0xFFu), unorm8_to_float(p >> 24));
+      if ((XF && P.colorSRGB) && P.blendEnable) {  // blended in linear space (PixelRoutine.cpp:1811-1827)
+        dst.x = srgb_to_linear(dst.x);
+        dst.y = srgb_to_linear(dst.y);
+        dst.z = srgb_to_linear(dst.z);
+      }
+    }
+    float4 o = P.blendEnable ? (FAST ? blend_src_alpha(s, dst) : alpha_blend<XF>(P, s, dst)) : s;
+    if (!FCOL && (XF && P.colorSRGB)) {  // writeColor encodes R, G, B first (PixelRoutine.cpp:1963-1969)
+      o.x = linear_to_srgb(o.x);
+      o.y = linear_to_srgb(o.y);
+      o.z = linear_to_srgb(o.z);
+    }
+    // Masked channels keep their value (selects, not branches).
+    if (FCOL) {
+      float4 &c = S.cf[FCOL ? q : 0];
+      c.x = (P.colorMask & 1) ? o.x : c.x;
+      c.y = (P.colorMask & 2) ? o.y : c.y;
+      c.z = (P.colorMask & 4) ? o.z : c.z;
+      c.w = (P.colorMask & 8) ? o.w : c.w;
+      S.id[FCOL ? q : 0] = tri - (uint32_t)P.triBase + 1u;
+    } else {
+      const uint32_t wm = ((P.colorMask & 1) ? 0x000000FFu : 0u) | ((P.colorMask & 2) ? 0x0000FF00u : 0u) |
+                          ((P.colorMask & 4) ? 0x00FF0000u : 0u) | ((P.colorMask & 8) ? 0xFF000000u : 0u);
+      const uint32_t o8 = float_to_unorm8(o.x) | (float_to_unorm8(o.y) << 8) | (float_to_unorm8(o.z) << 16) |
+                          (float_to_unorm8(o.w) << 24);
+      S.cb[FCOL ? 0 : q] = (S.cb[FCOL ? 0 : q] & ~wm) | (o8 & wm);
+    }
+  }
+}
+
+constexpr int kQueue = 64;  // deferred-shading queue entries per wave
+
+// One screen tile of draw P: `bin` is the tile's index in the draw's tile
+// grid, [start, end) its range of the sorted (tile, primitive) list.  The
+// workgroup has one wave per 8x8 block of the tile.
+// LEVEL 1: the draw has no stencil and no depth bias, tests and writes
+// depth and writes all four colour channels (the checks below fold away).
+// LEVEL 2 (3): also the common shading state with REPEAT (CLAMP_TO_EDGE)
+// addressing (shade's FA, blend_write's FAST).
+template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL>
+__device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32_t start, uint32_t end0,
+                                            const TriRecord *__restrict__ rec, const int *__restrict__ poly,
+                                            const uint32_t *__restrict__ binTri) {
+  constexpr bool SIMPLE = LEVEL >= 1, FAST = LEVEL >= 2;
+  constexpr int FA = LEVEL >= 2 ? LEVEL - 2 : -1;
+  const bool stencilActive = !SIMPLE && P.stencilActive, stencilWrite = !SIMPLE && P.stencilWrite;
+  const bool depthBias = !SIMPLE && P.depthBias, depthTest = SIMPLE || P.depthTest;
+  const bool depthWrite = SIMPLE || P.depthWrite;
+  const int colorMask = SIMPLE ? 15 : P.colorMask;
+  // Per-wave queue of fragments that passed the tests and await shading,
+  // in API order: primitive, owner lane | sample mask << 8, shaded colour.
+  __shared__ uint32_t qTri[4][kQueue];
+  __shared__ uint32_t qPix[4][kQueue];
+  __shared__ float4 qCol[4][kQueue];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int bx = bin % P.tilesX, by = bin / P.tilesX;
+  const int bw = P.tileW >> 3;  // 8x8 blocks per tile row
+  const int ox = bx * P.tileW + 8 * (wave % bw), oy = by * P.tileH + 8 * (wave / bw);
+  const int cx = lane_cx(lane), cy = lane_cy(lane);
+  const int px = ox + cx, py = oy + cy;
+  const int myBit = cy * 8 + cx;
+
+  // A block outside the scissor walks no list (no early return: the
+  // workgroup reduces its counters together at the end).
+  const bool waveActive = !(ox >= P.sx1 || oy >= P.sy1 || ox + 8 <= P.sx0 || oy + 8 <= P.sy0);
+  const uint32_t end = waveActive ? end0 : start;
+
+  uint64_t scissorMask = 0;
+  {
+    uint32_t cols = 0;
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+      if (ox + c >= P.sx0 && ox + c < P.sx1) cols |= 1u << c;
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+      if (oy + r >= P.sy0 && oy + r < P.sy1) scissorMask |= (uint64_t)cols << (8 * r);
+  }
+  const bool inside = (scissorMask >> myBit) & 1;
+
+  PixelState<MS, FCOL> S;
+#pragma unroll
+  for (int q = 0; q < MS; q++) {
+    S.zb[q] = 0.0f;
+    S.sb[q] = 0;
+    if (!FCOL) S.cb[FCOL ? 0 : q] = 0;
+    if (FCOL) S.cf[FCOL ? q : 0] = make_float4(0, 0, 0, 0);
+    if (FCOL) S.id[FCOL ? q : 0] = 0;
+    if (!inside) continue;
+    if (FCOL && P.primId)
+      S.id[FCOL ? q : 0] =
+          *reinterpret_cast<const uint32_t *>(P.primId + q * P.primIdSlice + (long long)py * P.primIdPitch + 4ll * px);
+    if (depthTest || (XF && P.depthBounds))  // D16 holds the float of its integer (readDepth16, PixelRoutine.cpp:466-481)
+      S.zb[q] = (XF && P.depth16) ? (float)*reinterpret_cast<const uint16_t *>(P.depth + q * P.depthSlice +
+                                                                        (long long)py * P.depthPitch + 2ll * px)
+                          : *reinterpret_cast<const float *>(P.depth + q * P.depthSlice +
+                                                             (long long)py * P.depthPitch + 4ll * px);
+    if (stencilActive) S.sb[q] = (uint8_t)P.stencil[q * P.stencilSlice + (long long)py * P.stencilPitch + px];
+    if (colorMask) {
+      if (FCOL)
+        S.cf[FCOL ? q : 0] =
+            *reinterpret_cast<const float4 *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 16ll * px);
+      else
+        S.cb[FCOL ? 0 : q] = bgra_swap(
+            (XF && P.colorBGRA),
+            *reinterpret_cast<const uint32_t *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 4ll * px));
+    }
+  }
+
+  // Hierarchical depth: a primitive whose evaluated depth is bounded below
+  // by zlo cannot pass LESS (LESS_OR_EQUAL) anywhere in a block whose
+  // largest stored depth is <= zlo (< zlo).  Only when a failing fragment
+  // has no side effect (no stencil writes).
+  const bool hiz = depthTest && !stencilWrite && (P.depthCompare == 1 || P.depthCompare == 3);
+
+  unsigned long long occl = 0;
+  uint32_t nTests = 0, nCovers = 0, nShaded = 0;  // statistics (profiling only)
+  int qCount = 0;           // wave-uniform queue length
+  uint64_t myEntries = 0;   // queue slots holding fragments of this lane's pixel
+
+  auto flush = [&]() __attribute__((always_inline)) {
+    // Shade the queued fragments, one per lane...
+    if (lane < qCount) {
+      const uint32_t t = qTri[wave][lane];
+      const uint32_t pix = qPix[wave][lane];
+      const int l = (int)(pix & 63u);
+      qCol[wave][lane] = shade<FCOL, FTEX, XF, FA>(P, rec[t], ox + lane_cx(l), oy + lane_cy(l));
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // ...then blend them into their pixels in queue (API) order.
+    uint64_t m = myEntries;
+    while (m) {
+      const int k = __builtin_ctzll(m);
+      m &= m - 1;
+      blend_write<MS, FCOL, XF, FAST>(P, S, qCol[wave][k], (int)(qPix[wave][k] >> 8), qTri[wave][k]);
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    myEntries = 0;
+    qCount = 0;
+  };
+
+  // Largest stored depth of the block (+inf when any is NaN): a primitive
+  // whose depth is bounded below by zl cannot pass where zl >= it (LESS) or
+  // zl > it (LESS_OR_EQUAL).
+  auto block_zmax = [&]() __attribute__((always_inline)) {
+    float v = -__builtin_inff();
+    bool nan = false;
+    if (inside) {
+#pragma unroll
+      for (int q = 0; q < MS; q++) {
+        v = fmaxf(v, S.zb[q]);
+        nan |= S.zb[q] != S.zb[q];
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+    return __ballot(nan) ? __builtin_inff() : v;
+  };
+
+  // One batch of up to 64 candidates in list order: each lane computes the
+  // exact coverage of its primitive; then the covering primitives are
+  // applied in list order.  A candidate waited in the ring while earlier
+  // ones wrote depth, so its depth bound zl is tested again first.
+  auto process_chunk = [&](bool act, uint32_t tid, float zl) __attribute__((always_inline)) {
+    if (hiz) {
+      const float zmax = block_zmax();
+      act = act && !(P.depthCompare == 1 ? zl >= zmax : zl > zmax);
+    }
+    // ---- triangle-parallel coverage of this block ----
+    uint32_t mlo[MS], mhi[MS];
+    int flags = 0;
+    float x0 = 0, y0 = 0, zA = 0, zB = 0, zC = 0, zBias = 0;
+#pragma unroll
+    for (int q = 0; q < MS; q++) { mlo[q] = 0; mhi[q] = 0; }
+    if (act) {
+      const int4 *rp = reinterpret_cast<const int4 *>(rec + tid);
+      const int4 h0 = rp[0];  // nflags, yMin, yMax, xMin
+      const int4 h1 = rp[1];  // xMax, X0, X1, X2
+      const int4 h2 = rp[2];  // Y0, Y1, Y2, zlo
+      const float4 h3 = reinterpret_cast<const float4 *>(rp)[3];  // x0, y0, zA, zB
+      const float4 h4 = reinterpret_cast<const float4 *>(rp)[4];  // zC, zBias, wA, wB
+      const int n = h0.x & 0xFF, d = (h0.x >> 8) & 1;
+      flags = h0.x >> 8;
+      x0 = h3.x; y0 = h3.y; zA = h3.z; zB = h3.w; zC = h4.x; zBias = h4.y;
+      const int *pp = poly + (size_t)tid * (2 * kMaxPolygon);
+      auto vtx = [&](int i, int &Xo, int &Yo) {
+        if (n == 3) {
+          // Mask selects: a conditional pick among the components of one
+          // vector would become an indexed access through scratch memory.
+          const int m0 = -(int)(i == 0), m1 = -(int)(i == 1), m2 = -(int)(i == 2);
+          Xo = (h1.y & m0) | (h1.z & m1) | (h1.w & m2);
+          Yo = (h2.x & m0) | (h2.y & m1) | (h2.z & m2);
+        } else {
+          Xo = pp[i];
+          Yo = pp[kMaxPolygon + i];
+        }
+      };
+#pragma unroll
+      for (int q = 0; q < MS; q++) {
+        if (!((P.msMask >> q) & 1)) continue;
+        const int xo = (MS > 1) ? kXf[q] : 0, yo = (MS > 1) ? kYf[q] : 0;
+        const uint64_t m = block_coverage(vtx, n, d, xo, yo, ox, oy) & scissorMask;
+        mlo[q] = (uint32_t)m;
+        mhi[q] = (uint32_t)(m >> 32);
+      }
+    }
+    uint32_t anyBits = 0;
+#pragma unroll
+    for (int q = 0; q < MS; q++) anyBits |= mlo[q] | mhi[q];
+    uint64_t todo = __ballot(anyBits != 0);
+    nCovers += anyBits != 0 ? 1u : 0u;
+
+    // ---- pixel-parallel tests, in list order ----
+    while (todo) {
+      const int j = __builtin_ctzll(todo);
+      todo &= todo - 1;
+      int cMask = 0;  // bit q: sample q of this lane's pixel is covered
+#pragma unroll
+      for (int q = 0; q < MS; q++) {
+        const uint32_t lo = __builtin_amdgcn_readlane(mlo[q], j), hi = __builtin_amdgcn_readlane(mhi[q], j);
+        const uint32_t word = myBit < 32 ? lo : hi;
+        cMask |= (int)((word >> (myBit & 31)) & 1u) << q;
+      }
+      const int fl = __builtin_amdgcn_readlane(flags, j);
+      const StencilParams &SP = (fl & 2) ? P.front : P.back;
+
+      int sMask = cMask, zMask = cMask;
+      if (stencilActive && cMask) {
+#pragma unroll
+        for (int q = 0; q < MS; q++)
+          if (((cMask >> q) & 1) && !stencil_compare(SP, S.sb[q])) sMask &= ~(1 << q);
+      }
+      if (XF && P.alphaToCoverage) {
+        // The reference shades before the depth test and keeps sample q
+        // only where !(alpha < a2c[q]) (alphaTest / alphaToCoverage,
+        // PixelProgram.cpp:243-259, PixelRoutine.cpp:317-337, 643-657); the
+        // alpha is clamped when the colour attachment is UNORM.  The
+        // fragment is shaded again, identically, if it reaches the queue.
+        if (cMask) {
+          const uint32_t tj = __builtin_amdgcn_readlane(tid, j);
+          const float a = shade<FCOL, FTEX, XF, FA>(P, rec[tj], px, py, P.color != nullptr).w;
+          int aMask = 0;
+#pragma unroll
+          for (int q = 0; q < MS; q++)
+            if (!(a < P.a2c[q])) aMask |= 1 << q;
+          cMask &= aMask;
+        }
+        sMask &= cMask;
+        zMask &= cMask;
+      }
+      float zq[MS];
+      if (depthTest) {
+        const float xf = (float)px - rdl(x0, j);  // xFragment (PixelRoutine.cpp:125)
+        const float yf = (float)py - rdl(y0, j);  // yFragment (QuadRasterizer.cpp:126)
+        const float a = rdl(zA, j), b = rdl(zB, j), c = rdl(zC, j);
+        const float zbias = depthBias ? rdl(zBias, j) : 0.0f;
+        zMask = 0;
+#pragma unroll
+        for (int q = 0; q < MS; q++) {
+          const float yy = (MS > 1) ? yf + kSampleY[q] : yf;
+          const float xx = (MS > 1) ? xf - kSampleX[q] : xf;
+          const float Dz = c + yy * b;
+          float z = xx * a + Dz;
+          if (depthBias) z = z + zbias;  // PixelRoutine.cpp:141-144, before the clamp
+          z = rr_min(rr_max(z, P.depthClampLo), P.depthClampHi);  // clampDepth
+          if ((XF && P.depth16)) z = d16_value(z);
+          zq[q] = z;
+          const float zb = S.zb[q];
+          // The compare op without branches: one of zb <= z, zb < z, zb == z
+          // or true, inverted for LESS, LESS_OR_EQUAL, NOT_EQUAL and NEVER.
+          const bool le = zb <= z, lt = zb < z, eq = zb == z;
+          const bool pr = P.zPred == 0 ? le : (P.zPred == 1 ? lt : (P.zPred == 2 ? eq : true));
+          if (pr != (P.zInv != 0)) zMask |= 1 << q;
+        }
+        zMask &= cMask;
+        if (stencilActive) zMask &= sMask;
+      }
+      if (XF && P.depthBounds && cMask) {
+        // depthBoundsTest (PixelRoutine.cpp:576-641) on the stored depth, D16
+        // as its code / 0xFFFF. With the depth test off the coverage loses
+        // the sample while zMask keeps it, so the occlusion count does too.
+        int bMask = 0;
+#pragma unroll
+        for (int q = 0; q < MS; q++) {
+          const float zs = P.depth16 ? S.zb[q] * (1.0f / 65535.0f) : S.zb[q];
+          if (P.depthBoundsMin <= zs && zs <= P.depthBoundsMax) bMask |= 1 << q;
+        }
+        if (depthTest) zMask &= bMask;
+        else cMask &= bMask;
+      }
+      if (stencilWrite && cMask) {
+#pragma unroll
+        for (int q = 0; q < MS; q++) {
+          if (!((cMask >> q) & 1)) continue;
+          int op;
+          if (!((sMask >> q) & 1)) op = SP.failOp;
+          else if (depthTest && !((zMask >> q) & 1)) op = SP.depthFailOp;
+          else op = SP.passOp;
+          const uint32_t bv = S.sb[q];
+          uint32_t nv = stencil_apply_op(bv, op, SP.reference);
+          if (SP.useWriteMask) nv = (nv & SP.writeMask) | (bv & ~SP.writeMask);
+          S.sb[q] = nv & 0xFFu;
+        }
+      }
+      if (depthWrite) {
+#pragma unroll
+        for (int q = 0; q < MS; q++)
+          if ((zMask >> q) & 1) S.zb[q] = zq[q];
+      }
+      occl += __builtin_popcount((unsigned)(zMask & sMask));
+      if (!colorMask) continue;
+      int xMask = depthTest ? zMask : cMask;
+      if (stencilActive) xMask &= sMask;
+      const uint64_t need = __ballot(xMask != 0);
+      if (!need) continue;
+      // Queue the fragments that write colour; shading is deferred so that
+      // it runs with every lane busy.
+      const int cnt = __builtin_popcountll(need);
+      if (qCount + cnt > kQueue) flush();
+      if (xMask) {
+        const int pos = qCount + __builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
+        qTri[wave][pos] = __builtin_amdgcn_readlane(tid, j);
+        qPix[wave][pos] = (uint32_t)lane | ((uint32_t)xMask << 8);
+        myEntries |= 1ull << pos;
+        nShaded++;
+      }
+      qCount += cnt;
+    }
+  };
+
+  // Candidates (box meets the block, hierarchical depth test passed) are
+  // compacted, in list order, into a per-wave ring, and the exact coverage
+  // runs on full batches of 64: a 64-entry chunk of the list yields about a
+  // third of a wave of candidates.
+  __shared__ uint32_t ring[4][128];
+  __shared__ float ringZ[4][128];
+  uint32_t ringHead = 0, ringCount = 0;  // wave-uniform
+
+  for (uint32_t base = start; base < end; base += 64) {
+    // ---- block depth bound for the hierarchical test ----
+    const float zmax = hiz ? block_zmax() : __builtin_inff();
+    // ---- candidate test: box overlap, then the hierarchical depth bound ----
+    const uint32_t e = base + lane;
+    bool test = false;
+    uint32_t tid = 0;
+    float zlo = -__builtin_inff();
+    // A binned pair carries the blocks of its tile that the primitive's
+    // edges may reach (bits 28-31); the box test completes the overlap test.
+    bool reach = true;
+    if (e < end) {
+      if (binTri) {
+        const uint32_t v = binTri[e];
+        tid = v & kSlotMask;
+        reach = (v >> (28 + wave)) & 1u;
+      } else {
+        tid = e;
+      }
+    }
+    if (e < end && reach) {
+      const int4 *rp = reinterpret_cast<const int4 *>(rec + tid);
+      const int4 h0 = rp[0];  // nflags, yMin, yMax, xMin
+      const int4 h1 = rp[1];  // xMax, ...
+      test = h0.y < oy + 8 && h0.z > oy && h0.w < ox + 8 && h1.x > ox;
+      if (hiz && test) {
+        const float zlo0 = __int_as_float(rp[2].w);                  // zlo
+        const float4 h3 = reinterpret_cast<const float4 *>(rp)[3];  // x0, y0, zA, zB
+        const float4 h4 = reinterpret_cast<const float4 *>(rp)[4];  // zC, zBias, ...
+        const float x0 = h3.x, y0 = h3.y, zA = h3.z, zB = h3.w, zC = h4.x;
+        const float zBias = depthBias ? h4.y : 0.0f;
+        // Lower bound of the evaluated plane over this block (sample offsets
+        // included), tightened with the primitive's bound over its box.
+        const float xa = (float)ox - 0.5f - x0, xb = (float)(ox + 7) + 0.5f - x0;
+        const float ya = (float)oy - 0.5f - y0, yb = (float)(oy + 7) + 0.5f - y0;
+        const float m =
+            fminf(fminf(zA * xa + zB * ya, zA * xb + zB * ya), fminf(zA * xa + zB * yb, zA * xb + zB * yb)) + zC +
+            zBias;
+        const float mag = fabsf(zA) * fmaxf(fabsf(xa), fabsf(xb)) + fabsf(zC) +
+                          2.0f * fabsf(zB) * fmaxf(fabsf(ya), fabsf(yb)) + 2.0f * fabsf(zBias);
+        float zl = fmaxf(zlo0, m - mag * 0x1p-19f);
+        if (!(zl == zl)) zl = -__builtin_inff();
+        zl = fminf(zl, P.depthClampHi);
+        if ((XF && P.depth16)) zl = d16_value(fmaxf(zl, 0.0f));  // the bound in stored units (monotone map)
+        test = !(P.depthCompare == 1 ? zl >= zmax : zl > zmax);
+        zlo = zl;
+      }
+    }
+    nTests += test ? 1u : 0u;
+    const uint64_t tb = __ballot(test);
+    if (test) {
+      const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(tb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tb, 0));
+      ring[wave][(ringHead + ringCount + pos) & 127] = tid;
+      ringZ[wave][(ringHead + ringCount + pos) & 127] = zlo;
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    ringCount += (uint32_t)__builtin_popcountll(tb);
+    if (ringCount >= 64) {
+      const uint32_t t2 = ring[wave][(ringHead + lane) & 127];
+      const float z2 = ringZ[wave][(ringHead + lane) & 127];
+      ringHead = (ringHead + 64) & 127;
+      ringCount -= 64;
+      process_chunk(true, t2, z2);
+    }
+  }
+  while (ringCount > 0) {
+    const uint32_t nb = ringCount < 64 ? ringCount : 64;
+    const bool act = (uint32_t)lane < nb;
+    const uint32_t t2 = act ? ring[wave][(ringHead + lane) & 127] : 0u;
+    const float z2 = act ? ringZ[wave][(ringHead + lane) & 127] : -__builtin_inff();
+    ringHead = (ringHead + nb) & 127;
+    ringCount -= nb;
+    process_chunk(act, t2, z2);
+  }
+  if (qCount) flush();
+
+  // Write the block back.
+  if (inside) {
+#pragma unroll
+    for (int q = 0; q < MS; q++) {
+      if (P.depthWrite) {
+        if ((XF && P.depth16))
+          *reinterpret_cast<uint16_t *>(P.depth + q * P.depthSlice + (long long)py * P.depthPitch + 2ll * px) =
+              (uint16_t)S.zb[q];
+        else
+          *reinterpret_cast<float *>(P.depth + q * P.depthSlice + (long long)py * P.depthPitch + 4ll * px) = S.zb[q];
+      }
+      if (P.stencilWrite) P.stencil[q * P.stencilSlice + (long long)py * P.stencilPitch + px] = (char)S.sb[q];
+      if (FCOL && P.primId)
+        *reinterpret_cast<uint32_t *>(P.primId + q * P.primIdSlice + (long long)py * P.primIdPitch + 4ll * px) =
+            S.id[FCOL ? q : 0];
+      if (P.colorMask) {
+        if (FCOL)
+          *reinterpret_cast<float4 *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 16ll * px) =
+              S.cf[FCOL ? q : 0];
+        else
+          *reinterpret_cast<uint32_t *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 4ll * px) =
+              bgra_swap((XF && P.colorBGRA), S.cb[FCOL ? 0 : q]);
+      }
+    }
+  }
+
+  // Counters: reduce over the wave, then over the workgroup, so that one
+  // atomic per counter and workgroup reaches the (single) global address.
+  __shared__ unsigned long long red[4][4];
+  if (P.occlusion || P.stats) {
+    unsigned long long v[4] = {occl, nTests, nCovers, nShaded};
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) red[wave][k] = v[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+      const int k = threadIdx.x;
+      const int nw = (int)(blockDim.x >> 6);
+      unsigned long long t = red[0][k];
+      for (int w = 1; w < nw; w++) t += red[w][k];
+      if (k == 0) {
+        if (P.occlusion && t) atomicAdd(P.occlusion, t);
+      } else if (P.stats) {
+        atomicAdd(P.stats + (k - 1), t);
+      }
+    }
+  }
+}
+
+// A batch of draws: persistent workgroups take global tiles [tileLo, tileHi)
+// from an atomic counter (or, with counter == NULL, workgroup b renders tile
+// tileLo + b once); tile t belongs to the draw d in [drawLo, drawHi) with
+// tileBase[d] <= t < tileBase[d + 1].
+//
+// binTri == NULL selects the unbinned pass: every tile walks the record
+// slots of its draw from *split on (the primitives the binned pass left out
+// because their pairs exceeded the planned capacity) in slot order, testing
+// each against its blocks as it would a binned list.  It does nothing when
+// *split >= segT (everything was binned).  With binTri and `tail`, each tile
+// walks its binned list and then those slots, so that one launch does both
+// passes (the tiles of one launch never share pixels, so only the order
+// within a tile matters).
+// Occupancy: 4 waves per SIMD (128 VGPRs) for the single-sample kernels
+// (the float-colour ones spill 12 bytes there and still run faster than at
+// 3 waves), 3 for the multisample ones.
+template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL>
+__global__ __launch_bounds__(256, MS == 1 ? 4 : 3) void raster_batch_kernel(
+                                                           const DrawParams *__restrict__ params,
+                                                           const uint32_t *__restrict__ tileBase, int drawLo,
+                                                           int drawHi, uint32_t tileLo, uint32_t tileHi,
+                                                           uint32_t *__restrict__ counter,
+                                                           const TriRecord *__restrict__ rec,
+                                                           const int *__restrict__ poly,
+                                                           const uint32_t *__restrict__ binTri,
+                                                           const uint32_t *__restrict__ tileStart,
+                                                           const uint32_t *__restrict__ tileEnd,
+                                                           const uint32_t *__restrict__ split, uint32_t segT,
+                                                           int tail) {
+  __shared__ uint32_t sTile;
+  const uint32_t from = (binTri && !tail) ? segT : *split;
+  if (!binTri && from >= segT) return;
+  // Passes per tile: 0 = the binned list, 1 = the slots from *split on.
+  const int pass0 = binTri ? 0 : 1, pass1 = from < segT ? 2 : 1;
+  for (uint32_t iter = 0;; iter++) {
+    uint32_t t;
+    if (counter) {
+      if (threadIdx.x == 0) sTile = tileLo + atomicAdd(counter, 1u);
+      __syncthreads();
+      t = __builtin_amdgcn_readfirstlane(sTile);
+      __syncthreads();
+    } else {
+      if (iter) break;
+      t = tileLo + blockIdx.x;
+    }
+    if (t >= tileHi) break;
+    int lo = drawLo, hi = drawHi;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (tileBase[mid] <= t) lo = mid;
+      else hi = mid;
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+#pragma nounroll
+    for (int pass = pass0; pass < pass1; pass++) {
+      uint32_t s, e;
+      if (pass == 0) {
+        s = tileStart[t];
+        e = tileEnd[t];
+      } else {
+        const uint32_t b = (uint32_t)params[lo].triBase;
+        s = from > b ? from : b;
+        e = b + (uint32_t)params[lo].triCount;
+      }
+      if (s < e)
+        raster_tile<MS, FCOL, FTEX, XF, LEVEL>(params[lo], (int)(t - tileBase[lo]), s, e, rec, poly,
+                                               pass == 0 ? binTri : nullptr);
+    }
+  }
+}
+
+template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL>
+void launch_raster_batch(dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
+  hipLaunchKernelGGL((raster_batch_kernel<MS, FCOL, FTEX, XF, LEVEL>), grid, block, 0, s, a.params, a.tileBase, a.lo,
+                     a.hi, a.tLo, a.tHi, a.counter, a.rec, a.poly, a.bin, a.ts, a.te, a.split, a.segT,
+                     a.tail);
+}
+
+// The raster kernel of variant v (variant_of).
+template <bool XF, int LEVEL>
+void launch_raster_variant(int v, dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
+  switch (v & 7) {
+    case 0: launch_raster_batch<1, false, false, XF, LEVEL>(grid, block, s, a); break;
+    case 1: launch_raster_batch<1, false, true, XF, LEVEL>(grid, block, s, a); break;
+    case 2: launch_raster_batch<1, true, false, XF, LEVEL>(grid, block, s, a); break;
+    case 3: launch_raster_batch<1, true, true, XF, LEVEL>(grid, block, s, a); break;
+    case 4: launch_raster_batch<4, false, false, XF, LEVEL>(grid, block, s, a); break;
+    case 5: launch_raster_batch<4, false, true, XF, LEVEL>(grid, block, s, a); break;
+    case 6: launch_raster_batch<4, true, false, XF, LEVEL>(grid, block, s, a); break;
+    default: launch_raster_batch<4, true, true, XF, LEVEL>(grid, block, s, a); break;
+  }
+}
+
+}  // namespace swr
