@@ -196,17 +196,27 @@ int blend_operation(int op, int sf, int df, bool isFloat) {
 int stencil_params(const swr_stencil_op_state &s, StencilParams &o) {
   if (s.compare_op > 7 || s.fail_op > 7 || s.pass_op > 7 || s.depth_fail_op > 7)
     return fail(SWR_ERROR_INVALID_ARGUMENT, "invalid stencil op state");
+  // (ref & mask) OP (value & mask); a compare mask of 0xFF keeps the value
+  // whole, which it is (8 bits).
   o.compareOp = (int)s.compare_op;
-  o.failOp = (int)s.fail_op;
-  o.passOp = (int)s.pass_op;
-  o.depthFailOp = (int)s.depth_fail_op;
-  o.useCompareMask = s.compare_mask != 0xFFu;
-  o.useWriteMask = (s.write_mask & 0xFFu) != 0xFFu;
   o.compareMask = s.compare_mask & 0xFFu;
-  o.writeMask = s.write_mask & 0xFFu;
-  o.reference = s.reference & 0xFFu;
   o.refMasked = s.reference & s.compare_mask & 0xFFu;
-  o.refSigned = (int32_t)(int8_t)(uint8_t)(((s.reference & s.compare_mask) + 0x80u) & 0xFFu);
+  o.writeMask = s.write_mask & 0xFFu;
+  auto op = [&](uint32_t k) {
+    switch (k) {
+      case SWR_STENCIL_OP_KEEP: return StencilOp{0, 255, 0, 0, 255};
+      case SWR_STENCIL_OP_ZERO: return StencilOp{0, 0, 0, 0, 255};
+      case SWR_STENCIL_OP_REPLACE: return StencilOp{0, 0, (int)(s.reference & 0xFFu), 0, 255};
+      case SWR_STENCIL_OP_INCREMENT_AND_CLAMP: return StencilOp{0, 255, 1, 0, 255};
+      case SWR_STENCIL_OP_DECREMENT_AND_CLAMP: return StencilOp{0, 255, -1, 0, 255};
+      case SWR_STENCIL_OP_INVERT: return StencilOp{255, 255, 0, 0, 255};
+      case SWR_STENCIL_OP_INCREMENT_AND_WRAP: return StencilOp{0, 255, 1, 0, 256};
+      default: return StencilOp{0, 255, -1, -1, 255};  // DECREMENT_AND_WRAP
+    }
+  };
+  o.fail = op(s.fail_op);
+  o.depthFail = op(s.depth_fail_op);
+  o.pass = op(s.pass_op);
   return SWR_OK;
 }
 
@@ -589,8 +599,11 @@ int variant_of(const DrawParams &P) {
   // linear or anisotropic filtering, linear mips, blending off or SRC_ALPHA /
   // ONE_MINUS_SRC_ALPHA / ADD, and REPEAT (level 2) or CLAMP_TO_EDGE (level
   // 3) on both axes.
+  // Its depth range ends at ordinary floats (+0 or normal), for which max and
+  // min instructions equal the ordered selects bit for bit.
+  auto ordinary = [](float v) { return v == 0.0f ? !std::signbit(v) : std::isnormal(v); };
   const bool simple = !xf && !P.stencilActive && !P.stencilWrite && !P.depthBias && P.depthTest && P.depthWrite &&
-                      P.colorMask == 15;
+                      P.colorMask == 15 && ordinary(P.depthClampLo) && ordinary(P.depthClampHi);
   const bool fast = simple && P.shader == SHADER_MODULATE && P.useColor && P.useUV &&
                     (!P.blendEnable || P.blendKind == 1) && !P.tex.skipLod && P.tex.mipmap == MIP_LINEAR &&
                     P.tex.addrU == P.tex.addrV && P.tex.addrU <= 1 &&

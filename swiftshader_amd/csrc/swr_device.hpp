@@ -571,34 +571,16 @@ __device__ __forceinline__ uint32_t float_to_unorm8(float c) {
   return (uint32_t)(i < 0 ? 0 : (i > 255 ? 255 : i));
 }
 
-__device__ __forceinline__ uint32_t stencil_apply_op(uint32_t v, int op, uint32_t ref) {
-  switch (op) {
-    case 0: return v;
-    case 1: return 0;
-    case 2: return ref & 0xFFu;
-    case 3: return v == 255u ? 255u : v + 1u;
-    case 4: return v == 0u ? 0u : v - 1u;
-    case 5: return (~v) & 0xFFu;
-    case 6: return (v + 1u) & 0xFFu;
-    default: return (v - 1u) & 0xFFu;
-  }
+__device__ __forceinline__ uint32_t stencil_apply_op(uint32_t v, const StencilOp &op) {
+  const int t = (int)((v ^ (uint32_t)op.flip) & (uint32_t)op.keep) + op.add;
+  return (uint32_t)min(max(t, op.lo), op.hi) & 255u;
 }
 
-// (ref & mask) OP (value & mask) through biased signed-byte compares (:405-449).
+// (ref & mask) OP (value & mask) (PixelRoutine.cpp:405-449).
 __device__ __forceinline__ bool stencil_compare(const StencilParams &S, uint32_t value) {
-  uint32_t val = S.useCompareMask ? (value & S.compareMask) : value;
-  int32_t vs = (int32_t)(int8_t)(uint8_t)(val + 0x80u);
-  int32_t rs = S.refSigned;
-  switch (S.compareOp) {
-    case 7: return true;
-    case 0: return false;
-    case 1: return vs > rs;
-    case 2: return val == S.refMasked;
-    case 5: return val != S.refMasked;
-    case 3: return vs > rs || val == S.refMasked;
-    case 4: return rs > vs;
-    default: return !(vs > rs);
-  }
+  const uint32_t val = value & S.compareMask;
+  return ((S.compareOp & 1) && S.refMasked < val) || ((S.compareOp & 2) && S.refMasked == val) ||
+         ((S.compareOp & 4) && S.refMasked > val);
 }
 
 }  // namespace swr

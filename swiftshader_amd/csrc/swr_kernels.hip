@@ -493,7 +493,15 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
     int *pp = poly + g * (2 * kMaxPolygon);
     for (int i = 0; i < n; i++) { pp[i] = X[i]; pp[kMaxPolygon + i] = Y[i]; }
   }
-  R.nflags = n | (d << 8) | (frontFacing ? 1 << 9 : 0);
+  int planes = 0;
+  if (n == 3) {
+    const int a0 = isPolygon ? X[0] : PX[0], a1 = isPolygon ? X[1] : PX[1], a2 = isPolygon ? X[2] : PX[2];
+    const int b0 = isPolygon ? Y[0] : PY[0], b1 = isPolygon ? Y[1] : PY[1], b2 = isPolygon ? Y[2] : PY[2];
+    const int lo = min(min(min(a0, a1), a2), min(min(b0, b1), b2)), hi = max(max(max(a0, a1), a2), max(max(b0, b1), b2));
+    const int ex = wsub(max(max(a0, a1), a2), min(min(a0, a1), a2)), ey = wsub(max(max(b0, b1), b2), min(min(b0, b1), b2));
+    if (lo > -(1 << 20) && hi < (1 << 20) && ex <= 32767 && ey <= 32767) planes = kRecHalfPlanes;
+  }
+  R.nflags = n | (d << 8) | (frontFacing ? 1 << 9 : 0) | planes;
   // Tiles are 8 or 16 pixels a side and xMin, yMin >= 0 (scissor-clamped to
   // a render area at x, y >= 0): shifts divide exactly.
   const int sw = __builtin_ctz((uint32_t)P.tileW), sh = __builtin_ctz((uint32_t)P.tileH);

@@ -42,11 +42,18 @@ struct TexParams {
   float mipLodBias, maxAnisotropy, minLod, maxLod;
 };
 
+// A stencil op as arithmetic on the stored value v, without branches:
+// clamp(((v ^ flip) & keep) + add, lo, hi) & 255.
+struct StencilOp {
+  int flip, keep, add, lo, hi;
+};
+
 struct StencilParams {
-  int compareOp, failOp, passOp, depthFailOp;
-  int useCompareMask, useWriteMask;
-  uint32_t compareMask, writeMask, reference, refMasked;
-  int32_t refSigned;
+  // The compare: which of reference < value, ==, > (masked) pass, as bits 0,
+  // 1 and 2 (VkCompareOp's own encoding).
+  int compareOp;
+  uint32_t compareMask, refMasked, writeMask;
+  StencilOp fail, depthFail, pass;
 };
 
 struct DrawParams {
@@ -125,7 +132,7 @@ struct DrawParams {
 // (w plane and attribute planes) is read when fragments are shaded.
 struct TriRecord {
   int nflags;       // bits 0-7: polygon vertex count n (3 unless clipped; 0: culled);
-                    // bit 8: d (winding); bit 9: front facing
+                    // bit 8: d (winding); bit 9: front facing; bit 10: kRecHalfPlanes
   int yMin, yMax;   // rows with possible coverage (scissor-clamped)
   int xMin, xMax;   // pixel columns with possible coverage
   int X[3], Y[3];   // 28.4 polygon vertices when n == 3
@@ -137,6 +144,11 @@ struct TriRecord {
   float V[6][3];    // colour rgba, uv
   int draw;         // index of the primitive's draw in its batch
 };
+
+// Triangle (n == 3) whose coverage is three half planes with 16-bit edge
+// extents: coordinates below 2^20 and edges up to 32767 (28.4), so that the
+// half planes step over a block with one 16-bit dot product each.
+constexpr int kRecHalfPlanes = 1 << 10;
 
 static_assert(sizeof(TriRecord) == 160, "TriRecord layout");
 

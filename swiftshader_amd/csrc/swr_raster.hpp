@@ -31,6 +31,7 @@ __device__ __constant__ const float kSampleX[4] = {-0.125f, 0.375f, -0.375f, 0.1
 __device__ __constant__ const float kSampleY[4] = {-0.375f, -0.125f, 0.125f, 0.375f};
 __device__ __constant__ const int kXf[4] = {-2, 6, -6, 2};
 __device__ __constant__ const int kYf[4] = {-6, -2, 2, 6};
+constexpr int kXf0 = -2, kYf0 = -6, kXf1 = 6, kYf1 = -2;  // of samples 0 and 1; 2 and 3 lie opposite 1 and 0
 
 // D16 compares and stores Min(Max(Round(z * 0xFFFF), 0), 0xFFFF) of the
 // clamped depth (PixelRoutine.cpp:506-510, 686-711; Round is to nearest even).
@@ -50,10 +51,10 @@ __device__ __forceinline__ uint32_t bgra_swap(int bgra, uint32_t v) {
 // Work decomposition: one workgroup per 16x16 bin, one wavefront per 8x8
 // block of the bin, one pixel per lane (lanes 4k..4k+3 form a 2x2 quad).
 // Each wave walks the bin's triangle list in API order, 64 entries at a
-// time: every lane computes the exact 8x8 coverage mask of one triangle
-// (triangle-parallel), a ballot compacts the triangles that cover the
-// block, and the wave then applies them one by one (pixel-parallel) to the
-// block's depth / stencil / colour, which stay in registers throughout.
+// time; the entries whose box and depth bound meet the block are compacted
+// into batches of 64, every lane sets up one of them (triangle-parallel),
+// and the wave then applies them one by one (pixel-parallel) to the block's
+// depth / stencil / colour, which stay in registers throughout.
 //
 // Coverage is the reference's span rule evaluated per sample point.  The
 // reference walks each edge with an exact integer DDA that stores
@@ -63,9 +64,22 @@ __device__ __forceinline__ uint32_t bgra_swap(int bgra, uint32_t v) {
 // (QuadRasterizer.cpp:181-206).  With
 //   E(x, y) = DY * (16 x - X1) - DX * (16 y - Y1),   DY = Y2 - Y1 > 0,
 // "ceil(Xe/16) <= x" is exactly E >= 0 and "x < ceil(Xe/16)" is exactly
-// E < 0, so the span test becomes two integer sign tests per sample.  E at
-// the block origin is formed in 64 bits and clamped to +-2^30: beyond that
-// its sign cannot change inside the block, and the 32-bit steps are exact.
+// E < 0, so the span test becomes two integer sign tests per sample.
+//
+// A triangle (n == 3) needs no spans: over the rows it spans, one left and
+// one right edge bound each row, so the rule equals three half planes.  With
+// an edge a -> b in the order the reference walks it (interior at F > 0),
+//   F(x, y) = (Yb - Ya) * (16 x - Xa) - (Xb - Xa) * (16 y - Ya),
+// a sample is covered iff F >= 0 for left edges (Yb > Ya) and for horizontal
+// top edges (Yb == Ya, Xb < Xa), and F > 0 for the others: left edges have
+// F = E, right ones F = -E, and the horizontal ones keep the row range.  The
+// three F add up to a constant (twice the area, signed by the winding), so a
+// degenerate triangle, or one whose winding the float determinant of the
+// setup misjudged, covers nothing under either rule.  F at the block origin
+// is formed in 64 bits and clamped to +-2^30: beyond that its sign cannot
+// change inside the block.  Edge extents below 2^15 (triangles up to 2047
+// pixels) make the step over the block one 16-bit dot product; larger
+// triangles and clipped polygons, lines and points take the spans.
 
 struct LaneEdge {
   int e;      // E at the block origin (clamped)
@@ -140,6 +154,37 @@ __device__ __forceinline__ uint64_t block_coverage(const VFetch &vtx, int n, int
   return mask;
 }
 
+// Edge a -> b of a triangle as its half plane over the block at (ox, oy):
+// `pk` holds (Yb - Ya, Xb - Xa) as 16-bit halves, and the pixel at (cx, cy)
+// of the block is inside iff dot2(pk, (16 cx, -16 cy)) >= nf (the sample at
+// 28.4 offset (xo, yo) iff the dot product >= nf - (DY xo - DX yo)).
+__device__ __forceinline__ void half_plane(int Xa, int Ya, int Xb, int Yb, int ox, int oy, int &pk, int &nf) {
+  const int DX = Xb - Xa, DY = Yb - Ya;
+  const bool closed = DY > 0 || (DY == 0 && DX < 0);
+  const long long v = (long long)DY * (long long)(16 * ox - Xa) - (long long)DX * (long long)(16 * oy - Ya);
+  const long long lim = 1ll << 30;
+  const int f = (int)(v > lim ? lim : (v < -lim ? -lim : v));
+  pk = (int)(((uint32_t)DY & 0xFFFFu) | ((uint32_t)DX << 16));
+  nf = (closed ? 0 : 1) - f;
+}
+
+typedef short Short2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ int dot2_i16(int a, int b) {
+  return __builtin_amdgcn_sdot2(__builtin_bit_cast(Short2, a), __builtin_bit_cast(Short2, b), 0, false);
+}
+
+// Largest value of v over the wave (wave-uniform), by DPP: the old value of
+// lanes without a source is the identity, so each step is one instruction.
+__device__ __forceinline__ int wave_max_i32(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+  v = max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x114, 0xf, 0xf, false));  // row_shr:4
+  v = max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x118, 0xf, 0xf, false));  // row_shr:8
+  v = max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  v = max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 template <int MS, bool FCOL>
 struct PixelState {
   float zb[MS];
@@ -156,10 +201,11 @@ __device__ __forceinline__ int lane_cy(int l) { return 2 * (l >> 4) + ((l >> 1) 
 
 // Blend a shaded colour into the samples of this lane's pixel selected by
 // xMask, then write (PixelRoutine.cpp:1617-2936).
+// srgbLut: srgb_to_linear of every 8-bit code (sRGB targets).
 // FAST: blending, when on, is SRC_ALPHA, ONE_MINUS_SRC_ALPHA, ADD.
 template <int MS, bool FCOL, bool XF, bool FAST = false>
 __device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, FCOL> &S, float4 s, int xMask,
-                                            uint32_t tri) {
+                                            uint32_t tri, const float *srgbLut) {
 #pragma unroll
   for (int q = 0; q < MS; q++) {
     if (!((xMask >> q) & 1)) continue;
@@ -171,9 +217,9 @@ __device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, 
       dst = make_float4(unorm8_to_float(p & 0xFFu), unorm8_to_float((p >> 8) & 0xFFu),
                         unorm8_to_float((p >> 16) & 0xFFu), unorm8_to_float(p >> 24));
       if ((XF && P.colorSRGB) && P.blendEnable) {  // blended in linear space (PixelRoutine.cpp:1811-1827)
-        dst.x = srgb_to_linear(dst.x);
-        dst.y = srgb_to_linear(dst.y);
-        dst.z = srgb_to_linear(dst.z);
+        dst.x = srgbLut[p & 0xFFu];
+        dst.y = srgbLut[(p >> 8) & 0xFFu];
+        dst.z = srgbLut[(p >> 16) & 0xFFu];
       }
     }
     float4 o = P.blendEnable ? (FAST ? blend_src_alpha(s, dst) : alpha_blend<XF>(P, s, dst)) : s;
@@ -280,14 +326,22 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     }
   }
 
+  // The 256 decoded codes of an sRGB target that is blended, so that a blend
+  // reads its three channels instead of evaluating three powers.
+  __shared__ float srgbLut[XF ? 256 : 1];
+  if (XF && P.colorSRGB && P.blendEnable) {
+    for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) srgbLut[i] = srgb_to_linear(unorm8_to_float(i));
+    __syncthreads();
+  }
+
   // Hierarchical depth: a primitive whose evaluated depth is bounded below
   // by zlo cannot pass LESS (LESS_OR_EQUAL) anywhere in a block whose
   // largest stored depth is <= zlo (< zlo).  Only when a failing fragment
   // has no side effect (no stencil writes).
   const bool hiz = depthTest && !stencilWrite && (P.depthCompare == 1 || P.depthCompare == 3);
 
-  unsigned long long occl = 0;
-  uint32_t nTests = 0, nCovers = 0, nShaded = 0;  // statistics (profiling only)
+  // Wave totals; nTests, nCovers and nShaded are statistics (profiling only).
+  unsigned long long occl = 0, nTests = 0, nCovers = 0, nShaded = 0;
   int qCount = 0;           // wave-uniform queue length
   uint64_t myEntries = 0;   // queue slots holding fragments of this lane's pixel
 
@@ -306,7 +360,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     while (m) {
       const int k = __builtin_ctzll(m);
       m &= m - 1;
-      blend_write<MS, FCOL, XF, FAST>(P, S, qCol[wave][k], (int)(qPix[wave][k] >> 8), qTri[wave][k]);
+      blend_write<MS, FCOL, XF, FAST>(P, S, qCol[wave][k], (int)(qPix[wave][k] >> 8), qTri[wave][k], srgbLut);
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -316,7 +370,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 
   // Largest stored depth of the block (+inf when any is NaN): a primitive
   // whose depth is bounded below by zl cannot pass where zl >= it (LESS) or
-  // zl > it (LESS_OR_EQUAL).
+  // zl > it (LESS_OR_EQUAL).  Reduced as integers that order like the floats.
   auto block_zmax = [&]() __attribute__((always_inline)) {
     float v = -__builtin_inff();
     bool nan = false;
@@ -327,25 +381,37 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
         nan |= S.zb[q] != S.zb[q];
       }
     }
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return __ballot(nan) ? __builtin_inff() : v;
+    const int i = __float_as_int(v);
+    const int m = wave_max_i32(i ^ ((i >> 31) & 0x7FFFFFFF));
+    return __ballot(nan) ? __builtin_inff() : __int_as_float(m ^ ((m >> 31) & 0x7FFFFFFF));
+  };
+  auto hidden = [&](float zl, float zmax) __attribute__((always_inline)) {
+    return P.depthCompare == 1 ? zl >= zmax : zl > zmax;
   };
 
-  // One batch of up to 64 candidates in list order: each lane computes the
-  // exact coverage of its primitive; then the covering primitives are
-  // applied in list order.  A candidate waited in the ring while earlier
-  // ones wrote depth, so its depth bound zl is tested again first.
+  // Coverage masks of a batch's primitives that take the spans.
+  __shared__ uint64_t spanMask[4][MS][64];
+  const int pixelStep = (int)((uint32_t)(16 * cx) | ((uint32_t)(-16 * cy) << 16));
+
+  // One batch of up to 64 candidates in list order: each lane sets up one
+  // primitive (its three half planes, or the span masks), then the primitives
+  // are applied in list order.  Most candidates of a deep block lie behind
+  // what the ones before them wrote, and the list of a block is seldom more
+  // than a batch or two, so the depth bounds zl are tested again before the
+  // batch and, all at once, after every kRetest primitives that wrote depth:
+  // at 1080p with 50 layers a block meets 86 candidates, of which 20 are not
+  // hidden by the time their turn comes.
+  constexpr int kRetest = 2;
   auto process_chunk = [&](bool act, uint32_t tid, float zl) __attribute__((always_inline)) {
     if (hiz) {
-      const float zmax = block_zmax();
-      act = act && !(P.depthCompare == 1 ? zl >= zmax : zl > zmax);
+      const float zmax = block_zmax();  // by every lane of the wave
+      act = act && !hidden(zl, zmax);
     }
-    // ---- triangle-parallel coverage of this block ----
-    uint32_t mlo[MS], mhi[MS];
+    // ---- triangle-parallel setup ----
+    int pk[3] = {0, 0, 0}, nf[3] = {0, 0, 0};
     int flags = 0;
     float x0 = 0, y0 = 0, zA = 0, zB = 0, zC = 0, zBias = 0;
-#pragma unroll
-    for (int q = 0; q < MS; q++) { mlo[q] = 0; mhi[q] = 0; }
+    bool spans = false;
     if (act) {
       const int4 *rp = reinterpret_cast<const int4 *>(rec + tid);
       const int4 h0 = rp[0];  // nflags, yMin, yMax, xMin
@@ -356,235 +422,307 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
       const int n = h0.x & 0xFF, d = (h0.x >> 8) & 1;
       flags = h0.x >> 8;
       x0 = h3.x; y0 = h3.y; zA = h3.z; zB = h3.w; zC = h4.x; zBias = h4.y;
-      const int *pp = poly + (size_t)tid * (2 * kMaxPolygon);
-      auto vtx = [&](int i, int &Xo, int &Yo) {
-        if (n == 3) {
-          // Mask selects: a conditional pick among the components of one
-          // vector would become an indexed access through scratch memory.
-          const int m0 = -(int)(i == 0), m1 = -(int)(i == 1), m2 = -(int)(i == 2);
-          Xo = (h1.y & m0) | (h1.z & m1) | (h1.w & m2);
-          Yo = (h2.x & m0) | (h2.y & m1) | (h2.z & m2);
-        } else {
-          Xo = pp[i];
-          Yo = pp[kMaxPolygon + i];
-        }
-      };
+      spans = !(h0.x & kRecHalfPlanes);
+      if (!spans) {
+        // Edge i runs from vertex i to i + 1 (d), or back.
+        const int X[3] = {h1.y, h1.z, h1.w}, Y[3] = {h2.x, h2.y, h2.z};
 #pragma unroll
-      for (int q = 0; q < MS; q++) {
-        if (!((P.msMask >> q) & 1)) continue;
-        const int xo = (MS > 1) ? kXf[q] : 0, yo = (MS > 1) ? kYf[q] : 0;
-        const uint64_t m = block_coverage(vtx, n, d, xo, yo, ox, oy) & scissorMask;
-        mlo[q] = (uint32_t)m;
-        mhi[q] = (uint32_t)(m >> 32);
+        for (int i = 0; i < 3; i++) {
+          const int k = (i + 1) % 3;
+          half_plane(d ? X[i] : X[k], d ? Y[i] : Y[k], d ? X[k] : X[i], d ? Y[k] : Y[i], ox, oy, pk[i], nf[i]);
+        }
+      } else {
+        const int *pp = poly + (size_t)tid * (2 * kMaxPolygon);
+        auto vtx = [&](int i, int &Xo, int &Yo) {
+          if (n == 3) {
+            // Mask selects: a conditional pick among the components of one
+            // vector would become an indexed access through scratch memory.
+            const int m0 = -(int)(i == 0), m1 = -(int)(i == 1), m2 = -(int)(i == 2);
+            Xo = (h1.y & m0) | (h1.z & m1) | (h1.w & m2);
+            Yo = (h2.x & m0) | (h2.y & m1) | (h2.z & m2);
+          } else {
+            Xo = pp[i];
+            Yo = pp[kMaxPolygon + i];
+          }
+        };
+        uint64_t any = 0;
+#pragma unroll
+        for (int q = 0; q < MS; q++) {
+          const int xo = (MS > 1) ? kXf[q] : 0, yo = (MS > 1) ? kYf[q] : 0;
+          const uint64_t m = block_coverage(vtx, n, d, xo, yo, ox, oy);
+          spanMask[wave][q][lane] = m;
+          any |= m;
+        }
+        act = any != 0;
       }
     }
-    uint32_t anyBits = 0;
-#pragma unroll
-    for (int q = 0; q < MS; q++) anyBits |= mlo[q] | mhi[q];
-    uint64_t todo = __ballot(anyBits != 0);
-    nCovers += anyBits != 0 ? 1u : 0u;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    uint64_t todo = __ballot(act);
+    const uint64_t spanLanes = __ballot(spans);
+    int wrote = 0;
 
-    // ---- pixel-parallel tests, in list order ----
+    // ---- pixel-parallel coverage and tests, in list order ----
     while (todo) {
       const int j = __builtin_ctzll(todo);
       todo &= todo - 1;
-      int cMask = 0;  // bit q: sample q of this lane's pixel is covered
+      bool cov[MS];
 #pragma unroll
-      for (int q = 0; q < MS; q++) {
-        const uint32_t lo = __builtin_amdgcn_readlane(mlo[q], j), hi = __builtin_amdgcn_readlane(mhi[q], j);
-        const uint32_t word = myBit < 32 ? lo : hi;
-        cMask |= (int)((word >> (myBit & 31)) & 1u) << q;
-      }
-      const int fl = __builtin_amdgcn_readlane(flags, j);
-      const StencilParams &SP = (fl & 2) ? P.front : P.back;
-
-      int sMask = cMask, zMask = cMask;
-      if (stencilActive && cMask) {
+      for (int q = 0; q < MS; q++) cov[q] = inside && ((P.msMask >> q) & 1);
+      if (!((spanLanes >> j) & 1)) {
 #pragma unroll
-        for (int q = 0; q < MS; q++)
-          if (((cMask >> q) & 1) && !stencil_compare(SP, S.sb[q])) sMask &= ~(1 << q);
-      }
-      if (XF && P.alphaToCoverage) {
-        // The reference shades before the depth test and keeps sample q
-        // only where !(alpha < a2c[q]) (alphaTest / alphaToCoverage,
-        // PixelProgram.cpp:243-259, PixelRoutine.cpp:317-337, 643-657); the
-        // alpha is clamped when the colour attachment is UNORM.  The
-        // fragment is shaded again, identically, if it reaches the queue.
-        if (cMask) {
-          const uint32_t tj = __builtin_amdgcn_readlane(tid, j);
-          const float a = shade<FCOL, FTEX, XF, FA>(P, rec[tj], px, py, P.color != nullptr).w;
-          int aMask = 0;
-#pragma unroll
-          for (int q = 0; q < MS; q++)
-            if (!(a < P.a2c[q])) aMask |= 1 << q;
-          cMask &= aMask;
+        for (int i = 0; i < 3; i++) {
+          const int p = __builtin_amdgcn_readlane(pk[i], j), n0 = __builtin_amdgcn_readlane(nf[i], j);
+          const int t = dot2_i16(p, pixelStep);
+          if (MS == 1) {
+            cov[0] &= t >= n0;
+          } else {
+            // The samples' offsets are +-(kXf[0], kYf[0]) and +-(kXf[1], kYf[1]).
+            const int DY = (int)(int16_t)p, DX = p >> 16;
+            const int o0 = DY * kXf0 - DX * kYf0, o1 = DY * kXf1 - DX * kYf1;
+            cov[0] &= t >= n0 - o0;
+            cov[MS > 1 ? 1 : 0] &= t >= n0 - o1;
+            cov[MS > 1 ? 2 : 0] &= t >= n0 + o1;
+            cov[MS > 1 ? 3 : 0] &= t >= n0 + o0;
+          }
         }
-        sMask &= cMask;
-        zMask &= cMask;
+      } else {
+#pragma unroll
+        for (int q = 0; q < MS; q++) cov[q] = cov[q] && ((spanMask[wave][q][j] >> myBit) & 1);
       }
-      float zq[MS];
-      if (depthTest) {
+      nTests++;
+      bool anyCov = false;
+#pragma unroll
+      for (int q = 0; q < MS; q++) anyCov |= cov[q];
+      if (!__ballot(anyCov)) continue;
+      nCovers++;
+
+      bool pass[MS];  // samples that pass every test
+      if constexpr (SIMPLE) {
         const float xf = (float)px - rdl(x0, j);  // xFragment (PixelRoutine.cpp:125)
         const float yf = (float)py - rdl(y0, j);  // yFragment (QuadRasterizer.cpp:126)
         const float a = rdl(zA, j), b = rdl(zB, j), c = rdl(zC, j);
-        const float zbias = depthBias ? rdl(zBias, j) : 0.0f;
-        zMask = 0;
+        float zq[MS];
 #pragma unroll
         for (int q = 0; q < MS; q++) {
           const float yy = (MS > 1) ? yf + kSampleY[q] : yf;
           const float xx = (MS > 1) ? xf - kSampleX[q] : xf;
           const float Dz = c + yy * b;
-          float z = xx * a + Dz;
-          if (depthBias) z = z + zbias;  // PixelRoutine.cpp:141-144, before the clamp
-          z = rr_min(rr_max(z, P.depthClampLo), P.depthClampHi);  // clampDepth
-          if ((XF && P.depth16)) z = d16_value(z);
-          zq[q] = z;
-          const float zb = S.zb[q];
-          // The compare op without branches: one of zb <= z, zb < z, zb == z
-          // or true, inverted for LESS, LESS_OR_EQUAL, NOT_EQUAL and NEVER.
-          const bool le = zb <= z, lt = zb < z, eq = zb == z;
-          const bool pr = P.zPred == 0 ? le : (P.zPred == 1 ? lt : (P.zPred == 2 ? eq : true));
-          if (pr != (P.zInv != 0)) zMask |= 1 << q;
+          // clampDepth; the common state's range is of ordinary floats, for
+          // which the hardware's max and min equal the ordered selects.
+          zq[q] = fminf(fmaxf(xx * a + Dz, P.depthClampLo), P.depthClampHi);
         }
-        zMask &= cMask;
-        if (stencilActive) zMask &= sMask;
-      }
-      if (XF && P.depthBounds && cMask) {
-        // depthBoundsTest (PixelRoutine.cpp:576-641) on the stored depth, D16
-        // as its code / 0xFFFF. With the depth test off the coverage loses
-        // the sample while zMask keeps it, so the occlusion count does too.
-        int bMask = 0;
+        // The compare op without branches per fragment: one of zb <= z,
+        // zb < z, zb == z or true, inverted for LESS, LESS_OR_EQUAL,
+        // NOT_EQUAL and NEVER; LESS on its own.
+        if (P.depthCompare == 1) {
+#pragma unroll
+          for (int q = 0; q < MS; q++) pass[q] = cov[q] && !(S.zb[q] <= zq[q]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < MS; q++) {
+            const bool le = S.zb[q] <= zq[q], lt = S.zb[q] < zq[q], eq = S.zb[q] == zq[q];
+            const bool pr = P.zPred == 0 ? le : (P.zPred == 1 ? lt : (P.zPred == 2 ? eq : true));
+            pass[q] = cov[q] && pr != (P.zInv != 0);
+          }
+        }
 #pragma unroll
         for (int q = 0; q < MS; q++) {
-          const float zs = P.depth16 ? S.zb[q] * (1.0f / 65535.0f) : S.zb[q];
-          if (P.depthBoundsMin <= zs && zs <= P.depthBoundsMax) bMask |= 1 << q;
+          S.zb[q] = pass[q] ? zq[q] : S.zb[q];
+          occl += (unsigned)__builtin_popcountll(__ballot(pass[q]));
         }
-        if (depthTest) zMask &= bMask;
-        else cMask &= bMask;
-      }
-      if (stencilWrite && cMask) {
+      } else {
+        const int fl = __builtin_amdgcn_readlane(flags, j);
+        const StencilParams &SP = (fl & 2) ? P.front : P.back;
+        bool sPass[MS], zPass[MS];
+#pragma unroll
+        for (int q = 0; q < MS; q++) sPass[q] = stencilActive ? cov[q] && stencil_compare(SP, S.sb[q]) : cov[q];
+        if (XF && P.alphaToCoverage) {
+          // The reference shades before the depth test and keeps sample q
+          // only where !(alpha < a2c[q]) (alphaTest / alphaToCoverage,
+          // PixelProgram.cpp:243-259, PixelRoutine.cpp:317-337, 643-657); the
+          // alpha is clamped when the colour attachment is UNORM.  The
+          // fragment is shaded again, identically, if it reaches the queue.
+          float alpha = 0.0f;
+          if (anyCov) alpha = shade<FCOL, FTEX, XF, FA>(P, rec[__builtin_amdgcn_readlane(tid, j)], px, py, P.color != nullptr).w;
+#pragma unroll
+          for (int q = 0; q < MS; q++) {
+            cov[q] = cov[q] && !(alpha < P.a2c[q]);
+            sPass[q] = sPass[q] && cov[q];
+          }
+        }
+        float zq[MS];
+#pragma unroll
+        for (int q = 0; q < MS; q++) zPass[q] = cov[q];
+        if (depthTest) {
+          const float xf = (float)px - rdl(x0, j);  // xFragment (PixelRoutine.cpp:125)
+          const float yf = (float)py - rdl(y0, j);  // yFragment (QuadRasterizer.cpp:126)
+          const float a = rdl(zA, j), b = rdl(zB, j), c = rdl(zC, j);
+          const float zbias = depthBias ? rdl(zBias, j) : 0.0f;
+#pragma unroll
+          for (int q = 0; q < MS; q++) {
+            const float yy = (MS > 1) ? yf + kSampleY[q] : yf;
+            const float xx = (MS > 1) ? xf - kSampleX[q] : xf;
+            const float Dz = c + yy * b;
+            float z = xx * a + Dz;
+            if (depthBias) z = z + zbias;  // PixelRoutine.cpp:141-144, before the clamp
+            z = rr_min(rr_max(z, P.depthClampLo), P.depthClampHi);  // clampDepth
+            if ((XF && P.depth16)) z = d16_value(z);
+            zq[q] = z;
+            const float zb = S.zb[q];
+            const bool le = zb <= z, lt = zb < z, eq = zb == z;
+            const bool pr = P.zPred == 0 ? le : (P.zPred == 1 ? lt : (P.zPred == 2 ? eq : true));
+            zPass[q] = (stencilActive ? sPass[q] : cov[q]) && pr != (P.zInv != 0);
+          }
+        }
+        if (XF && P.depthBounds) {
+          // depthBoundsTest (PixelRoutine.cpp:576-641) on the stored depth, D16
+          // as its code / 0xFFFF. With the depth test off the coverage loses
+          // the sample while zPass keeps it, so the occlusion count does too.
+#pragma unroll
+          for (int q = 0; q < MS; q++) {
+            const float zs = P.depth16 ? S.zb[q] * (1.0f / 65535.0f) : S.zb[q];
+            const bool in = P.depthBoundsMin <= zs && zs <= P.depthBoundsMax;
+            if (depthTest) zPass[q] = zPass[q] && in;
+            else cov[q] = cov[q] && in;
+          }
+        }
+        if (stencilWrite) {
+#pragma unroll
+          for (int q = 0; q < MS; q++) {
+            const uint32_t bv = S.sb[q];
+            uint32_t nv = stencil_apply_op(bv, SP.pass);
+            const bool zFail = depthTest && sPass[q] && !zPass[q];
+            if (__ballot(zFail)) {
+              const uint32_t v = stencil_apply_op(bv, SP.depthFail);
+              nv = zFail ? v : nv;
+            }
+            if (__ballot(cov[q] && !sPass[q])) {
+              const uint32_t v = stencil_apply_op(bv, SP.fail);
+              nv = sPass[q] ? nv : v;
+            }
+            nv = (nv & SP.writeMask) | (bv & ~SP.writeMask);
+            S.sb[q] = cov[q] ? nv : bv;
+          }
+        }
 #pragma unroll
         for (int q = 0; q < MS; q++) {
-          if (!((cMask >> q) & 1)) continue;
-          int op;
-          if (!((sMask >> q) & 1)) op = SP.failOp;
-          else if (depthTest && !((zMask >> q) & 1)) op = SP.depthFailOp;
-          else op = SP.passOp;
-          const uint32_t bv = S.sb[q];
-          uint32_t nv = stencil_apply_op(bv, op, SP.reference);
-          if (SP.useWriteMask) nv = (nv & SP.writeMask) | (bv & ~SP.writeMask);
-          S.sb[q] = nv & 0xFFu;
+          if (depthWrite) S.zb[q] = zPass[q] ? zq[q] : S.zb[q];
+          occl += (unsigned)__builtin_popcountll(__ballot(zPass[q] && sPass[q]));
+          pass[q] = (depthTest ? zPass[q] : cov[q]) && (!stencilActive || sPass[q]);
         }
       }
-      if (depthWrite) {
+
+      bool anyPass = false;
 #pragma unroll
-        for (int q = 0; q < MS; q++)
-          if ((zMask >> q) & 1) S.zb[q] = zq[q];
-      }
-      occl += __builtin_popcount((unsigned)(zMask & sMask));
-      if (!colorMask) continue;
-      int xMask = depthTest ? zMask : cMask;
-      if (stencilActive) xMask &= sMask;
-      const uint64_t need = __ballot(xMask != 0);
+      for (int q = 0; q < MS; q++) anyPass |= pass[q];
+      const uint64_t need = __ballot(anyPass);
       if (!need) continue;
-      // Queue the fragments that write colour; shading is deferred so that
-      // it runs with every lane busy.
-      const int cnt = __builtin_popcountll(need);
-      if (qCount + cnt > kQueue) flush();
-      if (xMask) {
-        const int pos = qCount + __builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
-        qTri[wave][pos] = __builtin_amdgcn_readlane(tid, j);
-        qPix[wave][pos] = (uint32_t)lane | ((uint32_t)xMask << 8);
-        myEntries |= 1ull << pos;
-        nShaded++;
+      if (colorMask) {
+        // Queue the fragments that write colour; shading is deferred so that
+        // it runs with every lane busy.
+        const int cnt = __builtin_popcountll(need);
+        if (qCount + cnt > kQueue) flush();
+        if (anyPass) {
+          const int pos = qCount + __builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
+          uint32_t xMask = 0;
+#pragma unroll
+          for (int q = 0; q < MS; q++) xMask |= pass[q] ? 1u << q : 0u;
+          qTri[wave][pos] = __builtin_amdgcn_readlane(tid, j);
+          qPix[wave][pos] = (uint32_t)lane | (xMask << 8);
+          myEntries |= 1ull << pos;
+        }
+        qCount += cnt;
+        nShaded += (unsigned)cnt;
       }
-      qCount += cnt;
+      // What the block shows now may hide the rest of the batch.
+      if (hiz && depthWrite && ++wrote >= kRetest && todo) {
+        wrote = 0;
+        const float zmax = block_zmax();
+        todo &= __ballot(!hidden(zl, zmax));
+      }
     }
   };
 
   // Candidates (box meets the block, hierarchical depth test passed) are
-  // compacted, in list order, into a per-wave ring, and the exact coverage
-  // runs on full batches of 64: a 64-entry chunk of the list yields about a
-  // third of a wave of candidates.
+  // compacted, in list order, into a per-wave ring, and set up in full
+  // batches of 64: a 64-entry chunk of the list yields about a third of a
+  // wave of candidates.
   __shared__ uint32_t ring[4][128];
   __shared__ float ringZ[4][128];
   uint32_t ringHead = 0, ringCount = 0;  // wave-uniform
 
-  for (uint32_t base = start; base < end; base += 64) {
-    // ---- block depth bound for the hierarchical test ----
-    const float zmax = hiz ? block_zmax() : __builtin_inff();
-    // ---- candidate test: box overlap, then the hierarchical depth bound ----
-    const uint32_t e = base + lane;
-    bool test = false;
-    uint32_t tid = 0;
-    float zlo = -__builtin_inff();
-    // A binned pair carries the blocks of its tile that the primitive's
-    // edges may reach (bits 28-31); the box test completes the overlap test.
-    bool reach = true;
-    if (e < end) {
-      if (binTri) {
-        const uint32_t v = binTri[e];
-        tid = v & kSlotMask;
-        reach = (v >> (28 + wave)) & 1u;
-      } else {
-        tid = e;
+  for (uint32_t base = start; base < end || ringCount > 0;) {
+    if (base < end) {
+      // ---- block depth bound for the hierarchical test ----
+      const float zmax = hiz ? block_zmax() : __builtin_inff();
+      // ---- candidate test: box overlap, then the hierarchical depth bound ----
+      const uint32_t e = base + lane;
+      bool test = false;
+      uint32_t tid = 0;
+      float zlo = -__builtin_inff();
+      // A binned pair carries the blocks of its tile that the primitive's
+      // edges may reach (bits 28-31); the box test completes the overlap test.
+      bool reach = true;
+      if (e < end) {
+        if (binTri) {
+          const uint32_t v = binTri[e];
+          tid = v & kSlotMask;
+          reach = (v >> (28 + wave)) & 1u;
+        } else {
+          tid = e;
+        }
       }
-    }
-    if (e < end && reach) {
-      const int4 *rp = reinterpret_cast<const int4 *>(rec + tid);
-      const int4 h0 = rp[0];  // nflags, yMin, yMax, xMin
-      const int4 h1 = rp[1];  // xMax, ...
-      test = h0.y < oy + 8 && h0.z > oy && h0.w < ox + 8 && h1.x > ox;
-      if (hiz && test) {
-        const float zlo0 = __int_as_float(rp[2].w);                  // zlo
-        const float4 h3 = reinterpret_cast<const float4 *>(rp)[3];  // x0, y0, zA, zB
-        const float4 h4 = reinterpret_cast<const float4 *>(rp)[4];  // zC, zBias, ...
-        const float x0 = h3.x, y0 = h3.y, zA = h3.z, zB = h3.w, zC = h4.x;
-        const float zBias = depthBias ? h4.y : 0.0f;
-        // Lower bound of the evaluated plane over this block (sample offsets
-        // included), tightened with the primitive's bound over its box.
-        const float xa = (float)ox - 0.5f - x0, xb = (float)(ox + 7) + 0.5f - x0;
-        const float ya = (float)oy - 0.5f - y0, yb = (float)(oy + 7) + 0.5f - y0;
-        const float m =
-            fminf(fminf(zA * xa + zB * ya, zA * xb + zB * ya), fminf(zA * xa + zB * yb, zA * xb + zB * yb)) + zC +
-            zBias;
-        const float mag = fabsf(zA) * fmaxf(fabsf(xa), fabsf(xb)) + fabsf(zC) +
-                          2.0f * fabsf(zB) * fmaxf(fabsf(ya), fabsf(yb)) + 2.0f * fabsf(zBias);
-        float zl = fmaxf(zlo0, m - mag * 0x1p-19f);
-        if (!(zl == zl)) zl = -__builtin_inff();
-        zl = fminf(zl, P.depthClampHi);
-        if ((XF && P.depth16)) zl = d16_value(fmaxf(zl, 0.0f));  // the bound in stored units (monotone map)
-        test = !(P.depthCompare == 1 ? zl >= zmax : zl > zmax);
-        zlo = zl;
+      if (e < end && reach) {
+        const int4 *rp = reinterpret_cast<const int4 *>(rec + tid);
+        const int4 h0 = rp[0];  // nflags, yMin, yMax, xMin
+        const int4 h1 = rp[1];  // xMax, ...
+        test = h0.y < oy + 8 && h0.z > oy && h0.w < ox + 8 && h1.x > ox;
+        if (hiz && test) {
+          const float zlo0 = __int_as_float(rp[2].w);                  // zlo
+          const float4 h3 = reinterpret_cast<const float4 *>(rp)[3];  // x0, y0, zA, zB
+          const float4 h4 = reinterpret_cast<const float4 *>(rp)[4];  // zC, zBias, ...
+          const float x0 = h3.x, y0 = h3.y, zA = h3.z, zB = h3.w, zC = h4.x;
+          const float zBias = depthBias ? h4.y : 0.0f;
+          // Lower bound of the evaluated plane over this block (sample offsets
+          // included), tightened with the primitive's bound over its box.
+          const float xa = (float)ox - 0.5f - x0, xb = (float)(ox + 7) + 0.5f - x0;
+          const float ya = (float)oy - 0.5f - y0, yb = (float)(oy + 7) + 0.5f - y0;
+          const float m =
+              fminf(fminf(zA * xa + zB * ya, zA * xb + zB * ya), fminf(zA * xa + zB * yb, zA * xb + zB * yb)) + zC +
+              zBias;
+          const float mag = fabsf(zA) * fmaxf(fabsf(xa), fabsf(xb)) + fabsf(zC) +
+                            2.0f * fabsf(zB) * fmaxf(fabsf(ya), fabsf(yb)) + 2.0f * fabsf(zBias);
+          float zl = fmaxf(zlo0, m - mag * 0x1p-19f);
+          if (!(zl == zl)) zl = -__builtin_inff();
+          zl = fminf(zl, P.depthClampHi);
+          if ((XF && P.depth16)) zl = d16_value(fmaxf(zl, 0.0f));  // the bound in stored units (monotone map)
+          test = !hidden(zl, zmax);
+          zlo = zl;
+        }
       }
+      const uint64_t tb = __ballot(test);
+      if (test) {
+        const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(tb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tb, 0));
+        ring[wave][(ringHead + ringCount + pos) & 127] = tid;
+        ringZ[wave][(ringHead + ringCount + pos) & 127] = zlo;
+      }
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      ringCount += (uint32_t)__builtin_popcountll(tb);
+      base += 64;
     }
-    nTests += test ? 1u : 0u;
-    const uint64_t tb = __ballot(test);
-    if (test) {
-      const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(tb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tb, 0));
-      ring[wave][(ringHead + ringCount + pos) & 127] = tid;
-      ringZ[wave][(ringHead + ringCount + pos) & 127] = zlo;
+    // A full batch, or what is left after the list's end.
+    if (ringCount >= 64 || base >= end) {
+      const uint32_t nb = ringCount < 64 ? ringCount : 64;
+      const bool act = (uint32_t)lane < nb;
+      const uint32_t t2 = act ? ring[wave][(ringHead + lane) & 127] : 0u;
+      const float z2 = act ? ringZ[wave][(ringHead + lane) & 127] : -__builtin_inff();
+      ringHead = (ringHead + nb) & 127;
+      ringCount -= nb;
+      process_chunk(act, t2, z2);
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    ringCount += (uint32_t)__builtin_popcountll(tb);
-    if (ringCount >= 64) {
-      const uint32_t t2 = ring[wave][(ringHead + lane) & 127];
-      const float z2 = ringZ[wave][(ringHead + lane) & 127];
-      ringHead = (ringHead + 64) & 127;
-      ringCount -= 64;
-      process_chunk(true, t2, z2);
-    }
-  }
-  while (ringCount > 0) {
-    const uint32_t nb = ringCount < 64 ? ringCount : 64;
-    const bool act = (uint32_t)lane < nb;
-    const uint32_t t2 = act ? ring[wave][(ringHead + lane) & 127] : 0u;
-    const float z2 = act ? ringZ[wave][(ringHead + lane) & 127] : -__builtin_inff();
-    ringHead = (ringHead + nb) & 127;
-    ringCount -= nb;
-    process_chunk(act, t2, z2);
   }
   if (qCount) flush();
 
@@ -614,17 +752,15 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     }
   }
 
-  // Counters: reduce over the wave, then over the workgroup, so that one
-  // atomic per counter and workgroup reaches the (single) global address.
+  // Counters: summed over the workgroup, so that one atomic per counter and
+  // workgroup reaches the (single) global address.
   __shared__ unsigned long long red[4][4];
   if (P.occlusion || P.stats) {
-    unsigned long long v[4] = {occl, nTests, nCovers, nShaded};
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-      for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
     if (lane == 0) {
-#pragma unroll
-      for (int k = 0; k < 4; k++) red[wave][k] = v[k];
+      red[wave][0] = occl;
+      red[wave][1] = nTests;
+      red[wave][2] = nCovers;
+      red[wave][3] = nShaded;
     }
     __syncthreads();
     if (threadIdx.x < 4) {
