@@ -609,7 +609,8 @@ int variant_of(const DrawParams &P) {
                     P.tex.addrU == P.tex.addrV && P.tex.addrU <= 1 &&
                     (P.tex.filter == FILT_LINEAR || P.tex.filter == FILT_ANISOTROPIC);
   const int level = fast ? 2 + P.tex.addrU : simple ? 1 : 0;
-  return (level << 4) | (xf ? 8 : 0) | (P.ms > 1 ? 4 : 0) | (P.colorFloat ? 2 : 0) | (ftex ? 1 : 0);
+  return level * kVarLevel1 | (xf ? kVarExtended : 0) | (P.blendEnable ? kVarBlend : 0) | (P.ms > 1 ? kVarSamples : 0) |
+         (P.colorFloat ? kVarFloatColor : 0) | (ftex ? kVarFloatTex : 0);
 }
 
 // Host plan of a batch: per-draw state in enqueue order, split into
@@ -784,15 +785,15 @@ int upload_layout(DeviceCtx *c, Pipeline &pipe, const BatchLayout &L, hipStream_
 }
 
 // Device words of Pipeline::counters: the persistent raster workgroups'
-// tile counters in [0, 80) (one per raster variant: at most 40 variants),
+// tile counters in [0, kVarCount) (one per raster variant of the segment),
 // the eager draws' overflow word, the segment's split
 // slot, the number of pairs the segment emitted and the backward's two work
 // counters.
-constexpr int kOverflowSlot = 80;
-constexpr int kSplitSlot = 81;
-constexpr int kEmittedSlot = 82;
-constexpr int kBackwardSlot = 84;
-constexpr int kCounterWords = 88;
+constexpr int kOverflowSlot = kVarCount;
+constexpr int kSplitSlot = kOverflowSlot + 1;
+constexpr int kEmittedSlot = kOverflowSlot + 2;
+constexpr int kBackwardSlot = kOverflowSlot + 4;
+constexpr int kCounterWords = kOverflowSlot + 8;
 
 // 8-bit radix passes that order every tile key below the key 0xFFFFFFFF of
 // unused capacity and dropped pairs: 2^(8 passes) > tiles, so the sorted
@@ -945,7 +946,7 @@ int enqueue_back(DeviceCtx *c, Pipeline &pipe, const BatchLayout &L, const Batch
     uint32_t *counters = pipe.counters.as<uint32_t>();
     const bool persistent = tuning.raster_workgroups_per_cu != ~0u;
     const uint32_t nv = (uint32_t)sg.variants.size();
-    if (persistent && !zeroed) hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, counters, 0u, nv);
+    if (persistent && !zeroed) hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(128), 0, s, counters, 0u, nv);
     // One launch per variant; with `unbinned`, each tile renders its binned
     // list and then the slots left out of it.
     for (uint32_t v = 0; v < nv; v++) {
@@ -975,8 +976,11 @@ int enqueue_back(DeviceCtx *c, Pipeline &pipe, const BatchLayout &L, const Batch
       a.split = split;
       a.segT = sg.T;
       const int var = variant_of(L.P[sg.first + lo]);
-      if (var >> 4 && !(var & 8)) launch_raster_common(var, dim3(wgs), block, s, a);
-      else launch_raster_general(var, dim3(wgs), block, s, a);
+      const bool common = (var & kVarLevel) != 0;
+      if (var & kVarBlend)
+        (common ? launch_raster_common<true> : launch_raster_general<true>)(var, dim3(wgs), block, s, a);
+      else
+        (common ? launch_raster_common<false> : launch_raster_general<false>)(var, dim3(wgs), block, s, a);
     }
   } else if (es) {
     SWR_HIP_CHECK(hipEventRecord(es->ev[EV_BIN], s));

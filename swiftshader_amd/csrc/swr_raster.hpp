@@ -7,7 +7,7 @@
 //                    list in order: coverage, stencil, depth, shading, blend.
 //
 // The kernel's variants are compiled in translation units of their own
-// (swr_raster_common.hip, swr_raster_general.hip), in parallel with the rest.
+// (swr_raster_{blend,opaque}_{common,general}.hip), in parallel with the rest.
 //
 // Reference semantics: src/Device/QuadRasterizer.cpp,
 // src/Pipeline/PixelRoutine.cpp, src/Pipeline/PixelProgram.cpp,
@@ -185,13 +185,19 @@ __device__ __forceinline__ int wave_max_i32(int v) {
   return __builtin_amdgcn_readlane(v, 63);
 }
 
-template <int MS, bool FCOL>
+// What a wave keeps of its block, per lane one pixel.  With BLEND the colours
+// themselves; without it the primitive that last wrote each sample: an
+// unblended fragment is replaced whole by the next one, so only the last one
+// of a sample is shaded, once the list is done (4.7 fragments a pixel pass
+// the depth test where 20 to 60 layers overlap).
+template <int MS, bool FCOL, bool BLEND>
 struct PixelState {
   float zb[MS];
   uint32_t sb[MS];
-  uint32_t cb[FCOL ? 1 : MS];
-  float4 cf[FCOL ? MS : 1];
-  uint32_t id[FCOL ? MS : 1];  // primitive_id record (float targets only)
+  uint32_t cb[BLEND && !FCOL ? MS : 1];
+  float4 cf[BLEND && FCOL ? MS : 1];
+  uint32_t id[BLEND && FCOL ? MS : 1];  // primitive_id record (float targets only)
+  uint32_t last[BLEND ? 1 : MS];        // 1 + record slot of the last writer, 0 for none
 };
 
 // Pixel of lane `l` inside its 8x8 block: lanes 4k..4k+3 form the 2x2 quad
@@ -204,7 +210,7 @@ __device__ __forceinline__ int lane_cy(int l) { return 2 * (l >> 4) + ((l >> 1) 
 // srgbLut: srgb_to_linear of every 8-bit code (sRGB targets).
 // FAST: blending, when on, is SRC_ALPHA, ONE_MINUS_SRC_ALPHA, ADD.
 template <int MS, bool FCOL, bool XF, bool FAST = false>
-__device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, FCOL> &S, float4 s, int xMask,
+__device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, FCOL, true> &S, float4 s, int xMask,
                                             uint32_t tri, const float *srgbLut) {
 #pragma unroll
   for (int q = 0; q < MS; q++) {
@@ -246,6 +252,53 @@ __device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, 
   }
 }
 
+// Writes an unblended shaded colour to a pixel's samples selected by xMask
+// (masked channels keep what the attachment holds), and the primitive_id
+// record of float targets.
+template <int MS, bool FCOL, bool XF>
+__device__ __forceinline__ void store_color(const DrawParams &P, int colorMask, int px, int py, float4 o, int xMask,
+                                            uint32_t tri) {
+  uint32_t o8 = 0;
+  if (!FCOL) {
+    if (XF && P.colorSRGB) {  // writeColor encodes R, G, B first (PixelRoutine.cpp:1963-1969)
+      o.x = linear_to_srgb(o.x);
+      o.y = linear_to_srgb(o.y);
+      o.z = linear_to_srgb(o.z);
+    }
+    o8 = float_to_unorm8(o.x) | (float_to_unorm8(o.y) << 8) | (float_to_unorm8(o.z) << 16) | (float_to_unorm8(o.w) << 24);
+    o8 = bgra_swap(XF && P.colorBGRA, o8);
+  }
+#pragma unroll
+  for (int q = 0; q < MS; q++) {
+    if (!((xMask >> q) & 1)) continue;
+    char *at = P.color + q * P.colorSlice + (long long)py * P.colorPitch + (FCOL ? 16ll : 4ll) * px;
+    if (FCOL) {
+      float4 c = o;
+      if (colorMask != 15) {
+        const float4 d = *reinterpret_cast<const float4 *>(at);
+        c.x = (colorMask & 1) ? c.x : d.x;
+        c.y = (colorMask & 2) ? c.y : d.y;
+        c.z = (colorMask & 4) ? c.z : d.z;
+        c.w = (colorMask & 8) ? c.w : d.w;
+      }
+      *reinterpret_cast<float4 *>(at) = c;
+      if (P.primId)
+        *reinterpret_cast<uint32_t *>(P.primId + q * P.primIdSlice + (long long)py * P.primIdPitch + 4ll * px) =
+            tri - (uint32_t)P.triBase + 1u;
+    } else {
+      uint32_t c = o8;
+      if (colorMask != 15) {
+        const uint32_t wm = bgra_swap(XF && P.colorBGRA, ((colorMask & 1) ? 0x000000FFu : 0u) |
+                                                             ((colorMask & 2) ? 0x0000FF00u : 0u) |
+                                                             ((colorMask & 4) ? 0x00FF0000u : 0u) |
+                                                             ((colorMask & 8) ? 0xFF000000u : 0u));
+        c = (*reinterpret_cast<const uint32_t *>(at) & ~wm) | (c & wm);
+      }
+      *reinterpret_cast<uint32_t *>(at) = c;
+    }
+  }
+}
+
 constexpr int kQueue = 64;  // deferred-shading queue entries per wave
 
 // One screen tile of draw P: `bin` is the tile's index in the draw's tile
@@ -255,7 +308,8 @@ constexpr int kQueue = 64;  // deferred-shading queue entries per wave
 // depth and writes all four colour channels (the checks below fold away).
 // LEVEL 2 (3): also the common shading state with REPEAT (CLAMP_TO_EDGE)
 // addressing (shade's FA, blend_write's FAST).
-template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL>
+// BLEND: the draw blends (see PixelState).
+template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL, bool BLEND>
 __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32_t start, uint32_t end0,
                                             const TriRecord *__restrict__ rec, const int *__restrict__ poly,
                                             const uint32_t *__restrict__ binTri) {
@@ -267,9 +321,10 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   const int colorMask = SIMPLE ? 15 : P.colorMask;
   // Per-wave queue of fragments that passed the tests and await shading,
   // in API order: primitive, owner lane | sample mask << 8, shaded colour.
-  __shared__ uint32_t qTri[4][kQueue];
-  __shared__ uint32_t qPix[4][kQueue];
-  __shared__ float4 qCol[4][kQueue];
+  constexpr bool QUEUE = BLEND || MS > 1;  // without blending, one pixel is one fragment unless it has samples
+  __shared__ uint32_t qTri[QUEUE ? 4 : 1][QUEUE ? kQueue : 1];
+  __shared__ uint32_t qPix[QUEUE ? 4 : 1][QUEUE ? kQueue : 1];
+  __shared__ float4 qCol[QUEUE ? 4 : 1][QUEUE ? kQueue : 1];
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -297,30 +352,31 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   }
   const bool inside = (scissorMask >> myBit) & 1;
 
-  PixelState<MS, FCOL> S;
+  PixelState<MS, FCOL, BLEND> S;
 #pragma unroll
   for (int q = 0; q < MS; q++) {
     S.zb[q] = 0.0f;
     S.sb[q] = 0;
-    if (!FCOL) S.cb[FCOL ? 0 : q] = 0;
-    if (FCOL) S.cf[FCOL ? q : 0] = make_float4(0, 0, 0, 0);
-    if (FCOL) S.id[FCOL ? q : 0] = 0;
+    if constexpr (!BLEND) S.last[q] = 0;
+    else if constexpr (FCOL) S.cf[q] = make_float4(0, 0, 0, 0), S.id[q] = 0;
+    else S.cb[q] = 0;
     if (!inside) continue;
-    if (FCOL && P.primId)
-      S.id[FCOL ? q : 0] =
-          *reinterpret_cast<const uint32_t *>(P.primId + q * P.primIdSlice + (long long)py * P.primIdPitch + 4ll * px);
+    if constexpr (BLEND && FCOL)
+      if (P.primId)
+        S.id[q] = *reinterpret_cast<const uint32_t *>(P.primId + q * P.primIdSlice + (long long)py * P.primIdPitch +
+                                                      4ll * px);
     if (depthTest || (XF && P.depthBounds))  // D16 holds the float of its integer (readDepth16, PixelRoutine.cpp:466-481)
       S.zb[q] = (XF && P.depth16) ? (float)*reinterpret_cast<const uint16_t *>(P.depth + q * P.depthSlice +
                                                                         (long long)py * P.depthPitch + 2ll * px)
                           : *reinterpret_cast<const float *>(P.depth + q * P.depthSlice +
                                                              (long long)py * P.depthPitch + 4ll * px);
     if (stencilActive) S.sb[q] = (uint8_t)P.stencil[q * P.stencilSlice + (long long)py * P.stencilPitch + px];
-    if (colorMask) {
-      if (FCOL)
-        S.cf[FCOL ? q : 0] =
+    if constexpr (BLEND) {
+      if constexpr (FCOL)
+        S.cf[q] =
             *reinterpret_cast<const float4 *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 16ll * px);
       else
-        S.cb[FCOL ? 0 : q] = bgra_swap(
+        S.cb[q] = bgra_swap(
             (XF && P.colorBGRA),
             *reinterpret_cast<const uint32_t *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 4ll * px));
     }
@@ -328,8 +384,8 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 
   // The 256 decoded codes of an sRGB target that is blended, so that a blend
   // reads its three channels instead of evaluating three powers.
-  __shared__ float srgbLut[XF ? 256 : 1];
-  if (XF && P.colorSRGB && P.blendEnable) {
+  __shared__ float srgbLut[XF && BLEND ? 256 : 1];
+  if (XF && BLEND && P.colorSRGB) {
     for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) srgbLut[i] = srgb_to_linear(unorm8_to_float(i));
     __syncthreads();
   }
@@ -346,6 +402,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   uint64_t myEntries = 0;   // queue slots holding fragments of this lane's pixel
 
   auto flush = [&]() __attribute__((always_inline)) {
+    if constexpr (!QUEUE) return;
     // Shade the queued fragments, one per lane...
     if (lane < qCount) {
       const uint32_t t = qTri[wave][lane];
@@ -355,17 +412,36 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // ...then blend them into their pixels in queue (API) order.
+    // ...then blend them into their pixels in queue (API) order, or write them.
     uint64_t m = myEntries;
     while (m) {
       const int k = __builtin_ctzll(m);
       m &= m - 1;
-      blend_write<MS, FCOL, XF, FAST>(P, S, qCol[wave][k], (int)(qPix[wave][k] >> 8), qTri[wave][k], srgbLut);
+      if constexpr (BLEND)
+        blend_write<MS, FCOL, XF, FAST>(P, S, qCol[wave][k], (int)(qPix[wave][k] >> 8), qTri[wave][k], srgbLut);
+      else
+        store_color<MS, FCOL, XF>(P, colorMask, px, py, qCol[wave][k], (int)(qPix[wave][k] >> 8), qTri[wave][k]);
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     myEntries = 0;
     qCount = 0;
+  };
+
+  // Queues the fragment of the lanes that `want` it: primitive tri on their
+  // pixel's samples xMask.
+  auto enqueue = [&](bool want, uint32_t tri, uint32_t xMask) __attribute__((always_inline)) {
+    const uint64_t need = __ballot(want);
+    const int cnt = __builtin_popcountll(need);
+    if (qCount + cnt > kQueue) flush();
+    if (want) {
+      const int pos = qCount + __builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
+      qTri[wave][pos] = tri;
+      qPix[wave][pos] = (uint32_t)lane | (xMask << 8);
+      myEntries |= 1ull << pos;
+    }
+    qCount += cnt;
   };
 
   // Largest stored depth of the block (+inf when any is NaN): a primitive
@@ -390,7 +466,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   };
 
   // Coverage masks of a batch's primitives that take the spans.
-  __shared__ uint64_t spanMask[4][MS][64];
+  __shared__ uint32_t spanMask[4][2 * MS][64];  // (sample, half) of the block
   const int pixelStep = (int)((uint32_t)(16 * cx) | ((uint32_t)(-16 * cy) << 16));
 
   // One batch of up to 64 candidates in list order: each lane sets up one
@@ -445,13 +521,13 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
             Yo = pp[kMaxPolygon + i];
           }
         };
-        uint64_t any = 0;
+        uint32_t any = 0;
 #pragma unroll
         for (int q = 0; q < MS; q++) {
           const int xo = (MS > 1) ? kXf[q] : 0, yo = (MS > 1) ? kYf[q] : 0;
           const uint64_t m = block_coverage(vtx, n, d, xo, yo, ox, oy);
-          spanMask[wave][q][lane] = m;
-          any |= m;
+          spanMask[wave][2*q][lane] = (uint32_t)m; spanMask[wave][2*q+1][lane] = (uint32_t)(m>>32);
+          any |= (uint32_t)m | (uint32_t)(m>>32);
         }
         act = any != 0;
       }
@@ -488,7 +564,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
         }
       } else {
 #pragma unroll
-        for (int q = 0; q < MS; q++) cov[q] = cov[q] && ((spanMask[wave][q][j] >> myBit) & 1);
+        for (int q = 0; q < MS; q++) cov[q] = cov[q] && ((spanMask[wave][2 * q + (myBit >> 5)][j] >> (myBit & 31)) & 1);
       }
       nTests++;
       bool anyCov = false;
@@ -613,28 +689,22 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
         }
       }
 
-      bool anyPass = false;
+      uint32_t xMask = 0;
 #pragma unroll
-      for (int q = 0; q < MS; q++) anyPass |= pass[q];
-      const uint64_t need = __ballot(anyPass);
+      for (int q = 0; q < MS; q++) xMask |= pass[q] ? 1u << q : 0u;
+      const uint64_t need = __ballot(xMask != 0);
       if (!need) continue;
       if (colorMask) {
-        // Queue the fragments that write colour; shading is deferred so that
-        // it runs with every lane busy.
-        const int cnt = __builtin_popcountll(need);
-        if (qCount + cnt > kQueue) flush();
-        if (anyPass) {
-          const int pos = qCount + __builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
-                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
-          uint32_t xMask = 0;
+        const uint32_t tj = __builtin_amdgcn_readlane(tid, j);
+        // Shading is deferred so that it runs with every lane busy: blended
+        // fragments queue, others leave their primitive's slot.
+        if constexpr (BLEND) {
+          enqueue(xMask != 0, tj, xMask);
+        } else {
 #pragma unroll
-          for (int q = 0; q < MS; q++) xMask |= pass[q] ? 1u << q : 0u;
-          qTri[wave][pos] = __builtin_amdgcn_readlane(tid, j);
-          qPix[wave][pos] = (uint32_t)lane | (xMask << 8);
-          myEntries |= 1ull << pos;
+          for (int q = 0; q < MS; q++) S.last[q] = pass[q] ? tj + 1u : S.last[q];
         }
-        qCount += cnt;
-        nShaded += (unsigned)cnt;
+        nShaded += (unsigned)__builtin_popcountll(need);
       }
       // What the block shows now may hide the rest of the batch.
       if (hiz && depthWrite && ++wrote >= kRetest && todo) {
@@ -724,7 +794,26 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
       process_chunk(act, t2, z2);
     }
   }
+  if constexpr (!BLEND && MS > 1) {
+    // One fragment per pixel and distinct last writer of its samples.
+#pragma unroll
+    for (int q = 0; q < MS; q++) {
+      bool first = S.last[q] != 0;
+      uint32_t xMask = 0;
+#pragma unroll
+      for (int k = 0; k < MS; k++) {
+        if (k < q) first = first && S.last[k] != S.last[q];
+        else xMask |= S.last[k] == S.last[q] ? 1u << k : 0u;
+      }
+      enqueue(first, S.last[q] - 1u, xMask);
+    }
+  }
   if (qCount) flush();
+  if constexpr (!BLEND && MS == 1)
+    if (S.last[0]) {
+      const uint32_t t = S.last[0] - 1u;
+      store_color<MS, FCOL, XF>(P, colorMask, px, py, shade<FCOL, FTEX, XF, FA>(P, rec[t], px, py), 1, t);
+    }
 
   // Write the block back.
   if (inside) {
@@ -738,16 +827,14 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
           *reinterpret_cast<float *>(P.depth + q * P.depthSlice + (long long)py * P.depthPitch + 4ll * px) = S.zb[q];
       }
       if (P.stencilWrite) P.stencil[q * P.stencilSlice + (long long)py * P.stencilPitch + px] = (char)S.sb[q];
-      if (FCOL && P.primId)
-        *reinterpret_cast<uint32_t *>(P.primId + q * P.primIdSlice + (long long)py * P.primIdPitch + 4ll * px) =
-            S.id[FCOL ? q : 0];
-      if (P.colorMask) {
-        if (FCOL)
-          *reinterpret_cast<float4 *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 16ll * px) =
-              S.cf[FCOL ? q : 0];
-        else
-          *reinterpret_cast<uint32_t *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 4ll * px) =
-              bgra_swap((XF && P.colorBGRA), S.cb[FCOL ? 0 : q]);
+      if constexpr (BLEND && FCOL) {
+        if (P.primId)
+          *reinterpret_cast<uint32_t *>(P.primId + q * P.primIdSlice + (long long)py * P.primIdPitch + 4ll * px) =
+              S.id[q];
+        *reinterpret_cast<float4 *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 16ll * px) = S.cf[q];
+      } else if constexpr (BLEND) {
+        *reinterpret_cast<uint32_t *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 4ll * px) =
+            bgra_swap((XF && P.colorBGRA), S.cb[q]);
       }
     }
   }
@@ -793,8 +880,8 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 // Occupancy: 4 waves per SIMD (128 VGPRs) for the single-sample kernels
 // (the float-colour ones spill 12 bytes there and still run faster than at
 // 3 waves), 3 for the multisample ones.
-template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL>
-__global__ __launch_bounds__(256, MS == 1 ? 4 : 3) void raster_batch_kernel(
+template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL, bool BLEND>
+__global__ __launch_bounds__(256, MS == 1 || !BLEND ? 4 : 3) void raster_batch_kernel(
                                                            const DrawParams *__restrict__ params,
                                                            const uint32_t *__restrict__ tileBase, int drawLo,
                                                            int drawHi, uint32_t tileLo, uint32_t tileHi,
@@ -842,32 +929,47 @@ __global__ __launch_bounds__(256, MS == 1 ? 4 : 3) void raster_batch_kernel(
         e = b + (uint32_t)params[lo].triCount;
       }
       if (s < e)
-        raster_tile<MS, FCOL, FTEX, XF, LEVEL>(params[lo], (int)(t - tileBase[lo]), s, e, rec, poly,
+        raster_tile<MS, FCOL, FTEX, XF, LEVEL, BLEND>(params[lo], (int)(t - tileBase[lo]), s, e, rec, poly,
                                                pass == 0 ? binTri : nullptr);
     }
   }
 }
 
-template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL>
+template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL, bool BLEND>
 void launch_raster_batch(dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
-  hipLaunchKernelGGL((raster_batch_kernel<MS, FCOL, FTEX, XF, LEVEL>), grid, block, 0, s, a.params, a.tileBase, a.lo,
-                     a.hi, a.tLo, a.tHi, a.counter, a.rec, a.poly, a.bin, a.ts, a.te, a.split, a.segT,
-                     a.tail);
+  hipLaunchKernelGGL((raster_batch_kernel<MS, FCOL, FTEX, XF, LEVEL, BLEND>), grid, block, 0, s, a.params, a.tileBase,
+                     a.lo, a.hi, a.tLo, a.tHi, a.counter, a.rec, a.poly, a.bin, a.ts, a.te, a.split, a.segT, a.tail);
 }
 
-// The raster kernel of variant v (variant_of).
-template <bool XF, int LEVEL>
+// The raster kernel of variant v.
+template <bool XF, int LEVEL, bool BLEND>
 void launch_raster_variant(int v, dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
-  switch (v & 7) {
-    case 0: launch_raster_batch<1, false, false, XF, LEVEL>(grid, block, s, a); break;
-    case 1: launch_raster_batch<1, false, true, XF, LEVEL>(grid, block, s, a); break;
-    case 2: launch_raster_batch<1, true, false, XF, LEVEL>(grid, block, s, a); break;
-    case 3: launch_raster_batch<1, true, true, XF, LEVEL>(grid, block, s, a); break;
-    case 4: launch_raster_batch<4, false, false, XF, LEVEL>(grid, block, s, a); break;
-    case 5: launch_raster_batch<4, false, true, XF, LEVEL>(grid, block, s, a); break;
-    case 6: launch_raster_batch<4, true, false, XF, LEVEL>(grid, block, s, a); break;
-    default: launch_raster_batch<4, true, true, XF, LEVEL>(grid, block, s, a); break;
+  switch (v & (kVarSamples | kVarFloatColor | kVarFloatTex)) {
+    case 0: launch_raster_batch<1, false, false, XF, LEVEL, BLEND>(grid, block, s, a); break;
+    case kVarFloatTex: launch_raster_batch<1, false, true, XF, LEVEL, BLEND>(grid, block, s, a); break;
+    case kVarFloatColor: launch_raster_batch<1, true, false, XF, LEVEL, BLEND>(grid, block, s, a); break;
+    case kVarFloatColor | kVarFloatTex: launch_raster_batch<1, true, true, XF, LEVEL, BLEND>(grid, block, s, a); break;
+    case kVarSamples: launch_raster_batch<4, false, false, XF, LEVEL, BLEND>(grid, block, s, a); break;
+    case kVarSamples | kVarFloatTex: launch_raster_batch<4, false, true, XF, LEVEL, BLEND>(grid, block, s, a); break;
+    case kVarSamples | kVarFloatColor: launch_raster_batch<4, true, false, XF, LEVEL, BLEND>(grid, block, s, a); break;
+    default: launch_raster_batch<4, true, true, XF, LEVEL, BLEND>(grid, block, s, a); break;
   }
+}
+
+// The kernels of the common output states (levels 1 to 3), and the rest.
+template <bool BLEND>
+void launch_raster_common(int v, dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
+  switch ((v & kVarLevel) / kVarLevel1) {
+    case 3: launch_raster_variant<false, 3, BLEND>(v, grid, block, s, a); break;
+    case 2: launch_raster_variant<false, 2, BLEND>(v, grid, block, s, a); break;
+    default: launch_raster_variant<false, 1, BLEND>(v, grid, block, s, a); break;
+  }
+}
+
+template <bool BLEND>
+void launch_raster_general(int v, dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
+  if (v & kVarExtended) launch_raster_variant<true, 0, BLEND>(v, grid, block, s, a);
+  else launch_raster_variant<false, 0, BLEND>(v, grid, block, s, a);
 }
 
 }  // namespace swr

@@ -1,0 +1,4 @@
+// swr_raster_opaque_common.hip -- raster kernels of draws that do not blend, for the common output states (levels 1 to 3).
+#include "swr_raster.hpp"
+
+template void swr::launch_raster_common<false>(int, dim3, dim3, hipStream_t, const swr::RasterArgs &);
