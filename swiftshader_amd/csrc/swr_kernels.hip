@@ -209,6 +209,34 @@ struct PolyWork {
   int X[kMaxPolygon], Y[kMaxPolygon];
 };
 
+// Whether polygon X, Y (n >= 3, coordinates below 2^20) is convex on the 28.4
+// grid, with no repeated vertex: every turn goes the same way or straight on,
+// and the edges change between downward and upward twice (one revolution).
+__device__ __forceinline__ bool convex_polygon(const int (&X)[kMaxPolygon], const int (&Y)[kMaxPolygon], int n) {
+  bool left = false, right = false, back = false;
+  int changes = 0, dir = 0, firstDir = 0;
+  int dx0 = X[0] - X[n - 1], dy0 = Y[0] - Y[n - 1];
+  for (int i = 0; i < n; i++) {
+    const int k = i + 1 < n ? i + 1 : 0;
+    const int dx1 = X[k] - X[i], dy1 = Y[k] - Y[i];
+    const long long c = (long long)dx0 * dy1 - (long long)dy0 * dx1;
+    left |= c > 0;
+    right |= c < 0;
+    // Straight on, and neither edge of zero length.
+    back |= c == 0 && (long long)dx0 * dx1 + (long long)dy0 * dy1 <= 0;
+    const int s = dy1 > 0 ? 1 : (dy1 < 0 ? -1 : 0);
+    if (s) {
+      if (!firstDir) firstDir = s;
+      else if (s != dir) changes++;
+      dir = s;
+    }
+    dx0 = dx1;
+    dy0 = dy1;
+  }
+  if (dir != firstDir) changes++;
+  return !(left && right) && !back && changes == 2;
+}
+
 // Setup of primitive t of the draw P, written to record slot g (the
 // primitive's index in the batch); `draw` is the draw's index in the batch;
 // w holds the polygon path's arrays.  Without POLY, the primitives that need
@@ -338,6 +366,7 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
     xLo = min(min(PX[0], PX[1]), PX[2]);
     xHi = max(max(PX[0], PX[1]), PX[2]);
   }
+  const int yLo = yMin, yHi = yMax;
   if (P.ms > 1) {
     yMin = wadd(yMin, 9) >> 4;   // yMinMultiSampleOffset (Constants.hpp:51)
     yMax = wadd(yMax, 21) >> 4;  // yMaxMultiSampleOffset (Constants.hpp:52)
@@ -493,14 +522,11 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
     int *pp = poly + g * (2 * kMaxPolygon);
     for (int i = 0; i < n; i++) { pp[i] = X[i]; pp[kMaxPolygon + i] = Y[i]; }
   }
-  int planes = 0;
-  if (n == 3) {
-    const int a0 = isPolygon ? X[0] : PX[0], a1 = isPolygon ? X[1] : PX[1], a2 = isPolygon ? X[2] : PX[2];
-    const int b0 = isPolygon ? Y[0] : PY[0], b1 = isPolygon ? Y[1] : PY[1], b2 = isPolygon ? Y[2] : PY[2];
-    const int lo = min(min(min(a0, a1), a2), min(min(b0, b1), b2)), hi = max(max(max(a0, a1), a2), max(max(b0, b1), b2));
-    const int ex = wsub(max(max(a0, a1), a2), min(min(a0, a1), a2)), ey = wsub(max(max(b0, b1), b2), min(min(b0, b1), b2));
-    if (lo > -(1 << 20) && hi < (1 << 20) && ex <= 32767 && ey <= 32767) planes = kRecHalfPlanes;
-  }
+  // An unclipped triangle is convex; a polygon is when its turns agree.
+  const int ext = 32767, big = 1 << 20;
+  const int xMinV = xLo, xMaxV = xHi;
+  const bool small = xMinV > -big && xMaxV < big && yLo > -big && yHi < big && wsub(xMaxV, xMinV) <= ext && wsub(yHi, yLo) <= ext;
+  const int planes = small && (!isPolygon || n == 3 || (n <= kMaxHalfPlanes && convex_polygon(X, Y, n))) ? kRecHalfPlanes : 0;
   R.nflags = n | (d << 8) | (frontFacing ? 1 << 9 : 0) | planes;
   // Tiles are 8 or 16 pixels a side and xMin, yMin >= 0 (scissor-clamped to
   // a render area at x, y >= 0): shifts divide exactly.

@@ -145,10 +145,12 @@ struct TriRecord {
   int draw;         // index of the primitive's draw in its batch
 };
 
-// Triangle (n == 3) whose coverage is three half planes with 16-bit edge
-// extents: coordinates below 2^20 and edges up to 32767 (28.4), so that the
-// half planes step over a block with one 16-bit dot product each.
+// A polygon whose coverage is its half planes: convex, at most
+// kMaxHalfPlanes vertices, coordinates below 2^20 and edges up to 32767
+// (28.4), so that each half plane steps over a block with one 16-bit dot
+// product.
 constexpr int kRecHalfPlanes = 1 << 10;
+constexpr int kMaxHalfPlanes = 5;
 
 static_assert(sizeof(TriRecord) == 160, "TriRecord layout");
 

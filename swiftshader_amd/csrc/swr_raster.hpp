@@ -27,11 +27,10 @@ namespace swr {
 
 // Standard 4x sample locations relative to the pixel centre
 // (Constants.hpp:26-47) and their 28.4 offsets Xf/Yf (Constants.cpp:291-297).
-__device__ __constant__ const float kSampleX[4] = {-0.125f, 0.375f, -0.375f, 0.125f};
-__device__ __constant__ const float kSampleY[4] = {-0.375f, -0.125f, 0.125f, 0.375f};
-__device__ __constant__ const int kXf[4] = {-2, 6, -6, 2};
-__device__ __constant__ const int kYf[4] = {-6, -2, 2, 6};
-constexpr int kXf0 = -2, kYf0 = -6, kXf1 = 6, kYf1 = -2;  // of samples 0 and 1; 2 and 3 lie opposite 1 and 0
+constexpr float kSampleX[4] = {-0.125f, 0.375f, -0.375f, 0.125f};
+constexpr float kSampleY[4] = {-0.375f, -0.125f, 0.125f, 0.375f};
+constexpr int kXf[4] = {-2, 6, -6, 2};
+constexpr int kYf[4] = {-6, -2, 2, 6};
 
 // D16 compares and stores Min(Max(Round(z * 0xFFFF), 0), 0xFFFF) of the
 // clamped depth (PixelRoutine.cpp:506-510, 686-711; Round is to nearest even).
@@ -66,53 +65,42 @@ __device__ __forceinline__ uint32_t bgra_swap(int bgra, uint32_t v) {
 // "ceil(Xe/16) <= x" is exactly E >= 0 and "x < ceil(Xe/16)" is exactly
 // E < 0, so the span test becomes two integer sign tests per sample.
 //
-// A triangle (n == 3) needs no spans: over the rows it spans, one left and
-// one right edge bound each row, so the rule equals three half planes.  With
-// an edge a -> b in the order the reference walks it (interior at F > 0),
+// A convex polygon needs no spans: over the rows it meets, one left and one
+// right edge bound each row, so the rule equals its half planes.  With an
+// edge a -> b in the order the reference walks it (interior at F > 0),
 //   F(x, y) = (Yb - Ya) * (16 x - Xa) - (Xb - Xa) * (16 y - Ya),
 // a sample is covered iff F >= 0 for left edges (Yb > Ya) and for horizontal
 // top edges (Yb == Ya, Xb < Xa), and F > 0 for the others: left edges have
 // F = E, right ones F = -E, and the horizontal ones keep the row range.  The
-// three F add up to a constant (twice the area, signed by the winding), so a
-// degenerate triangle, or one whose winding the float determinant of the
-// setup misjudged, covers nothing under either rule.  F at the block origin
-// is formed in 64 bits and clamped to +-2^30: beyond that its sign cannot
-// change inside the block.  Edge extents below 2^15 (triangles up to 2047
-// pixels) make the step over the block one 16-bit dot product; larger
-// triangles and clipped polygons, lines and points take the spans.
+// F of a polygon add up to a constant (twice the area, signed by the
+// winding), so a degenerate polygon, or one whose winding the float
+// determinant of the setup misjudged, covers nothing under either rule.  F
+// at the block origin is formed in 64 bits and clamped to +-2^30: beyond that
+// its sign cannot change inside the block.  Edge extents below 2^15 (2047
+// pixels) make the step over the block one 16-bit dot product.  The setup
+// marks the polygons that qualify (kRecHalfPlanes: all but the largest
+// triangles, and what clipping leaves convex on the 28.4 grid); the rest
+// take the spans, edge by edge.
 
-struct LaneEdge {
-  int e;      // E at the block origin (clamped)
-  int ex;     // dE / dx (16 DY > 0)
-  int ey;     // dE / dy (-16 DX)
-  int y1, y2; // rows the edge spans
-  int right;  // writes the right span
-};
-
-__device__ __forceinline__ LaneEdge lane_edge(int Xa, int Ya, int Xb, int Yb, int ox, int oy) {
-  LaneEdge E;
-  const bool swap = Yb < Ya;
-  const int X1 = swap ? Xb : Xa, X2 = swap ? Xa : Xb;
-  const int Y1 = swap ? Yb : Ya, Y2 = swap ? Ya : Yb;
-  const int DX = X2 - X1, DY = Y2 - Y1;
-  E.y1 = (Y1 + 15) >> 4;  // a horizontal edge gets y1 == y2 and spans no row
-  E.y2 = (Y2 + 15) >> 4;
-  long long v = (long long)DY * (long long)(16 * ox - X1) - (long long)DX * (long long)(16 * oy - Y1);
+// Edge a -> b of a convex polygon as its half plane over the block at
+// (ox, oy): pk holds (Yb - Ya, Xb - Xa) as 16-bit halves, and the sample at
+// 28.4 offset (x, y) from the block's origin is inside iff
+// dot2(pk, (x, -y)) + f >= 0.
+__device__ __forceinline__ void half_plane(int Xa, int Ya, int Xb, int Yb, int ox, int oy, int &f, int &pk) {
+  const int DX = Xb - Xa, DY = Yb - Ya;
+  const bool closed = DY > 0 || (DY == 0 && DX < 0);
+  const long long v = (long long)DY * (long long)(16 * ox - Xa) - (long long)DX * (long long)(16 * oy - Ya);
   const long long lim = 1ll << 30;
-  E.e = (int)(v > lim ? lim : (v < -lim ? -lim : v));
-  E.ex = 16 * DY;
-  E.ey = -16 * DX;
-  E.right = swap ? 1 : 0;
-  return E;
+  f = (int)(v > lim ? lim : (v < -lim ? -lim : v)) - (closed ? 0 : 1);
+  pk = (int)(((uint32_t)DY & 0xFFFFu) | ((uint32_t)DX << 16));
 }
 
-// Coverage mask (bit r*8+c = pixel (ox+c, oy+r)) of polygon (X, Y, n) for
-// the sample at 28.4 offset (xo, yo), before the scissor mask is applied.
+// The span rule at one sample point (28.4): whether the last left-writing
+// edge spanning its row lies at or left of it, and the last right-writing one
+// right of it.  Wave-uniform polygon, one point per lane.
 template <typename VFetch>
-__device__ __forceinline__ uint64_t block_coverage(const VFetch &vtx, int n, int d, int xo, int yo, int ox, int oy) {
-  int Lv[8], Lx[8], Rv[8], Rx[8];
-#pragma unroll
-  for (int r = 0; r < 8; r++) { Lv[r] = -1; Lx[r] = 0; Rv[r] = 0; Rx[r] = 0; }
+__device__ __forceinline__ bool span_covers(const VFetch &vtx, int n, int d, int x, int y) {
+  bool left = false, right = false;
   for (int i = 0; i < n; i++) {
     int ia = i + 1 - d, ib = i + d;
     ia = ia >= n ? ia - n : ia;
@@ -120,57 +108,20 @@ __device__ __forceinline__ uint64_t block_coverage(const VFetch &vtx, int n, int
     int Xa, Ya, Xb, Yb;
     vtx(ia, Xa, Ya);
     vtx(ib, Xb, Yb);
-    const LaneEdge E = lane_edge(Xa - xo, Ya - yo, Xb - xo, Yb - yo, ox, oy);
-    // Rows of the block the edge spans, as a bit mask, routed to the left or
-    // right span; each row then takes (E, dE/dx) under a select mask
-    // (bitfield insert), so the update has no branches.
-    const int r1 = min(max(E.y1 - oy, 0), 8), r2 = min(max(E.y2 - oy, 0), 8);
-    const uint32_t rows = (0xFFu << r1) & ~(0xFFu << r2) & 0xFFu;
-    const uint32_t rowsR = E.right ? rows : 0u, rowsL = rows ^ rowsR;
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-      const int v = E.e + E.ey * r;
-      const uint32_t ml = 0u - ((rowsL >> r) & 1u), mr = 0u - ((rowsR >> r) & 1u);
-      Lv[r] = (int)(((uint32_t)v & ml) | ((uint32_t)Lv[r] & ~ml));
-      Lx[r] = (int)(((uint32_t)E.ex & ml) | ((uint32_t)Lx[r] & ~ml));
-      Rv[r] = (int)(((uint32_t)v & mr) | ((uint32_t)Rv[r] & ~mr));
-      Rx[r] = (int)(((uint32_t)E.ex & mr) | ((uint32_t)Rx[r] & ~mr));
-    }
+    const bool swap = Yb < Ya;
+    const int X1 = swap ? Xb : Xa, X2 = swap ? Xa : Xb;
+    const int Y1 = swap ? Yb : Ya, Y2 = swap ? Ya : Yb;
+    const long long E = (long long)(Y2 - Y1) * (long long)(x - X1) - (long long)(X2 - X1) * (long long)(y - Y1);
+    const bool spans = Y1 <= y && y < Y2;
+    if (swap) right = spans ? E < 0 : right;
+    else left = spans ? E >= 0 : left;
   }
-  uint64_t mask = 0;
-#pragma unroll
-  for (int r = 0; r < 8; r++) {
-    // Covered iff lv >= 0 && rv < 0, i.e. the sign bit of (rv & ~lv).
-    int lv = Lv[r] + 7 * Lx[r], rv = Rv[r] + 7 * Rx[r];
-    uint32_t bits = 0;
-#pragma unroll
-    for (int c = 7; c >= 0; c--) {
-      bits = (bits << 1) | ((uint32_t)(rv & ~lv) >> 31);
-      lv -= Lx[r];
-      rv -= Rx[r];
-    }
-    mask |= (uint64_t)bits << (8 * r);
-  }
-  return mask;
-}
-
-// Edge a -> b of a triangle as its half plane over the block at (ox, oy):
-// `pk` holds (Yb - Ya, Xb - Xa) as 16-bit halves, and the pixel at (cx, cy)
-// of the block is inside iff dot2(pk, (16 cx, -16 cy)) >= nf (the sample at
-// 28.4 offset (xo, yo) iff the dot product >= nf - (DY xo - DX yo)).
-__device__ __forceinline__ void half_plane(int Xa, int Ya, int Xb, int Yb, int ox, int oy, int &pk, int &nf) {
-  const int DX = Xb - Xa, DY = Yb - Ya;
-  const bool closed = DY > 0 || (DY == 0 && DX < 0);
-  const long long v = (long long)DY * (long long)(16 * ox - Xa) - (long long)DX * (long long)(16 * oy - Ya);
-  const long long lim = 1ll << 30;
-  const int f = (int)(v > lim ? lim : (v < -lim ? -lim : v));
-  pk = (int)(((uint32_t)DY & 0xFFFFu) | ((uint32_t)DX << 16));
-  nf = (closed ? 0 : 1) - f;
+  return left && right;
 }
 
 typedef short Short2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ int dot2_i16(int a, int b) {
-  return __builtin_amdgcn_sdot2(__builtin_bit_cast(Short2, a), __builtin_bit_cast(Short2, b), 0, false);
+__device__ __forceinline__ int dot2_i16(int a, int b, int c) {
+  return __builtin_amdgcn_sdot2(__builtin_bit_cast(Short2, a), __builtin_bit_cast(Short2, b), c, false);
 }
 
 // Largest value of v over the wave (wave-uniform), by DPP: the old value of
@@ -465,18 +416,24 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     return P.depthCompare == 1 ? zl >= zmax : zl > zmax;
   };
 
-  // Coverage masks of a batch's primitives that take the spans.
-  __shared__ uint32_t spanMask[4][2 * MS][64];  // (sample, half) of the block
-  const int pixelStep = (int)((uint32_t)(16 * cx) | ((uint32_t)(-16 * cy) << 16));
+  // One batch of candidates, set up one per lane and then read back one at a
+  // time by the whole wave (a broadcast, which leaves the vector units the
+  // arithmetic): half planes 0 to 2 as (f, pk), x0, y0, zA, zB, zC, zBias;
+  // half planes 3 and 4 of the polygons that have them.
+  __shared__ int4 cand[4][3][64];
+  __shared__ int4 candMore[4][64];
+  int step[MS];  // the pixel's samples from the block's origin, as half_plane's operand
+#pragma unroll
+  for (int q = 0; q < MS; q++)
+    step[q] = (int)(((uint32_t)(16 * cx + (MS > 1 ? kXf[q] : 0)) & 0xFFFFu) |
+                    ((uint32_t)(-16 * cy - (MS > 1 ? kYf[q] : 0)) << 16));
 
-  // One batch of up to 64 candidates in list order: each lane sets up one
-  // primitive (its three half planes, or the span masks), then the primitives
-  // are applied in list order.  Most candidates of a deep block lie behind
-  // what the ones before them wrote, and the list of a block is seldom more
-  // than a batch or two, so the depth bounds zl are tested again before the
-  // batch and, all at once, after every kRetest primitives that wrote depth:
-  // at 1080p with 50 layers a block meets 86 candidates, of which 20 are not
-  // hidden by the time their turn comes.
+  // Applies a batch of up to 64 candidates in list order.  Most candidates of
+  // a deep block lie behind what the ones before them wrote, and the list of
+  // a block is seldom more than a batch or two, so the depth bounds zl are
+  // tested again before the batch and, all at once, after every kRetest
+  // primitives that wrote depth: at 1080p with 50 layers a block meets 86
+  // candidates, of which 20 are not hidden by the time their turn comes.
   constexpr int kRetest = 2;
   auto process_chunk = [&](bool act, uint32_t tid, float zl) __attribute__((always_inline)) {
     if (hiz) {
@@ -484,88 +441,84 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
       act = act && !hidden(zl, zmax);
     }
     // ---- triangle-parallel setup ----
-    int pk[3] = {0, 0, 0}, nf[3] = {0, 0, 0};
-    int flags = 0;
-    float x0 = 0, y0 = 0, zA = 0, zB = 0, zC = 0, zBias = 0;
-    bool spans = false;
+    int nflags = 0;
     if (act) {
       const int4 *rp = reinterpret_cast<const int4 *>(rec + tid);
-      const int4 h0 = rp[0];  // nflags, yMin, yMax, xMin
+      nflags = rp[0].x;       // nflags, yMin, yMax, xMin
       const int4 h1 = rp[1];  // xMax, X0, X1, X2
       const int4 h2 = rp[2];  // Y0, Y1, Y2, zlo
-      const float4 h3 = reinterpret_cast<const float4 *>(rp)[3];  // x0, y0, zA, zB
-      const float4 h4 = reinterpret_cast<const float4 *>(rp)[4];  // zC, zBias, wA, wB
-      const int n = h0.x & 0xFF, d = (h0.x >> 8) & 1;
-      flags = h0.x >> 8;
-      x0 = h3.x; y0 = h3.y; zA = h3.z; zB = h3.w; zC = h4.x; zBias = h4.y;
-      spans = !(h0.x & kRecHalfPlanes);
-      if (!spans) {
+      const int4 h3 = rp[3];  // x0, y0, zA, zB
+      const int4 h4 = rp[4];  // zC, zBias, wA, wB
+      const int n = nflags & 0xFF, d = (nflags >> 8) & 1;
+      int f[3] = {0, 0, 0}, pk[3] = {0, 0, 0};
+      if (nflags & kRecHalfPlanes) {
         // Edge i runs from vertex i to i + 1 (d), or back.
-        const int X[3] = {h1.y, h1.z, h1.w}, Y[3] = {h2.x, h2.y, h2.z};
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-          const int k = (i + 1) % 3;
-          half_plane(d ? X[i] : X[k], d ? Y[i] : Y[k], d ? X[k] : X[i], d ? Y[k] : Y[i], ox, oy, pk[i], nf[i]);
-        }
-      } else {
-        const int *pp = poly + (size_t)tid * (2 * kMaxPolygon);
-        auto vtx = [&](int i, int &Xo, int &Yo) {
-          if (n == 3) {
-            // Mask selects: a conditional pick among the components of one
-            // vector would become an indexed access through scratch memory.
-            const int m0 = -(int)(i == 0), m1 = -(int)(i == 1), m2 = -(int)(i == 2);
-            Xo = (h1.y & m0) | (h1.z & m1) | (h1.w & m2);
-            Yo = (h2.x & m0) | (h2.y & m1) | (h2.z & m2);
-          } else {
-            Xo = pp[i];
-            Yo = pp[kMaxPolygon + i];
-          }
+        auto edge = [&](int Xi, int Yi, int Xk, int Yk, int &fo, int &po) {
+          half_plane(d ? Xi : Xk, d ? Yi : Yk, d ? Xk : Xi, d ? Yk : Yi, ox, oy, fo, po);
         };
-        uint32_t any = 0;
-#pragma unroll
-        for (int q = 0; q < MS; q++) {
-          const int xo = (MS > 1) ? kXf[q] : 0, yo = (MS > 1) ? kYf[q] : 0;
-          const uint64_t m = block_coverage(vtx, n, d, xo, yo, ox, oy);
-          spanMask[wave][2*q][lane] = (uint32_t)m; spanMask[wave][2*q+1][lane] = (uint32_t)(m>>32);
-          any |= (uint32_t)m | (uint32_t)(m>>32);
+        if (n == 3) {
+          edge(h1.y, h2.x, h1.z, h2.y, f[0], pk[0]);
+          edge(h1.z, h2.y, h1.w, h2.z, f[1], pk[1]);
+          edge(h1.w, h2.z, h1.y, h2.x, f[2], pk[2]);
+        } else {
+          const int *pp = poly + (size_t)tid * (2 * kMaxPolygon);
+          const int4 X = *reinterpret_cast<const int4 *>(pp), Y = *reinterpret_cast<const int4 *>(pp + kMaxPolygon);
+          const int X4 = n > 4 ? pp[4] : X.x, Y4 = n > 4 ? pp[kMaxPolygon + 4] : Y.x;
+          int4 m = make_int4(0, 0, 1 << 30, 0);  // no fifth half plane: always inside
+          edge(X.x, Y.x, X.y, Y.y, f[0], pk[0]);
+          edge(X.y, Y.y, X.z, Y.z, f[1], pk[1]);
+          edge(X.z, Y.z, X.w, Y.w, f[2], pk[2]);
+          edge(X.w, Y.w, X4, Y4, m.x, m.y);
+          if (n > 4) edge(X4, Y4, X.x, Y.x, m.z, m.w);
+          candMore[wave][lane] = m;
         }
-        act = any != 0;
       }
+      cand[wave][0][lane] = make_int4(f[0], pk[0], f[1], pk[1]);
+      cand[wave][1][lane] = make_int4(f[2], pk[2], h3.x, h3.y);
+      cand[wave][2][lane] = make_int4(h3.z, h3.w, h4.x, h4.y);
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     uint64_t todo = __ballot(act);
-    const uint64_t spanLanes = __ballot(spans);
+    const uint64_t spanLanes = __ballot(act && !(nflags & kRecHalfPlanes));
+    const uint64_t moreLanes = __ballot((nflags & kRecHalfPlanes) && (nflags & 0xFF) > 3);
+    const uint64_t frontLanes = SIMPLE ? 0ull : __ballot((nflags >> 9) & 1);
     int wrote = 0;
 
     // ---- pixel-parallel coverage and tests, in list order ----
     while (todo) {
       const int j = __builtin_ctzll(todo);
       todo &= todo - 1;
+      const int4 c0 = cand[wave][0][j], c1 = cand[wave][1][j], c2 = cand[wave][2][j];
       bool cov[MS];
-#pragma unroll
-      for (int q = 0; q < MS; q++) cov[q] = inside && ((P.msMask >> q) & 1);
       if (!((spanLanes >> j) & 1)) {
+        int in[MS];
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
-          const int p = __builtin_amdgcn_readlane(pk[i], j), n0 = __builtin_amdgcn_readlane(nf[i], j);
-          const int t = dot2_i16(p, pixelStep);
-          if (MS == 1) {
-            cov[0] &= t >= n0;
-          } else {
-            // The samples' offsets are +-(kXf[0], kYf[0]) and +-(kXf[1], kYf[1]).
-            const int DY = (int)(int16_t)p, DX = p >> 16;
-            const int o0 = DY * kXf0 - DX * kYf0, o1 = DY * kXf1 - DX * kYf1;
-            cov[0] &= t >= n0 - o0;
-            cov[MS > 1 ? 1 : 0] &= t >= n0 - o1;
-            cov[MS > 1 ? 2 : 0] &= t >= n0 + o1;
-            cov[MS > 1 ? 3 : 0] &= t >= n0 + o0;
-          }
+        for (int q = 0; q < MS; q++)
+          in[q] = min(min(dot2_i16(c0.y, step[q], c0.x), dot2_i16(c0.w, step[q], c0.z)), dot2_i16(c1.y, step[q], c1.x));
+        if ((moreLanes >> j) & 1) {
+          const int4 m = candMore[wave][j];
+#pragma unroll
+          for (int q = 0; q < MS; q++)
+            in[q] = min(min(in[q], dot2_i16(m.y, step[q], m.x)), dot2_i16(m.w, step[q], m.z));
         }
-      } else {
 #pragma unroll
-        for (int q = 0; q < MS; q++) cov[q] = cov[q] && ((spanMask[wave][2 * q + (myBit >> 5)][j] >> (myBit & 31)) & 1);
+        for (int q = 0; q < MS; q++) cov[q] = in[q] >= 0;
+      } else {
+        const uint32_t tj = __builtin_amdgcn_readlane(tid, j);
+        const TriRecord &R = rec[tj];
+        const int *pp = poly + (size_t)tj * (2 * kMaxPolygon);
+        const int n = R.nflags & 0xFF, d = (R.nflags >> 8) & 1;
+        auto vtx = [&](int i, int &Xo, int &Yo) {
+          Xo = n == 3 ? R.X[i] : pp[i];
+          Yo = n == 3 ? R.Y[i] : pp[kMaxPolygon + i];
+        };
+#pragma unroll
+        for (int q = 0; q < MS; q++)
+          cov[q] = span_covers(vtx, n, d, 16 * px + (MS > 1 ? kXf[q] : 0), 16 * py + (MS > 1 ? kYf[q] : 0));
       }
+#pragma unroll
+      for (int q = 0; q < MS; q++) cov[q] = cov[q] && inside && ((P.msMask >> q) & 1);
       nTests++;
       bool anyCov = false;
 #pragma unroll
@@ -575,9 +528,9 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 
       bool pass[MS];  // samples that pass every test
       if constexpr (SIMPLE) {
-        const float xf = (float)px - rdl(x0, j);  // xFragment (PixelRoutine.cpp:125)
-        const float yf = (float)py - rdl(y0, j);  // yFragment (QuadRasterizer.cpp:126)
-        const float a = rdl(zA, j), b = rdl(zB, j), c = rdl(zC, j);
+        const float xf = (float)px - __int_as_float(c1.z);  // xFragment (PixelRoutine.cpp:125)
+        const float yf = (float)py - __int_as_float(c1.w);  // yFragment (QuadRasterizer.cpp:126)
+        const float a = __int_as_float(c2.x), b = __int_as_float(c2.y), c = __int_as_float(c2.z);
         float zq[MS];
 #pragma unroll
         for (int q = 0; q < MS; q++) {
@@ -608,8 +561,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
           occl += (unsigned)__builtin_popcountll(__ballot(pass[q]));
         }
       } else {
-        const int fl = __builtin_amdgcn_readlane(flags, j);
-        const StencilParams &SP = (fl & 2) ? P.front : P.back;
+        const StencilParams &SP = ((frontLanes >> j) & 1) ? P.front : P.back;
         bool sPass[MS], zPass[MS];
 #pragma unroll
         for (int q = 0; q < MS; q++) sPass[q] = stencilActive ? cov[q] && stencil_compare(SP, S.sb[q]) : cov[q];
@@ -631,10 +583,10 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 #pragma unroll
         for (int q = 0; q < MS; q++) zPass[q] = cov[q];
         if (depthTest) {
-          const float xf = (float)px - rdl(x0, j);  // xFragment (PixelRoutine.cpp:125)
-          const float yf = (float)py - rdl(y0, j);  // yFragment (QuadRasterizer.cpp:126)
-          const float a = rdl(zA, j), b = rdl(zB, j), c = rdl(zC, j);
-          const float zbias = depthBias ? rdl(zBias, j) : 0.0f;
+          const float xf = (float)px - __int_as_float(c1.z);  // xFragment (PixelRoutine.cpp:125)
+          const float yf = (float)py - __int_as_float(c1.w);  // yFragment (QuadRasterizer.cpp:126)
+          const float a = __int_as_float(c2.x), b = __int_as_float(c2.y), c = __int_as_float(c2.z);
+          const float zbias = depthBias ? __int_as_float(c2.w) : 0.0f;
 #pragma unroll
           for (int q = 0; q < MS; q++) {
             const float yy = (MS > 1) ? yf + kSampleY[q] : yf;

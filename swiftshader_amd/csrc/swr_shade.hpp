@@ -8,10 +8,6 @@
 
 namespace swr {
 
-__device__ __forceinline__ float rdl(float v, int j) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
-}
-
 // Interpolated attribute k at (xf, yf): (x*A + (C + y*B)) * rhw, the
 // reference's operation order (QuadRasterizer.cpp:235-250).
 __device__ __forceinline__ float interp(const TriRecord &R, int k, float xf, float yf, float rhw) {
