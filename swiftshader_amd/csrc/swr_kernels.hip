@@ -41,7 +41,7 @@ __device__ __forceinline__ float clip_dist(const ClipVtx &p, int plane) {
 }
 
 __device__ __forceinline__ ClipVtx clip_edge(const ClipVtx &Vi, const ClipVtx &Vj, float di, float dj) {
-  float D = 1.0f / (dj - di);
+  float D = rr_rcp(dj - di);
   ClipVtx o;
 #pragma unroll
   for (int k = 0; k < 4; k++) o.v[k] = (dj * Vi.v[k] - di * Vj.v[k]) * D;
@@ -286,7 +286,7 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
     flags[k] = f;
     // Projection (VertexRoutine.cpp:601-611).
     float ww = __uint_as_float(__float_as_uint(w) | ((w == 0.0f) ? 0x3F800000u : 0u));
-    float rhw = 1.0f / ww;
+    float rhw = rr_rcp(ww);
     PX[k] = rr_round_int_clamped(P.X0xF + (x * rhw) * P.WxF);
     PY[k] = rr_round_int_clamped(P.Y0xF + (y * rhw) * P.HxF);
     pz[k] = z * rhw;
@@ -351,7 +351,7 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
   if (isPolygon) {
     for (int i = 0; i < n; i++) {
       float w = cp[i].v[3];
-      float rhw = (w != 0.0f) ? 1.0f / w : 1.0f;
+      float rhw = (w != 0.0f) ? rr_rcp(w) : 1.0f;
       X[i] = rr_round_int(P.X0xF + (cp[i].v[0] * rhw) * P.WxF);
       Y[i] = rr_round_int(P.Y0xF + (cp[i].v[1] * rhw) * P.HxF);
     }
@@ -422,7 +422,7 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
   float a = x1 * y2 - x2 * y1;
   float M00 = 0.0f, M01 = 0.0f, M02 = rhw0, M10 = 0.0f, M11 = 0.0f, M20 = 0.0f, M21 = 0.0f;
   if (a != 0.0f) {
-    float A = 1.0f / a;
+    float A = rr_rcp(a);
     float D = A * rhw0;
     M00 = (y1 * w2 - y2 * w1) * D;
     M01 = (x2 * w1 - x1 * w2) * D;

@@ -196,8 +196,7 @@ __device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, 
     } else {
       const uint32_t wm = ((P.colorMask & 1) ? 0x000000FFu : 0u) | ((P.colorMask & 2) ? 0x0000FF00u : 0u) |
                           ((P.colorMask & 4) ? 0x00FF0000u : 0u) | ((P.colorMask & 8) ? 0xFF000000u : 0u);
-      const uint32_t o8 = float_to_unorm8(o.x) | (float_to_unorm8(o.y) << 8) | (float_to_unorm8(o.z) << 16) |
-                          (float_to_unorm8(o.w) << 24);
+      const uint32_t o8 = float4_to_unorm8(o);
       S.cb[FCOL ? 0 : q] = (S.cb[FCOL ? 0 : q] & ~wm) | (o8 & wm);
     }
   }
@@ -216,8 +215,7 @@ __device__ __forceinline__ void store_color(const DrawParams &P, int colorMask, 
       o.y = linear_to_srgb(o.y);
       o.z = linear_to_srgb(o.z);
     }
-    o8 = float_to_unorm8(o.x) | (float_to_unorm8(o.y) << 8) | (float_to_unorm8(o.z) << 16) | (float_to_unorm8(o.w) << 24);
-    o8 = bgra_swap(XF && P.colorBGRA, o8);
+    o8 = bgra_swap(XF && P.colorBGRA, float4_to_unorm8(o));
   }
 #pragma unroll
   for (int q = 0; q < MS; q++) {

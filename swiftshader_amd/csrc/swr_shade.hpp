@@ -16,7 +16,7 @@ __device__ __forceinline__ float interp(const TriRecord &R, int k, float xf, flo
 
 __device__ __forceinline__ float quad_rhw(const TriRecord &R, float xf, float yf) {
   const float Dw = R.wC + yf * R.wB;
-  return 1.0f / (xf * R.wA + Dw);
+  return rr_rcp(xf * R.wA + Dw);
 }
 
 // Texture LOD state of the 2x2 quad holding pixel (px, py): the lane
