@@ -49,11 +49,11 @@ __device__ __forceinline__ uint32_t bgra_swap(int bgra, uint32_t v) {
 // ---------------------------------------------------------------------------
 // Work decomposition: one workgroup per 16x16 bin, one wavefront per 8x8
 // block of the bin, one pixel per lane (lanes 4k..4k+3 form a 2x2 quad).
-// Each wave walks the bin's triangle list in API order, 64 entries at a
-// time; the entries whose box and depth bound meet the block are compacted
-// into batches of 64, every lane sets up one of them (triangle-parallel),
-// and the wave then applies them one by one (pixel-parallel) to the block's
-// depth / stencil / colour, which stay in registers throughout.
+// Each wave walks the bin's triangle list in API order; the entries that may
+// reach its block are compacted into batches of 64, every lane tests and
+// sets up one of them (triangle-parallel), and the wave then applies them
+// one by one (pixel-parallel) to the block's depth / stencil / colour, which
+// stay in registers throughout.
 //
 // Coverage is the reference's span rule evaluated per sample point.  The
 // reference walks each edge with an exact integer DDA that stores
@@ -248,7 +248,7 @@ __device__ __forceinline__ void store_color(const DrawParams &P, int colorMask, 
   }
 }
 
-constexpr int kQueue = 64;  // deferred-shading queue entries per wave
+constexpr int kQueue = 128;  // deferred-shading queue entries per wave: two batches of 64
 
 // One screen tile of draw P: `bin` is the tile's index in the draw's tile
 // grid, [start, end) its range of the sorted (tile, primitive) list.  The
@@ -273,7 +273,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   constexpr bool QUEUE = BLEND || MS > 1;  // without blending, one pixel is one fragment unless it has samples
   __shared__ uint32_t qTri[QUEUE ? 4 : 1][QUEUE ? kQueue : 1];
   __shared__ uint32_t qPix[QUEUE ? 4 : 1][QUEUE ? kQueue : 1];
-  __shared__ float4 qCol[QUEUE ? 4 : 1][QUEUE ? kQueue : 1];
+  __shared__ float4 qCol[QUEUE ? 4 : 1][QUEUE ? 64 : 1];
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -347,50 +347,59 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 
   // Wave totals; nTests, nCovers and nShaded are statistics (profiling only).
   unsigned long long occl = 0, nTests = 0, nCovers = 0, nShaded = 0;
-  int qCount = 0;           // wave-uniform queue length
-  uint64_t myEntries = 0;   // queue slots holding fragments of this lane's pixel
+  // The queue is a ring of two batches; a batch is shaded when it is full
+  // (and the last one at the end), so every lane of it has a fragment.
+  int qHead = 0, qCount = 0;  // wave-uniform: first entry (0 or 64), entries
+  // Entries holding fragments of this lane's pixel: of the first batch, and of the next.
+  uint64_t mine = 0, mineNext = 0;
 
+  // Shades the first batch of the queue and applies it.
   auto flush = [&]() __attribute__((always_inline)) {
     if constexpr (!QUEUE) return;
     // Shade the queued fragments, one per lane...
     if (lane < qCount) {
-      const uint32_t t = qTri[wave][lane];
-      const uint32_t pix = qPix[wave][lane];
+      const uint32_t t = qTri[wave][qHead + lane];
+      const uint32_t pix = qPix[wave][qHead + lane];
       const int l = (int)(pix & 63u);
       qCol[wave][lane] = shade<FCOL, FTEX, XF, FA>(P, rec[t], ox + lane_cx(l), oy + lane_cy(l));
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     // ...then blend them into their pixels in queue (API) order, or write them.
-    uint64_t m = myEntries;
+    uint64_t m = mine;
     while (m) {
       const int k = __builtin_ctzll(m);
       m &= m - 1;
+      const int xMask = MS > 1 ? (int)(qPix[wave][qHead + k] >> 8) : 1;
+      const uint32_t tri = FCOL ? qTri[wave][qHead + k] : 0u;
       if constexpr (BLEND)
-        blend_write<MS, FCOL, XF, FAST>(P, S, qCol[wave][k], (int)(qPix[wave][k] >> 8), qTri[wave][k], srgbLut);
+        blend_write<MS, FCOL, XF, FAST>(P, S, qCol[wave][k], xMask, tri, srgbLut);
       else
-        store_color<MS, FCOL, XF>(P, colorMask, px, py, qCol[wave][k], (int)(qPix[wave][k] >> 8), qTri[wave][k]);
+        store_color<MS, FCOL, XF>(P, colorMask, px, py, qCol[wave][k], xMask, tri);
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    myEntries = 0;
-    qCount = 0;
+    mine = mineNext;
+    mineNext = 0;
+    qHead ^= 64;
+    qCount = qCount > 64 ? qCount - 64 : 0;
   };
 
   // Queues the fragment of the lanes that `want` it: primitive tri on their
   // pixel's samples xMask.
   auto enqueue = [&](bool want, uint32_t tri, uint32_t xMask) __attribute__((always_inline)) {
     const uint64_t need = __ballot(want);
-    const int cnt = __builtin_popcountll(need);
-    if (qCount + cnt > kQueue) flush();
+    const int pos = qCount + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
     if (want) {
-      const int pos = qCount + __builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
-                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
-      qTri[wave][pos] = tri;
-      qPix[wave][pos] = (uint32_t)lane | (xMask << 8);
-      myEntries |= 1ull << pos;
+      qTri[wave][(qHead + pos) & (kQueue - 1)] = tri;
+      qPix[wave][(qHead + pos) & (kQueue - 1)] = (uint32_t)lane | (xMask << 8);
+      const uint64_t bit = 1ull << (pos & 63);
+      mine |= pos < 64 ? bit : 0ull;
+      mineNext |= pos < 64 ? 0ull : bit;
     }
-    qCount += cnt;
+    qCount += __builtin_popcountll(need);
+    if (qCount >= 64) flush();
   };
 
   // Largest stored depth of the block (+inf when any is NaN): a primitive
@@ -429,24 +438,45 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   // Applies a batch of up to 64 candidates in list order.  Most candidates of
   // a deep block lie behind what the ones before them wrote, and the list of
   // a block is seldom more than a batch or two, so the depth bounds zl are
-  // tested again before the batch and, all at once, after every kRetest
+  // tested before the batch and again, all at once, after every kRetest
   // primitives that wrote depth: at 1080p with 50 layers a block meets 86
   // candidates, of which 20 are not hidden by the time their turn comes.
   constexpr int kRetest = 2;
-  auto process_chunk = [&](bool act, uint32_t tid, float zl) __attribute__((always_inline)) {
-    if (hiz) {
-      const float zmax = block_zmax();  // by every lane of the wave
-      act = act && !hidden(zl, zmax);
-    }
-    // ---- triangle-parallel setup ----
+  auto process_chunk = [&](bool act, uint32_t tid) __attribute__((always_inline)) {
+    const float zmax0 = hiz ? block_zmax() : __builtin_inff();  // by every lane of the wave
+    // ---- triangle-parallel setup: box, depth bound, half planes ----
     int nflags = 0;
+    float zl = -__builtin_inff();
+    int4 h1, h2, h3, h4;
     if (act) {
       const int4 *rp = reinterpret_cast<const int4 *>(rec + tid);
-      nflags = rp[0].x;       // nflags, yMin, yMax, xMin
-      const int4 h1 = rp[1];  // xMax, X0, X1, X2
-      const int4 h2 = rp[2];  // Y0, Y1, Y2, zlo
-      const int4 h3 = rp[3];  // x0, y0, zA, zB
-      const int4 h4 = rp[4];  // zC, zBias, wA, wB
+      const int4 h0 = rp[0];  // nflags, yMin, yMax, xMin
+      h1 = rp[1];             // xMax, X0, X1, X2
+      h2 = rp[2];             // Y0, Y1, Y2, zlo
+      h3 = rp[3];             // x0, y0, zA, zB
+      h4 = rp[4];             // zC, zBias, wA, wB
+      nflags = h0.x;
+      act = h0.y < oy + 8 && h0.z > oy && h0.w < ox + 8 && h1.x > ox;
+      if (hiz) {
+        // Lower bound of the evaluated plane over this block (sample offsets
+        // included), tightened with the primitive's bound over its box.
+        const float x0 = __int_as_float(h3.x), y0 = __int_as_float(h3.y), zA = __int_as_float(h3.z);
+        const float zB = __int_as_float(h3.w), zC = __int_as_float(h4.x);
+        const float zBias = depthBias ? __int_as_float(h4.y) : 0.0f;
+        const float xa = (float)ox - 0.5f - x0, xb = (float)(ox + 7) + 0.5f - x0;
+        const float ya = (float)oy - 0.5f - y0, yb = (float)(oy + 7) + 0.5f - y0;
+        const float m =
+            fminf(fminf(zA * xa + zB * ya, zA * xb + zB * ya), fminf(zA * xa + zB * yb, zA * xb + zB * yb)) + zC + zBias;
+        const float mag = fabsf(zA) * fmaxf(fabsf(xa), fabsf(xb)) + fabsf(zC) +
+                          2.0f * fabsf(zB) * fmaxf(fabsf(ya), fabsf(yb)) + 2.0f * fabsf(zBias);
+        zl = fmaxf(__int_as_float(h2.w), m - mag * 0x1p-19f);
+        if (!(zl == zl)) zl = -__builtin_inff();
+        zl = fminf(zl, P.depthClampHi);
+        if ((XF && P.depth16)) zl = d16_value(fmaxf(zl, 0.0f));  // the bound in stored units (monotone map)
+        act = act && !hidden(zl, zmax0);
+      }
+    }
+    if (act) {
       const int n = nflags & 0xFF, d = (nflags >> 8) & 1;
       int f[3] = {0, 0, 0}, pk[3] = {0, 0, 0};
       if (nflags & kRecHalfPlanes) {
@@ -479,7 +509,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     uint64_t todo = __ballot(act);
     const uint64_t spanLanes = __ballot(act && !(nflags & kRecHalfPlanes));
-    const uint64_t moreLanes = __ballot((nflags & kRecHalfPlanes) && (nflags & 0xFF) > 3);
+    const uint64_t moreLanes = __ballot(act && (nflags & kRecHalfPlanes) && (nflags & 0xFF) > 3);
     const uint64_t frontLanes = SIMPLE ? 0ull : __ballot((nflags >> 9) & 1);
     int wrote = 0;
 
@@ -665,84 +695,48 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     }
   };
 
-  // Candidates (box meets the block, hierarchical depth test passed) are
-  // compacted, in list order, into a per-wave ring, and set up in full
-  // batches of 64: a 64-entry chunk of the list yields about a third of a
-  // wave of candidates.
-  __shared__ uint32_t ring[4][128];
-  __shared__ float ringZ[4][128];
+  // The entries of the tile's list that may reach this wave's block (a binned
+  // pair carries the blocks its primitive's edges may reach in bits 28-31)
+  // wait, in list order, in a per-wave ring, and are set up in full batches
+  // of 64: about a quarter of the entries reach a given block, so testing
+  // each chunk of the list on its own would leave most lanes idle.  Four
+  // chunks are loaded at a time (1080p frame 516 us, 528 with two; the general
+  // kernels take two, for the LDS of their fifth wave).
+  constexpr int kChunks = LEVEL == 0 ? 2 : 4;
+  constexpr uint32_t kRing = 128 * kChunks;  // at least 63 + 64 * kChunks; a power of two
+  __shared__ uint32_t ring[4][kRing];
   uint32_t ringHead = 0, ringCount = 0;  // wave-uniform
-
-  for (uint32_t base = start; base < end || ringCount > 0;) {
-    if (base < end) {
-      // ---- block depth bound for the hierarchical test ----
-      const float zmax = hiz ? block_zmax() : __builtin_inff();
-      // ---- candidate test: box overlap, then the hierarchical depth bound ----
-      const uint32_t e = base + lane;
-      bool test = false;
-      uint32_t tid = 0;
-      float zlo = -__builtin_inff();
-      // A binned pair carries the blocks of its tile that the primitive's
-      // edges may reach (bits 28-31); the box test completes the overlap test.
-      bool reach = true;
-      if (e < end) {
-        if (binTri) {
-          const uint32_t v = binTri[e];
-          tid = v & kSlotMask;
-          reach = (v >> (28 + wave)) & 1u;
-        } else {
-          tid = e;
-        }
+  for (uint32_t base = start;;) {
+    while (ringCount < 64 && base < end) {
+      uint32_t v[kChunks];
+#pragma unroll
+      for (int u = 0; u < kChunks; u++) {
+        const uint32_t e = base + 64u * u + (uint32_t)lane;
+        v[u] = binTri ? 0u : e | 0xF0000000u;
+        if (binTri && e < end) v[u] = binTri[e];
       }
-      if (e < end && reach) {
-        const int4 *rp = reinterpret_cast<const int4 *>(rec + tid);
-        const int4 h0 = rp[0];  // nflags, yMin, yMax, xMin
-        const int4 h1 = rp[1];  // xMax, ...
-        test = h0.y < oy + 8 && h0.z > oy && h0.w < ox + 8 && h1.x > ox;
-        if (hiz && test) {
-          const float zlo0 = __int_as_float(rp[2].w);                  // zlo
-          const float4 h3 = reinterpret_cast<const float4 *>(rp)[3];  // x0, y0, zA, zB
-          const float4 h4 = reinterpret_cast<const float4 *>(rp)[4];  // zC, zBias, ...
-          const float x0 = h3.x, y0 = h3.y, zA = h3.z, zB = h3.w, zC = h4.x;
-          const float zBias = depthBias ? h4.y : 0.0f;
-          // Lower bound of the evaluated plane over this block (sample offsets
-          // included), tightened with the primitive's bound over its box.
-          const float xa = (float)ox - 0.5f - x0, xb = (float)(ox + 7) + 0.5f - x0;
-          const float ya = (float)oy - 0.5f - y0, yb = (float)(oy + 7) + 0.5f - y0;
-          const float m =
-              fminf(fminf(zA * xa + zB * ya, zA * xb + zB * ya), fminf(zA * xa + zB * yb, zA * xb + zB * yb)) + zC +
-              zBias;
-          const float mag = fabsf(zA) * fmaxf(fabsf(xa), fabsf(xb)) + fabsf(zC) +
-                            2.0f * fabsf(zB) * fmaxf(fabsf(ya), fabsf(yb)) + 2.0f * fabsf(zBias);
-          float zl = fmaxf(zlo0, m - mag * 0x1p-19f);
-          if (!(zl == zl)) zl = -__builtin_inff();
-          zl = fminf(zl, P.depthClampHi);
-          if ((XF && P.depth16)) zl = d16_value(fmaxf(zl, 0.0f));  // the bound in stored units (monotone map)
-          test = !hidden(zl, zmax);
-          zlo = zl;
-        }
+#pragma unroll
+      for (int u = 0; u < kChunks; u++) {
+        const uint32_t e = base + 64u * u + (uint32_t)lane;
+        const bool want = e < end && ((v[u] >> (28 + wave)) & 1u);
+        const uint64_t tb = __ballot(want);
+        if (want)
+          ring[wave][(ringHead + ringCount +
+                      __builtin_amdgcn_mbcnt_hi((uint32_t)(tb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tb, 0))) &
+                     (kRing - 1)] = v[u] & kSlotMask;
+        ringCount += (uint32_t)__builtin_popcountll(tb);
       }
-      const uint64_t tb = __ballot(test);
-      if (test) {
-        const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(tb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tb, 0));
-        ring[wave][(ringHead + ringCount + pos) & 127] = tid;
-        ringZ[wave][(ringHead + ringCount + pos) & 127] = zlo;
-      }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      ringCount += (uint32_t)__builtin_popcountll(tb);
-      base += 64;
+      base = end - base > 64u * kChunks ? base + 64u * kChunks : end;
     }
-    // A full batch, or what is left after the list's end.
-    if (ringCount >= 64 || base >= end) {
-      const uint32_t nb = ringCount < 64 ? ringCount : 64;
-      const bool act = (uint32_t)lane < nb;
-      const uint32_t t2 = act ? ring[wave][(ringHead + lane) & 127] : 0u;
-      const float z2 = act ? ringZ[wave][(ringHead + lane) & 127] : -__builtin_inff();
-      ringHead = (ringHead + nb) & 127;
-      ringCount -= nb;
-      process_chunk(act, t2, z2);
-    }
+    if (!ringCount) break;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint32_t nb = ringCount < 64 ? ringCount : 64;
+    const bool act = (uint32_t)lane < nb;
+    const uint32_t t2 = act ? ring[wave][(ringHead + lane) & (kRing - 1)] : 0u;
+    ringHead = (ringHead + nb) & (kRing - 1);
+    ringCount -= nb;
+    process_chunk(act, t2);
   }
   if constexpr (!BLEND && MS > 1) {
     // One fragment per pixel and distinct last writer of its samples.
@@ -827,11 +821,19 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 // walks its binned list and then those slots, so that one launch does both
 // passes (the tiles of one launch never share pixels, so only the order
 // within a tile matters).
-// Occupancy: 4 waves per SIMD (128 VGPRs) for the single-sample kernels
-// (the float-colour ones spill 12 bytes there and still run faster than at
-// 3 waves), 3 for the multisample ones.
+// Occupancy, in waves per SIMD.  A wave alternates between chains of scalar,
+// LDS and vector work, so more waves pay until registers spill: single-sample
+// unblended kernels take 5 (mesh 386 -> 377 us, 16-view step 2230 -> 2148
+// against 4; 6 spill), and so do the blended general ones (sRGB frame 501 ->
+// 468); the blended ones of the common states 4 (1080p frame 514 us, 549 at
+// 5); the 4x ones 4 (4x frame 713 -> 611 against 3) but with float colours to
+// blend, whose 16 registers of colour would spill, 3.
+constexpr int raster_waves(int ms, bool floatColor, int level, bool blend) {
+  return ms == 1 ? (blend && level > 0 ? 4 : 5) : (blend && floatColor ? 3 : 4);
+}
+
 template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL, bool BLEND>
-__global__ __launch_bounds__(256, MS == 1 || !BLEND ? 4 : 3) void raster_batch_kernel(
+__global__ __launch_bounds__(256, raster_waves(MS, FCOL, LEVEL, BLEND)) void raster_batch_kernel(
                                                            const DrawParams *__restrict__ params,
                                                            const uint32_t *__restrict__ tileBase, int drawLo,
                                                            int drawHi, uint32_t tileLo, uint32_t tileHi,
