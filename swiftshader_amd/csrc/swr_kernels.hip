@@ -131,8 +131,9 @@ __device__ __forceinline__ void tri_vertices(const DrawParams &P, uint32_t t, ui
 // P.lineWidth centred on the segment P0-P1, or, in the Bresenham mode, the
 // parallelogram joining P0's and P1's diamonds of half-width lineWidth / 2
 // along the major axis, in clip space.  Returns false for a rejected line.
+template <int N>
 __device__ __forceinline__ bool line_polygon(const DrawParams &P, const float (&P0)[4], const float (&P1)[4],
-                                             ClipVtx (&cp)[kMaxPolygon]) {
+                                             ClipVtx (&cp)[N]) {
   if (P0[3] <= 0.0f && P1[3] <= 0.0f) return false;
   const float W = P.WxF * (1.0f / 16.0f);
   const float H = P.HxF * (1.0f / 16.0f);
@@ -181,8 +182,9 @@ __device__ __forceinline__ bool line_polygon(const DrawParams &P, const float (&
 // PointSize (clamped to [1, 1023] by two compares, so a NaN passes) centred
 // on the vertex, offsets pSize * w * halfPixel, halfPixel = 0.5 / (viewport
 // extent / 2).
+template <int N>
 __device__ __forceinline__ void point_polygon(const DrawParams &P, const float (&V)[4], float size,
-                                              ClipVtx (&cp)[kMaxPolygon]) {
+                                              ClipVtx (&cp)[N]) {
   float pSize = size;
   if (pSize < 1.0f) pSize = 1.0f;
   if (pSize > 1023.0f) pSize = 1023.0f;
@@ -202,34 +204,34 @@ __device__ __forceinline__ void point_polygon(const DrawParams &P, const float (
 template <typename T>
 __device__ __forceinline__ T pick3(T a, T b, T c, int i) { return i == 0 ? a : (i == 1 ? b : c); }
 
-// Vertex arrays of the polygon path (clipped triangles, lines, points),
+// Vertex arrays of the polygon path (clipped triangles, lines and points),
 // indexed at run time.
 struct PolyWork {
   ClipVtx cp[kMaxPolygon], tmp[kMaxPolygon];
   int X[kMaxPolygon], Y[kMaxPolygon];
 };
 
-// Whether polygon X, Y (n >= 3, coordinates below 2^20) is convex on the 28.4
+// Whether polygon X, Y (n >= 3, extents up to 32767) is convex on the 28.4
 // grid, with no repeated vertex: every turn goes the same way or straight on,
 // and the edges change between downward and upward twice (one revolution).
-__device__ __forceinline__ bool convex_polygon(const int (&X)[kMaxPolygon], const int (&Y)[kMaxPolygon], int n) {
+// The products of 16-bit edges, and the sums of two, fit 32 bits.
+template <int N>
+__device__ __forceinline__ bool convex_polygon(const int (&X)[N], const int (&Y)[N], int n) {
   bool left = false, right = false, back = false;
   int changes = 0, dir = 0, firstDir = 0;
   int dx0 = X[0] - X[n - 1], dy0 = Y[0] - Y[n - 1];
   for (int i = 0; i < n; i++) {
     const int k = i + 1 < n ? i + 1 : 0;
     const int dx1 = X[k] - X[i], dy1 = Y[k] - Y[i];
-    const long long c = (long long)dx0 * dy1 - (long long)dy0 * dx1;
+    const int c = __mul24(dx0, dy1) - __mul24(dy0, dx1);
     left |= c > 0;
     right |= c < 0;
     // Straight on, and neither edge of zero length.
-    back |= c == 0 && (long long)dx0 * dx1 + (long long)dy0 * dy1 <= 0;
+    back |= c == 0 && __mul24(dx0, dx1) + __mul24(dy0, dy1) <= 0;
     const int s = dy1 > 0 ? 1 : (dy1 < 0 ? -1 : 0);
-    if (s) {
-      if (!firstDir) firstDir = s;
-      else if (s != dir) changes++;
-      dir = s;
-    }
+    changes += s != 0 && firstDir != 0 && s != dir ? 1 : 0;
+    firstDir = firstDir ? firstDir : s;
+    dir = s ? s : dir;
     dx0 = dx1;
     dy0 = dy1;
   }
@@ -240,14 +242,14 @@ __device__ __forceinline__ bool convex_polygon(const int (&X)[kMaxPolygon], cons
 // Setup of primitive t of the draw P, written to record slot g (the
 // primitive's index in the batch); `draw` is the draw's index in the batch;
 // w holds the polygon path's arrays.  Without POLY, the primitives that need
-// the polygon path are left alone and false is returned (w is not touched),
-// so that a kernel can give that path workspace in LDS for a few lanes at a
-// time instead of scratch memory for every thread.
+// the polygon path (those that clipping changes) are left alone and false is
+// returned (w is not touched), so that a kernel can give that path workspace
+// in LDS for a few lanes at a time instead of scratch memory for every
+// thread.  Points and lines inside the frustum keep their four corners in
+// registers.
 template <bool POLY = true>
 __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, int draw, TriRecord *__restrict__ rec,
                                           int *__restrict__ poly, uint32_t *__restrict__ tileCount, PolyWork &w) {
-  if (!POLY && (P.point || P.line)) return false;
-
   uint32_t vi[3];
   tri_vertices(P, (uint32_t)t, vi);
 
@@ -302,20 +304,35 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
   int stages = 0;
   int d = 1;
   int frontFacing = 1;
-  if (P.point) {
-    // setupPoint: the point's square, clipped against every frustum plane;
-    // no culling, front-facing, d = 1 (SetupRoutine.cpp:115-119).
-    point_polygon(P, pos[0], P.psize ? P.psize[vi[0]] : 1.0f, cp);
+  const bool quad = P.point || P.line;
+  int QX[4] = {0, 0, 0, 0}, QY[4] = {0, 0, 0, 0};  // a point's or line's corners (without POLY)
+  if (quad) {
+    // setupPoint: the point's square; setupLine: the line's polygon.  Clipped
+    // against every frustum plane; no culling, front-facing, d = 1
+    // (SetupRoutine.cpp:115-119).
     n = 4;
-    stages = clip_polygon(cp, n, P.depthClip ? CLIP_FRUSTUM : CLIP_SIDES, w.tmp);
-    if (n < 3) return true;
-  } else if (P.line) {
-    // setupLine: the line's polygon, clipped against every frustum plane;
-    // no culling, front-facing, d = 1 (SetupRoutine.cpp:115-119).
-    if (!line_polygon(P, pos[0], pos[1], cp)) return true;
-    n = 4;
-    stages = clip_polygon(cp, n, P.depthClip ? CLIP_FRUSTUM : CLIP_SIDES, w.tmp);
-    if (n < 3) return true;
+    if constexpr (POLY) {
+      if (P.point) point_polygon(P, pos[0], P.psize ? P.psize[vi[0]] : 1.0f, cp);
+      else if (!line_polygon(P, pos[0], pos[1], cp)) return true;
+      stages = clip_polygon(cp, n, P.depthClip ? CLIP_FRUSTUM : CLIP_SIDES, w.tmp);
+      if (n < 3) return true;
+    } else {
+      ClipVtx q[4];
+      if (P.point) point_polygon(P, pos[0], P.psize ? P.psize[vi[0]] : 1.0f, q);
+      else if (!line_polygon(P, pos[0], pos[1], q)) return true;
+      // Clipping keeps a polygon whose vertices all lie inside as it is.
+      bool inside = true;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+#pragma unroll
+        for (int k = 0; k < 6; k++) inside = inside && ((k < 2 && !P.depthClip) || clip_dist(q[i], k) >= 0);
+        const float cw = q[i].v[3];
+        const float rhw = (cw != 0.0f) ? rr_rcp(cw) : 1.0f;
+        QX[i] = rr_round_int(P.X0xF + (q[i].v[0] * rhw) * P.WxF);
+        QY[i] = rr_round_int(P.Y0xF + (q[i].v[1] * rhw) * P.HxF);
+      }
+      if (!inside) return false;
+    }
   } else {
     // setupSolidTriangles (Renderer.cpp:733-776).
     if ((flags[0] & flags[1] & flags[2]) != CLIP_FINITE) return true;
@@ -342,9 +359,9 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
 
   // Polygon in 28.4 (reprojected when clipped or a line,
   // SetupRoutine.cpp:122-143).
-  // An unclipped triangle keeps its three vertices in registers; only a
-  // clipped polygon, a line or a point goes through the n-vertex arrays.
-  const bool isPolygon = POLY && (stages != 0 || P.line || P.point);
+  // An unclipped triangle, point or line keeps its vertices in registers; only
+  // a clipped polygon goes through the n-vertex arrays.
+  const bool isPolygon = POLY && (stages != 0 || quad);
   int (&X)[kMaxPolygon] = w.X;
   int (&Y)[kMaxPolygon] = w.Y;
   int yMin, yMax, xLo, xHi;
@@ -360,6 +377,11 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
       yMin = min(yMin, Y[i]); yMax = max(yMax, Y[i]);
       xLo = min(xLo, X[i]); xHi = max(xHi, X[i]);
     }
+  } else if (quad) {
+    yMin = min(min(QY[0], QY[1]), min(QY[2], QY[3]));
+    yMax = max(max(QY[0], QY[1]), max(QY[2], QY[3]));
+    xLo = min(min(QX[0], QX[1]), min(QX[2], QX[3]));
+    xHi = max(max(QX[0], QX[1]), max(QX[2], QX[3]));
   } else {
     yMin = min(min(PY[0], PY[1]), PY[2]);
     yMax = max(max(PY[0], PY[1]), PY[2]);
@@ -513,7 +535,11 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
   R.yMax = yMax;
   R.xMin = xMin;
   R.xMax = xMax;
-  if (!isPolygon) {
+  if (!POLY && quad) {
+    int4 *pp = reinterpret_cast<int4 *>(poly + g * (2 * kMaxPolygon));
+    pp[0] = make_int4(QX[0], QX[1], QX[2], QX[3]);
+    pp[kMaxPolygon / 4] = make_int4(QY[0], QY[1], QY[2], QY[3]);
+  } else if (!isPolygon) {
 #pragma unroll
     for (int i = 0; i < 3; i++) { R.X[i] = PX[i]; R.Y[i] = PY[i]; }
   } else if (n == 3) {
@@ -522,12 +548,14 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
     int *pp = poly + g * (2 * kMaxPolygon);
     for (int i = 0; i < n; i++) { pp[i] = X[i]; pp[kMaxPolygon + i] = Y[i]; }
   }
-  // An unclipped triangle is convex; a polygon is when its turns agree.
-  const int ext = 32767, big = 1 << 20;
-  const int xMinV = xLo, xMaxV = xHi;
-  const bool small = xMinV > -big && xMaxV < big && yLo > -big && yHi < big && wsub(xMaxV, xMinV) <= ext && wsub(yHi, yLo) <= ext;
-  const int planes = small && (!isPolygon || n == 3 || (n <= kMaxHalfPlanes && convex_polygon(X, Y, n))) ? kRecHalfPlanes : 0;
-  R.nflags = n | (d << 8) | (frontFacing ? 1 << 9 : 0) | planes;
+  // A triangle is convex; a polygon is when its turns agree.
+  const int big = 1 << 20, ext = 32767;
+  bool planes = xLo > -big && xHi < big && yLo > -big && yHi < big && wsub(xHi, xLo) <= ext && wsub(yHi, yLo) <= ext;
+  if (planes && n > 3) {
+    if (!POLY) planes = convex_polygon(QX, QY, 4);
+    else planes = n <= kMaxHalfPlanes && convex_polygon(X, Y, n);
+  }
+  R.nflags = n | (d << 8) | (frontFacing ? 1 << 9 : 0) | (planes ? kRecHalfPlanes : 0);
   // Tiles are 8 or 16 pixels a side and xMin, yMin >= 0 (scissor-clamped to
   // a render area at x, y >= 0): shifts divide exactly.
   const int sw = __builtin_ctz((uint32_t)P.tileW), sh = __builtin_ctz((uint32_t)P.tileH);
@@ -542,7 +570,7 @@ constexpr int kPolySlots = 16;
 
 // Setup of primitive t (slot g, draw `draw`) by the calling lane, t < 0 for
 // none: every lane first runs the setup without the polygon path; the lanes
-// whose primitive needs it (clipped triangles, lines, points) then run it
+// whose primitive needs it (what clipping changes) then run it
 // kPolySlots at a time per wave, each with a workspace in `work` (the
 // wave's kPolySlots entries in LDS), so that no thread uses scratch memory.
 // Called by every lane of the wave.
