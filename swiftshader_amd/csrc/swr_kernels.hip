@@ -506,9 +506,12 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
   }
 
   // Lower bound of z as the rasteriser evaluates it, x*A + (C + y*B) in
-  // float, over the bounding box widened by half a pixel (sample offsets):
-  // the affine minimum at a corner, less a margin of 8 ulp of the largest
-  // term.  Lets a tile skip primitives that cannot pass its depth test.
+  // float: covered sample points lie in the polygon, so the affine minimum is
+  // at one of its vertices; a sample's depth is taken at the point mirrored in
+  // x about its pixel's centre, up to 3/4 pixel away; less a margin of 8 ulp
+  // of the largest term over the bounding box.  Lets a tile skip primitives
+  // that cannot pass its depth test (over the bounding box's corners, as this
+  // bound once was, half the triangles of a deep scene reach down to 0).
   float zlo = -__builtin_inff();
   if (P.depthTest && __builtin_isfinite(R.zA) && __builtin_isfinite(R.zB) && __builtin_isfinite(R.zC) &&
       __builtin_isfinite(R.zBias)) {
@@ -516,8 +519,19 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
     const double ya = (double)yMin - 0.5 - (double)R.y0, yb = (double)(yMax - 1) + 0.5 - (double)R.y0;
     const double A = R.zA, B = R.zB, C = R.zC;
     const double Zb = P.depthBias ? (double)R.zBias : 0.0;
-    const double m =
-        fmin(fmin(A * xa + B * ya, A * xb + B * ya), fmin(A * xa + B * yb, A * xb + B * yb)) + C + Zb;
+    auto at = [&](int vx, int vy) {
+      return A * ((double)vx * 0.0625 - (double)R.x0) + B * ((double)vy * 0.0625 - (double)R.y0);
+    };
+    double m;
+    if (isPolygon) {
+      m = at(X[0], Y[0]);
+      for (int i = 1; i < n; i++) m = fmin(m, at(X[i], Y[i]));
+    } else if (quad) {
+      m = fmin(fmin(at(QX[0], QY[0]), at(QX[1], QY[1])), fmin(at(QX[2], QY[2]), at(QX[3], QY[3])));
+    } else {
+      m = fmin(fmin(at(PX[0], PY[0]), at(PX[1], PY[1])), at(PX[2], PY[2]));
+    }
+    m += C + Zb - (P.ms > 1 ? 0.75 * fabs(A) : 0.0);
     const double mag =
         fabs(A) * fmax(fabs(xa), fabs(xb)) + fabs(C) + 2.0 * fabs(B) * fmax(fabs(ya), fabs(yb)) + 2.0 * fabs(Zb);
     const double lo = m - mag * 0x1p-21 - 1e-30;
