@@ -1544,8 +1544,9 @@ int plan_build_bins(swr_batch_plan *pl, const std::vector<GradParams> &G, int cu
       dg[k] = (int8_t)gi;
       cap += (uint64_t)P.width * (uint64_t)P.height * (uint64_t)P.ms;
     }
-    // Up to two gather launches (one per sample count) of cus * 2 workgroups of 4 waves.
-    cap += 2ull * (uint64_t)cus * 2u * 4u * kBinReserve;
+    // Up to two gather launches (one per sample count) of cus * kGatherPerCuMax
+    // workgroups of 4 waves at most.
+    cap += 2ull * (uint64_t)cus * kGatherPerCuMax * 4u * kBinReserve;
     if (!ok || rep.empty() || cap >= (1ull << 31)) continue;
     sb.on = true;
     sb.cap = (uint32_t)cap;
@@ -1662,7 +1663,7 @@ int plan_enqueue_backward(swr_batch_plan *pl, int cus, hipStream_t s) {
       const DrawParams &Ph = pl->L.P[sg.first + hi - 1];
       const uint32_t bHi = pl->bwBase[sg.first + hi - 1] + (uint32_t)(((Ph.width + 15) / 16) * ((Ph.height + 15) / 16));
       if (bHi > bLo) {
-        const uint32_t wgs = std::min<uint32_t>(bHi - bLo, (uint32_t)cus * 2u);
+        const uint32_t wgs = std::min<uint32_t>(bHi - bLo, (uint32_t)(cus * gather_per_cu(ms, sb.on)));
         const TriRecord *rec = pipe.rec.as<TriRecord>();
         if (ms == 1 && sb.on)
           hipLaunchKernelGGL((backward_batch_kernel<1, true>), dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi,

@@ -67,6 +67,15 @@ constexpr uint32_t kBinChunk = 8192;                  // records per scatter wor
 constexpr int kScatterThreads = 512;                   // tap_scatter_kernel workgroup (two per CU fit in LDS)
 constexpr int kMaxBinGroups = 8;
 constexpr uint32_t kBinReserve = 512;                 // record slots a wave reserves at a time
+// Workgroups of backward_batch_kernel that a CU holds at once (and waves per
+// SIMD, for its registers).  The kernel waits on its fragments' gathers and
+// FP64 chains, so a third wave hides more of them as long as its smaller
+// register share holds: with records and one sample it does (16-view step
+// 2102 -> 2037 us), with four samples it spills (64-view step 17.7 -> 18.2
+// ms), and the texel tables of the kernels without records fill the LDS at
+// two.
+constexpr int gather_per_cu(int ms, bool bin) { return ms == 1 && bin ? 3 : 2; }
+constexpr int kGatherPerCuMax = 3;
 constexpr uint32_t kNoBucket = 0xFFFFFFFFu;           // key of a reserved slot left unused
 
 // Footprint of one fragment: texture coordinate, frozen sampling state and
@@ -893,7 +902,8 @@ __global__ __launch_bounds__(256) void backward_kernel(DrawParams P, GradParams 
 // gradients leave as footprint records (bin), which tap_scatter_kernel
 // scatters.
 template <int MS, bool BIN>
-__global__ __launch_bounds__(256) void backward_batch_kernel(const DrawParams *__restrict__ params,
+__global__ __launch_bounds__(256, gather_per_cu(MS, BIN)) void backward_batch_kernel(
+                                                             const DrawParams *__restrict__ params,
                                                              const GradParams *__restrict__ grads,
                                                              const uint32_t *__restrict__ blockBase, int drawLo,
                                                              int drawHi, uint32_t blockLo, uint32_t blockHi,
