@@ -44,7 +44,7 @@ __device__ __forceinline__ float rr_rcp(float x) {
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r), x, 1.0f);
 }
 __device__ __forceinline__ float rr_frac(float x) {
-  return rr_min(x - __builtin_floorf(x), __uint_as_float(0x3F7FFFFFu));
+  return fminf(x - __builtin_floorf(x), __uint_as_float(0x3F7FFFFFu));  // a NaN takes the bound, as the ordered select does
 }
 __device__ __forceinline__ uint32_t mulhi16(uint32_t a, uint32_t b) { return (a * b) >> 16; }
 
@@ -83,8 +83,8 @@ __device__ __forceinline__ float uv_start(int n) { return n <= 1 ? -0.0f : -(flo
 template <bool XF>
 __device__ __forceinline__ uint32_t address16(float uw, int mode) {
   if (mode == 1) {
-    float cl = rr_min(rr_max(uw, 0.0f), 65535.0f / 65536.0f);
-    return (uint32_t)rr_trunc_int(cl * 65536.0f) & 0xFFFFu;
+    float cl = fminf(fmaxf(uw, 0.0f), 65535.0f / 65536.0f);  // in [0, 1), a NaN 0
+    return (uint32_t)(int32_t)(cl * 65536.0f);
   }
   if (XF && mode == 2) {  // bit 16 of the fixed-point coordinate flips the low 16 bits
     const int32_t conv = rr_trunc_int(uw * 65536.0f);
@@ -132,8 +132,9 @@ __device__ __forceinline__ TexLevel tex_level(const TexParams &T, int lvl) {
 
 template <bool XF>
 __device__ __forceinline__ void fetch16(const TexLevel &L, uint32_t u, uint32_t v, uint32_t out[4]) {
-  uint32_t uu = mulhi16(u, (uint32_t)L.width);
-  uint32_t vv = mulhi16(v, (uint32_t)L.height);
+  // 16-bit coordinates by level sizes of at most 16384: 24-bit products.
+  uint32_t uu = __umul24(u, (uint32_t)L.width) >> 16;
+  uint32_t vv = __umul24(v, (uint32_t)L.height) >> 16;
   int32_t index = (int32_t)(int16_t)uu + (int32_t)(int16_t)vv * (int32_t)(int16_t)L.pitch;
   uint32_t p = reinterpret_cast<const uint32_t *>(L.data)[(uint32_t)index];
   out[0] = (p & 0xFFu) << 8;
@@ -191,8 +192,8 @@ __device__ __forceinline__ void sample_quad16(const TexParams &T, const TexLevel
   fetch16<XF>(L, u1, v0, c10);
   fetch16<XF>(L, u0, v1, c01);
   fetch16<XF>(L, u1, v1, c11);
-  uint32_t f0u = (u0 * (uint32_t)L.width) & 0xFFFFu;
-  uint32_t f0v = (v0 * (uint32_t)L.height) & 0xFFFFu;
+  uint32_t f0u = __umul24(u0, (uint32_t)L.width) & 0xFFFFu;
+  uint32_t f0v = __umul24(v0, (uint32_t)L.height) & 0xFFFFu;
   uint32_t f1u = f0u ^ 0xFFFFu, f1v = f0v ^ 0xFFFFu;
   uint32_t f0u0v = mulhi16(f0u, f0v), f1u0v = mulhi16(f1u, f0v);
   uint32_t f0u1v = mulhi16(f0u, f1v), f1u1v = mulhi16(f1u, f1v);
@@ -249,7 +250,7 @@ __device__ __forceinline__ void address_float(const TexParams &T, float uvw, int
   const float one = __uint_as_float(0x3F7FFFFFu);  // just under 1
   float coord;
   if (mode == 1) {
-    coord = rr_min(rr_max(uvw, 0.0f), one);
+    coord = fminf(fmaxf(uvw, 0.0f), one);
   } else if (XF && mode == 2) {
     const float h = uvw * 0.5f;
     coord = rr_min(2.0f * __uint_as_float(__float_as_uint(h - __builtin_rintf(h)) & 0x7FFFFFFFu), one);
@@ -258,9 +259,9 @@ __device__ __forceinline__ void address_float(const TexParams &T, float uvw, int
   } else {
     coord = rr_frac(uvw);
   }
-  coord = coord * (float)dim;
+  coord = coord * (float)dim;  // in [0, dim], a NaN coordinate included: conversions stay in range
   if (tex_filter<FA>(T) == FILT_POINT) {
-    x0 = rr_trunc_int(coord);
+    x0 = (int32_t)coord;
     f = 0.0f;
   } else {
     if (tex_filter<FA>(T) == FILT_MIN_POINT_MAG_LINEAR || tex_filter<FA>(T) == FILT_MIN_LINEAR_MAG_POINT)
@@ -268,7 +269,7 @@ __device__ __forceinline__ void address_float(const TexParams &T, float uvw, int
     else
       coord = coord - 0.5f;
     float fl = __builtin_floorf(coord);
-    x0 = rr_trunc_int(fl);
+    x0 = (int32_t)fl;
     f = coord - fl;
   }
   x1 = x0 - filterMask;
@@ -294,9 +295,9 @@ __device__ __forceinline__ float4 sample_float2d(const TexParams &T, const TexLe
   address_float<XF, FA>(T, u, L.width, tex_addr_u<FA>(T), lod, x0, x1, fu);
   address_float<XF, FA>(T, v, L.height, tex_addr_v<FA>(T), lod, y0, y1, fv);
   int pitch = L.pitch;
-  y0 = (int)((uint32_t)y0 * (uint32_t)pitch);
+  y0 = __mul24(y0, pitch);  // at most 16384 x 32767
   if (tex_filter<FA>(T) == FILT_POINT) return fetchf(L, x0, y0);
-  y1 = (int)((uint32_t)y1 * (uint32_t)pitch);
+  y1 = __mul24(y1, pitch);
   float4 c00 = fetchf(L, x0, y0), c10 = fetchf(L, x1, y0);
   float4 c01 = fetchf(L, x0, y1), c11 = fetchf(L, x1, y1);
   float4 r;
