@@ -600,7 +600,8 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
           // alpha is clamped when the colour attachment is UNORM.  The
           // fragment is shaded again, identically, if it reaches the queue.
           float alpha = 0.0f;
-          if (anyCov) alpha = shade<FCOL, FTEX, XF, FA>(P, rec[__builtin_amdgcn_readlane(tid, j)], px, py, P.color != nullptr).w;
+          const uint32_t tj = __builtin_amdgcn_readlane(tid, j);  // read where every lane is active: lane j need not be covered
+          if (anyCov) alpha = shade<FCOL, FTEX, XF, FA>(P, rec[tj], px, py, P.color != nullptr).w;
 #pragma unroll
           for (int q = 0; q < MS; q++) {
             cov[q] = cov[q] && !(alpha < P.a2c[q]);
