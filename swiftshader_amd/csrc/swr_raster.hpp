@@ -276,7 +276,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   __shared__ float4 qCol[QUEUE ? 4 : 1][QUEUE ? 64 : 1];
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar, as what follows from it: frees up to 14 vector registers
   const int bx = bin % P.tilesX, by = bin / P.tilesX;
   const int bw = P.tileW >> 3;  // 8x8 blocks per tile row
   const int ox = bx * P.tileW + 8 * (wave % bw), oy = by * P.tileH + 8 * (wave / bw);
@@ -702,8 +702,9 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   // of 64: about a quarter of the entries reach a given block, so testing
   // each chunk of the list on its own would leave most lanes idle.  Four
   // chunks are loaded at a time (1080p frame 516 us, 528 with two; the general
-  // kernels take two, for the LDS of their fifth wave).
-  constexpr int kChunks = LEVEL == 0 ? 2 : 4;
+  // kernels and the unblended 4x ones take two, for the LDS of their fifth
+  // wave per SIMD).
+  constexpr int kChunks = LEVEL == 0 || (MS > 1 && !BLEND) ? 2 : 4;
   constexpr uint32_t kRing = 128 * kChunks;  // at least 63 + 64 * kChunks; a power of two
   __shared__ uint32_t ring[4][kRing];
   uint32_t ringHead = 0, ringCount = 0;  // wave-uniform
@@ -823,14 +824,17 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 // passes (the tiles of one launch never share pixels, so only the order
 // within a tile matters).
 // Occupancy, in waves per SIMD.  A wave alternates between chains of scalar,
-// LDS and vector work, so more waves pay until registers spill: single-sample
-// unblended kernels take 5 (mesh 386 -> 377 us, 16-view step 2230 -> 2148
-// against 4; 6 spill), and so do the blended general ones (sRGB frame 501 ->
-// 468); the blended ones of the common states 4 (1080p frame 514 us, 549 at
-// 5); the 4x ones 4 (4x frame 713 -> 611 against 3) but with float colours to
-// blend, whose 16 registers of colour would spill, 3.
+// LDS and vector work, so more waves pay until registers spill.  With one
+// sample, the unblended kernels of the common states take 6 (16-view step
+// 2050 -> 2015 us against 5, shapes frame 476 -> 469) and the general
+// ones, blended ones included, 5 (sRGB frame 501 -> 468 against 4); the
+// blended ones of the common states 4 (1080p frame 514 us, 549 at 5).  With
+// four, the unblended ones of the common states take 5 (64-view step 18.05 ->
+// 17.56 ms against 4) and the others 4 (4x frame 713 -> 611 against 3), but
+// with float colours to blend, whose 16 registers of colour would spill, 3.
 constexpr int raster_waves(int ms, bool floatColor, int level, bool blend) {
-  return ms == 1 ? (blend && level > 0 ? 4 : 5) : (blend && floatColor ? 3 : 4);
+  if (ms == 1) return level == 0 ? 5 : blend ? 4 : 6;
+  return blend ? (floatColor ? 3 : 4) : level == 0 ? 4 : 5;
 }
 
 template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL, bool BLEND>
