@@ -239,17 +239,18 @@ __device__ __forceinline__ bool convex_polygon(const int (&X)[N], const int (&Y)
   return !(left && right) && !back && changes == 2;
 }
 
-// Setup of primitive t of the draw P, written to record slot g (the
-// primitive's index in the batch); `draw` is the draw's index in the batch;
-// w holds the polygon path's arrays.  Without POLY, the primitives that need
-// the polygon path (those that clipping changes) are left alone and false is
-// returned (w is not touched), so that a kernel can give that path workspace
-// in LDS for a few lanes at a time instead of scratch memory for every
-// thread.  Points and lines inside the frustum keep their four corners in
-// registers.
+// Setup of primitive t of the draw P into R (all but R.draw), and the tiles
+// of its box into `tiles`; R's n and box and `tiles` are zero on entry and
+// stay so when it is culled.  Polygons of more than three vertices also write
+// `poly`; w holds the polygon path's arrays.  Without POLY, the primitives
+// that need the polygon path (those that clipping changes) are left alone and
+// false is returned (w is not touched), so that a kernel can give that path
+// workspace in LDS for a few lanes at a time instead of scratch memory for
+// every thread.  Points and lines inside the frustum keep their four corners
+// in registers.
 template <bool POLY = true>
-__device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, int draw, TriRecord *__restrict__ rec,
-                                          int *__restrict__ poly, uint32_t *__restrict__ tileCount, PolyWork &w) {
+__device__ __forceinline__ bool setup_one(const DrawParams &P, int t, TriRecord &R, int *__restrict__ poly,
+                                          uint32_t &tiles, PolyWork &w) {
   uint32_t vi[3];
   tri_vertices(P, (uint32_t)t, vi);
 
@@ -295,10 +296,6 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
     pw[k] = rhw;
   }
 
-  TriRecord &R = rec[g];
-  tileCount[g] = 0;
-  R.nflags = 0;
-  R.draw = draw;
   ClipVtx (&cp)[kMaxPolygon] = w.cp;
   int n = 3;
   int stages = 0;
@@ -550,7 +547,7 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
   R.xMin = xMin;
   R.xMax = xMax;
   if (!POLY && quad) {
-    int4 *pp = reinterpret_cast<int4 *>(poly + g * (2 * kMaxPolygon));
+    int4 *pp = reinterpret_cast<int4 *>(poly);
     pp[0] = make_int4(QX[0], QX[1], QX[2], QX[3]);
     pp[kMaxPolygon / 4] = make_int4(QY[0], QY[1], QY[2], QY[3]);
   } else if (!isPolygon) {
@@ -559,8 +556,7 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
   } else if (n == 3) {
     for (int i = 0; i < 3; i++) { R.X[i] = X[i]; R.Y[i] = Y[i]; }
   } else {
-    int *pp = poly + g * (2 * kMaxPolygon);
-    for (int i = 0; i < n; i++) { pp[i] = X[i]; pp[kMaxPolygon + i] = Y[i]; }
+    for (int i = 0; i < n; i++) { poly[i] = X[i]; poly[kMaxPolygon + i] = Y[i]; }
   }
   // A triangle is convex; a polygon is when its turns agree.
   const int big = 1 << 20, ext = 32767;
@@ -575,33 +571,71 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, size_t g, 
   const int sw = __builtin_ctz((uint32_t)P.tileW), sh = __builtin_ctz((uint32_t)P.tileH);
   int tx0 = xMin >> sw, tx1 = (xMax - 1) >> sw;
   int ty0 = yMin >> sh, ty1 = (yMax - 1) >> sh;
-  tileCount[g] = (uint32_t)((tx1 - tx0 + 1) * (ty1 - ty0 + 1));
+  tiles = (uint32_t)((tx1 - tx0 + 1) * (ty1 - ty0 + 1));
   return true;
 }
 
 // Polygon-path workspaces per wave of the setup kernels (640 B each).
 constexpr int kPolySlots = 16;
+// A record's words as staged in LDS: all but the last, R.draw.  An odd stride,
+// so that the lanes' writes of one word fall in different banks.
+constexpr int kStageWords = (int)(sizeof(TriRecord) / 4) - 1;
+static_assert(64 * kStageWords * 4 <= kPolySlots * sizeof(PolyWork) && kStageWords % 2 == 1, "record staging");
 
 // Setup of primitive t (slot g, draw `draw`) by the calling lane, t < 0 for
 // none: every lane first runs the setup without the polygon path; the lanes
 // whose primitive needs it (what clipping changes) then run it
 // kPolySlots at a time per wave, each with a workspace in `work` (the
 // wave's kPolySlots entries in LDS), so that no thread uses scratch memory.
-// Called by every lane of the wave.
+// Called by every lane of the wave, with consecutive slots.
+//
+// The kernel is bound by its record stores: 160 bytes a lane, 160 bytes
+// apart, took some 13 store instructions of 64 cache lines each.  The wave's
+// records are therefore staged in LDS (in the polygon path's workspaces, which
+// are used afterwards) and leave as whole lines, 64 consecutive 16-byte pieces
+// to an instruction; of a culled primitive's record only the first piece.
 __device__ __forceinline__ void setup_lanes(const DrawParams &P, int t, size_t g, int draw, TriRecord *__restrict__ rec,
                                             int *__restrict__ poly, uint32_t *__restrict__ tileCount,
                                             PolyWork *work) {
   const int lane = threadIdx.x & 63;
-  bool later = t >= 0 && !setup_one<false>(P, t, g, draw, rec, poly, tileCount, work[0]);
+  int *stage = reinterpret_cast<int *>(work);
+  bool later = false;
+  uint32_t tiles = 0;
+  if (t >= 0) {
+    TriRecord &R = *reinterpret_cast<TriRecord *>(stage + lane * kStageWords);
+    R.nflags = R.yMin = R.yMax = R.xMin = R.xMax = 0;
+    later = !setup_one<false>(P, t, R, poly + g * (2 * kMaxPolygon), tiles, work[0]);
+    if (!later) tileCount[g] = tiles;
+  }
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  {
+    const uint64_t has = __ballot(t >= 0 && !later), full = __ballot(tiles != 0);
+    int4 *out = reinterpret_cast<int4 *>(rec + (g - (size_t)lane));  // the wave's first record
+    constexpr int kParts = (int)(sizeof(TriRecord) / 16);
+#pragma unroll
+    for (int i = 0; i < kParts; i++) {
+      const int q = 64 * i + lane, r = q / kParts, part = q % kParts;
+      if (!((part == 0 ? has : full) >> r & 1)) continue;
+      const int *w = stage + r * kStageWords + 4 * part;
+      out[q] = make_int4(w[0], w[1], w[2], part == kParts - 1 ? draw : w[3]);
+    }
+  }
   const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   for (uint64_t m = __ballot(later); m; m = __ballot(later)) {  // wave-uniform
-    const uint32_t rank = (uint32_t)__builtin_popcountll(m & below);
-    const bool mine = later && rank < (uint32_t)kPolySlots;
-    if (mine) setup_one<true>(P, t, g, draw, rec, poly, tileCount, work[rank]);
-    later = later && !mine;
-    // The next round's lanes reuse these workspaces.
+    // The next round's lanes reuse the workspaces.
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint32_t rank = (uint32_t)__builtin_popcountll(m & below);
+    const bool mine = later && rank < (uint32_t)kPolySlots;
+    if (mine) {
+      TriRecord &R = rec[g];
+      R.nflags = R.yMin = R.yMax = R.xMin = R.xMax = 0;
+      R.draw = draw;
+      setup_one<true>(P, t, R, poly + g * (2 * kMaxPolygon), tiles, work[rank]);
+      tileCount[g] = tiles;
+    }
+    later = later && !mine;
   }
 }
 
