@@ -662,8 +662,9 @@ __device__ bool fragment_backward(GradLds<BIN> &S, const DrawParams &P, const Gr
 // Adds each lane's primitive gradients val (primitive t; t = kEmptyKey: none)
 // to the primitive table.  Lanes of one primitive usually sit next to each
 // other in the batch: runs of equal t are summed first (a segmented scan
-// across the wave), and the last lane of each run adds the run's sums, so a
-// run of L lanes costs one set of float LDS atomics instead of L.
+// across the wave, of as many steps as its longest run takes), and the last
+// lane of each run adds the run's sums, so a run of L lanes costs one set of
+// float LDS atomics instead of L.
 template <bool BIN>
 __device__ __forceinline__ void tri_add_wave(GradLds<BIN> &S, const DrawParams &P, const GradParams &G, uint32_t t,
                                              float (&val)[kTriVals]) {
@@ -676,8 +677,9 @@ __device__ __forceinline__ void tri_add_wave(GradLds<BIN> &S, const DrawParams &
   if (starts != ~0ull) {
     const uint64_t upTo = lane == 63 ? ~0ull : (2ull << lane) - 1ull;
     const int runStart = 63 - __builtin_clzll(starts & upTo);
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
+    // `more`: lanes whose run has d lanes before them (wave-uniform).
+    uint64_t more = ~starts;
+    for (int d = 1; more; more &= more << d, d <<= 1) {
       const bool take = lane - d >= runStart;
 #pragma unroll
       for (int k = 0; k < kTriVals; k++) {
