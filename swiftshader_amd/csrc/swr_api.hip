@@ -1319,6 +1319,7 @@ struct swr_batch_plan {
   std::vector<swr_grad_desc> gradDescs;  // caller order
   Scratch gparams, gbase;
   std::vector<uint32_t> bwBase;
+  std::vector<uint8_t> bwAttr;  // per draw: wants gradients of vertex attributes
   bool hasGrads = false;
   // Binned texel scatter, per segment (see BinArgs): whether it is used,
   // its bucket count, record capacity and offsets into the plan's tables.
@@ -1544,9 +1545,8 @@ int plan_build_bins(swr_batch_plan *pl, const std::vector<GradParams> &G, int cu
       dg[k] = (int8_t)gi;
       cap += (uint64_t)P.width * (uint64_t)P.height * (uint64_t)P.ms;
     }
-    // Up to two gather launches (one per sample count) of cus * kGatherPerCuMax
-    // workgroups of 4 waves at most.
-    cap += 2ull * (uint64_t)cus * kGatherPerCuMax * 4u * kBinReserve;
+    // Up to two gather launches (one per sample count).
+    cap += 2ull * (uint64_t)cus * kGatherSlack;
     if (!ok || rep.empty() || cap >= (1ull << 31)) continue;
     sb.on = true;
     sb.cap = (uint32_t)cap;
@@ -1605,6 +1605,7 @@ int plan_upload_grads(DeviceCtx *c, swr_batch_plan *pl, hipStream_t s) {
   const size_t n = pl->L.P.size();
   std::vector<GradParams> G(n);
   pl->bwBase.assign(n, 0);
+  pl->bwAttr.assign(n, 0);
   for (const auto &sg : pl->L.segs) {
     uint32_t base = 0;
     for (int k = 0; k < sg.count; k++) {
@@ -1614,6 +1615,7 @@ int plan_upload_grads(DeviceCtx *c, swr_batch_plan *pl, hipStream_t s) {
       int r = grad_params(&pl->descs[o], P, &pl->gradDescs[o], G[i]);
       if (r != SWR_OK) return fail(r, "draw %d: %s", o, g_error.c_str());
       pl->bwBase[i] = base;
+      pl->bwAttr[i] = G[i].dPos || G[i].dCol || G[i].dUV;
       base += (uint32_t)(((P.width + 15) / 16) * ((P.height + 15) / 16));
     }
   }
@@ -1663,20 +1665,19 @@ int plan_enqueue_backward(swr_batch_plan *pl, int cus, hipStream_t s) {
       const DrawParams &Ph = pl->L.P[sg.first + hi - 1];
       const uint32_t bHi = pl->bwBase[sg.first + hi - 1] + (uint32_t)(((Ph.width + 15) / 16) * ((Ph.height + 15) / 16));
       if (bHi > bLo) {
-        const uint32_t wgs = std::min<uint32_t>(bHi - bLo, (uint32_t)(cus * gather_per_cu(ms, sb.on)));
+        const bool attr = std::any_of(pl->bwAttr.begin() + sg.first + lo, pl->bwAttr.begin() + sg.first + hi,
+                                      [](uint8_t a) { return a != 0; });
+        const uint32_t wgs = std::min<uint32_t>(bHi - bLo, (uint32_t)(cus * gather_per_cu(ms, sb.on, attr || !sb.on)));
         const TriRecord *rec = pipe.rec.as<TriRecord>();
-        if (ms == 1 && sb.on)
-          hipLaunchKernelGGL((backward_batch_kernel<1, true>), dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi,
-                             bLo, bHi, ctr + group, rec, bin);
-        else if (ms == 1)
-          hipLaunchKernelGGL((backward_batch_kernel<1, false>), dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi,
-                             bLo, bHi, ctr + group, rec, bin);
-        else if (sb.on)
-          hipLaunchKernelGGL((backward_batch_kernel<4, true>), dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi,
-                             bLo, bHi, ctr + group, rec, bin);
-        else
-          hipLaunchKernelGGL((backward_batch_kernel<4, false>), dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi,
-                             bLo, bHi, ctr + group, rec, bin);
+        auto launch = [&](auto *kernel) {
+          hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi, bLo, bHi, ctr + group, rec,
+                             bin);
+        };
+        // Draws that want only the texture's gradient take the kernels without
+        // vertex attributes, whatever their number: they do strictly less.
+        if (!sb.on) launch(ms == 1 ? backward_batch_kernel<1, false, true> : backward_batch_kernel<4, false, true>);
+        else if (attr) launch(ms == 1 ? backward_batch_kernel<1, true, true> : backward_batch_kernel<4, true, true>);
+        else launch(ms == 1 ? backward_batch_kernel<1, true, false> : backward_batch_kernel<4, true, false>);
       }
       group++;
       lo = hi;

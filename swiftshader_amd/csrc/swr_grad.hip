@@ -51,7 +51,7 @@ struct GradParams {
 // writes one footprint record per fragment, keyed by the kBinTile-texel tile
 // of its finer mip level within its texture group (draws that share
 // texture-gradient buffers and sampler state), into slots its wave reserves
-// kBinReserve at a time.  The (key, slot) pairs of every draw of the segment
+// bin_reserve at a time.  The (key, slot) pairs of every draw of the segment
 // are then sorted by key with the stable radix sort of the binning front
 // end, and each tile's records are scattered, one group at a time, into LDS
 // copies of the tile (with a halo for the probes that cross its edges) at
@@ -66,16 +66,22 @@ constexpr int kBinCells = kBinR0 * kBinR0 + kBinR1 * kBinR1;  // LDS cells of bo
 constexpr uint32_t kBinChunk = 8192;                  // records per scatter work item
 constexpr int kScatterThreads = 512;                   // tap_scatter_kernel workgroup (two per CU fit in LDS)
 constexpr int kMaxBinGroups = 8;
-constexpr uint32_t kBinReserve = 512;                 // record slots a wave reserves at a time
+// Record slots a wave reserves at a time: fewer for the kernels without
+// attribute gradients, of which more waves run at once.
+constexpr uint32_t bin_reserve(bool attr) { return attr ? 512 : 256; }
 // Workgroups of backward_batch_kernel that a CU holds at once (and waves per
 // SIMD, for its registers).  The kernel waits on its fragments' gathers and
-// FP64 chains, so a third wave hides more of them as long as its smaller
-// register share holds: with records and one sample it does (16-view step
-// 2102 -> 2037 us), with four samples it spills (64-view step 17.7 -> 18.2
-// ms), and the texel tables of the kernels without records fill the LDS at
-// two.
-constexpr int gather_per_cu(int ms, bool bin) { return ms == 1 && bin ? 3 : 2; }
-constexpr int kGatherPerCuMax = 3;
+// FP64 chains, so more waves hide more of them as long as their smaller
+// register share holds.  Without attribute gradients (attr) it needs 78 to 95
+// registers and five fit (64-view 4x step 15.8 -> 14.9 ms against the general
+// kernel with two).  With them, records and one sample take three (16-view
+// step 2102 -> 2037 us against two), four samples spill at three (64-view step
+// 17.7 -> 18.2 ms), and the texel tables of the kernels without records fill
+// the LDS at two.
+constexpr int gather_per_cu(int ms, bool bin, bool attr) { return !attr ? 5 : ms == 1 && bin ? 3 : 2; }
+// Slots that the last reservations of all of a launch's waves may leave unused, per CU.
+constexpr uint32_t kGatherSlack = 4u * 3u * bin_reserve(true);
+static_assert(4u * 5u * bin_reserve(false) <= kGatherSlack, "slack of the attribute-free kernels");
 constexpr uint32_t kNoBucket = 0xFFFFFFFFu;           // key of a reserved slot left unused
 
 // Footprint of one fragment: texture coordinate, frozen sampling state and
@@ -521,8 +527,9 @@ __device__ __forceinline__ void texture_backward(GradLds<BIN> &S, const TexParam
 // With BIN the texel gradient is not scattered: the fragment's footprint
 // record goes to `rec` and the function returns true.  The primitive's 27
 // attribute gradients go to `val` (all zero when none are wanted or the
-// fragment has none); the caller adds them to the primitive table.
-template <bool BIN>
+// fragment has none); the caller adds them to the primitive table.  Without
+// ATTR no draw wants them, and val is not touched.
+template <bool BIN, bool ATTR>
 __device__ bool fragment_backward(GradLds<BIN> &S, const DrawParams &P, const GradParams &G, uint32_t t, int px,
                                   int py, const Acc4 &g, const QuadLod &L, TapRecord &rec, float (&val)[kTriVals]) {
   bool has = false;
@@ -593,7 +600,7 @@ __device__ bool fragment_backward(GradLds<BIN> &S, const DrawParams &P, const Gr
   const float4 gf = make_float4((float)g.x, (float)g.y, (float)g.z, (float)g.w);
   float4 dcol = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float dU = 0.0f, dV = 0.0f;
-  const bool attrGrads = G.dPos || G.dCol || G.dUV;
+  const bool attrGrads = ATTR && (G.dPos || G.dCol || G.dUV);
   if (P.useUV) {
     const float4 gTex = P.useColor ? make_float4(gf.x * col.x, gf.y * col.y, gf.z * col.z, gf.w * col.w) : gf;
     float4 tex = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -791,9 +798,10 @@ __device__ __forceinline__ void release_slots(const BinArgs &bin, SlotRange &sr)
 // Writes the records of the wave's lanes that have one (all lanes call
 // this together) into the wave's reserved slots; when they do not all fit,
 // the first ones fill the reservation and the rest start a new one of
-// kBinReserve slots (one atomic per reservation).  No slot is skipped, so
+// RESERVE slots (one atomic per reservation).  No slot is skipped, so
 // the slots reserved never exceed the records plus one reservation per
 // wave.
+template <uint32_t RESERVE>
 __device__ __forceinline__ void emit_records(const BinArgs &bin, SlotRange &sr, bool has, const TapRecord &r,
                                              uint32_t key) {
   const int lane = threadIdx.x & 63;
@@ -802,7 +810,7 @@ __device__ __forceinline__ void emit_records(const BinArgs &bin, SlotRange &sr, 
   const uint32_t cnt = (uint32_t)__builtin_popcountll(want);
   uint32_t fresh = 0;
   if (cnt > sr.left) {
-    if (lane == 0) fresh = atomicAdd(bin.reserved, kBinReserve);
+    if (lane == 0) fresh = atomicAdd(bin.reserved, RESERVE);
     fresh = __builtin_amdgcn_readfirstlane(fresh);
   }
   const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
@@ -815,7 +823,7 @@ __device__ __forceinline__ void emit_records(const BinArgs &bin, SlotRange &sr, 
   }
   if (cnt > sr.left) {
     sr.base = fresh + (cnt - sr.left);
-    sr.left = kBinReserve - (cnt - sr.left);
+    sr.left = RESERVE - (cnt - sr.left);
   } else {
     sr.base += cnt;
     sr.left -= cnt;
@@ -827,7 +835,7 @@ __device__ __forceinline__ void emit_records(const BinArgs &bin, SlotRange &sr, 
 // that edge pixels with several primitives cost extra lanes rather than
 // extra passes, and partial batches occur only at draw changes.  With BIN
 // the texel gradients leave as footprint records of draw group `grp`.
-template <int MS, bool BIN>
+template <int MS, bool BIN, bool ATTR>
 __device__ __forceinline__ void drain_fragments(GradLds<BIN> &S, FragQueue &Q, RingPos &rp, const DrawParams &P,
                                                 const GradParams &G, const TriRecord *__restrict__ rec, bool all,
                                                 const BinArgs &bin, SlotRange &sr, int grp) {
@@ -865,12 +873,13 @@ __device__ __forceinline__ void drain_fragments(GradLds<BIN> &S, FragQueue &Q, R
             *reinterpret_cast<float4 *>(G.state + q * G.stateSlice + (long long)y * G.statePitch + 16ll * x) =
                 make_float4(L.lod, L.aniso, L.uDelta, L.vDelta);
       }
-      has = fragment_backward<BIN>(S, P, G, t, x, y, g, L, r, val);
+      has = fragment_backward<BIN, ATTR>(S, P, G, t, x, y, g, L, r, val);
       if (BIN && has) key = tap_bucket(P.tex, bin.groups[grp], r.u, r.v, r.L.lod);
       tv = t;
     }
-    if (G.dPos || G.dCol || G.dUV) tri_add_wave(S, P, G, tv, val);
-    if constexpr (BIN) emit_records(bin, sr, has, r, key);
+    if constexpr (ATTR)
+      if (G.dPos || G.dCol || G.dUV) tri_add_wave(S, P, G, tv, val);
+    if constexpr (BIN) emit_records<bin_reserve(ATTR)>(bin, sr, has, r, key);
     rp.head = (rp.head + n) & (kRing - 1);
     rp.count -= n;
   }
@@ -886,7 +895,7 @@ __global__ __launch_bounds__(256) void backward_kernel(DrawParams P, GradParams 
   const BinArgs none = {};
   SlotRange sr = {0u, 0u};
   enqueue_fragments<MS>(Q, rp, P, blockIdx.x * 16 + (threadIdx.x & 15), blockIdx.y * 16 + (threadIdx.x >> 4));
-  drain_fragments<MS, false>(S, Q, rp, P, G, rec, true, none, sr, 0);
+  drain_fragments<MS, false, true>(S, Q, rp, P, G, rec, true, none, sr, 0);
   lds_flush(S, P, G);
 }
 
@@ -903,8 +912,8 @@ __global__ __launch_bounds__(256) void backward_kernel(DrawParams P, GradParams 
 // the same draw.  With BIN there are no texel tables: the draws' texel
 // gradients leave as footprint records (bin), which tap_scatter_kernel
 // scatters.
-template <int MS, bool BIN>
-__global__ __launch_bounds__(256, gather_per_cu(MS, BIN)) void backward_batch_kernel(
+template <int MS, bool BIN, bool ATTR>
+__global__ __launch_bounds__(256, gather_per_cu(MS, BIN, ATTR)) void backward_batch_kernel(
                                                              const DrawParams *__restrict__ params,
                                                              const GradParams *__restrict__ grads,
                                                              const uint32_t *__restrict__ blockBase, int drawLo,
@@ -937,7 +946,7 @@ __global__ __launch_bounds__(256, gather_per_cu(MS, BIN)) void backward_batch_ke
     if (cur >= 0 && lo != cur) {
       // The rest of draw cur's fragments, before its tables are flushed (the
       // primitive table is shared: every wave finishes adding first).
-      drain_fragments<MS, BIN>(S, Q, rp, params[cur], grads[cur], rec + params[cur].triBase, true, bin, sr,
+      drain_fragments<MS, BIN, ATTR>(S, Q, rp, params[cur], grads[cur], rec + params[cur].triBase, true, bin, sr,
                                BIN ? bin.drawGroup[cur] : 0);
       __syncthreads();
     }
@@ -966,7 +975,7 @@ __global__ __launch_bounds__(256, gather_per_cu(MS, BIN)) void backward_batch_ke
     const uint32_t bx = (uint32_t)(P.width + 15) >> 4;
     const int px = (int)(local % bx) * 16 + (threadIdx.x & 15), py = (int)(local / bx) * 16 + (threadIdx.x >> 4);
     enqueue_fragments<MS>(Q, rp, P, px, py);
-    drain_fragments<MS, BIN>(S, Q, rp, P, grads[lo], rec + P.triBase, false, bin, sr, BIN ? bin.drawGroup[lo] : 0);
+    drain_fragments<MS, BIN, ATTR>(S, Q, rp, P, grads[lo], rec + P.triBase, false, bin, sr, BIN ? bin.drawGroup[lo] : 0);
     __syncthreads();
   }
   if constexpr (BIN) release_slots(bin, sr);
@@ -1317,17 +1326,23 @@ __global__ void mip_up_rgba32f_kernel(float4 *fine, int fw, int fh, int fp, cons
 
 template __global__ void backward_kernel<1>(DrawParams, GradParams, const TriRecord *);
 template __global__ void backward_kernel<4>(DrawParams, GradParams, const TriRecord *);
-template __global__ void backward_batch_kernel<1, false>(const DrawParams *, const GradParams *, const uint32_t *, int,
-                                                         int, uint32_t, uint32_t, uint32_t *, const TriRecord *,
-                                                         BinArgs);
-template __global__ void backward_batch_kernel<4, false>(const DrawParams *, const GradParams *, const uint32_t *, int,
-                                                         int, uint32_t, uint32_t, uint32_t *, const TriRecord *,
-                                                         BinArgs);
-template __global__ void backward_batch_kernel<1, true>(const DrawParams *, const GradParams *, const uint32_t *, int,
-                                                        int, uint32_t, uint32_t, uint32_t *, const TriRecord *,
-                                                        BinArgs);
-template __global__ void backward_batch_kernel<4, true>(const DrawParams *, const GradParams *, const uint32_t *, int,
-                                                        int, uint32_t, uint32_t, uint32_t *, const TriRecord *,
-                                                        BinArgs);
+template __global__ void backward_batch_kernel<1, false, true>(const DrawParams *, const GradParams *, const uint32_t *,
+                                                              int, int, uint32_t, uint32_t, uint32_t *,
+                                                              const TriRecord *, BinArgs);
+template __global__ void backward_batch_kernel<1, true, true>(const DrawParams *, const GradParams *, const uint32_t *,
+                                                              int, int, uint32_t, uint32_t, uint32_t *,
+                                                              const TriRecord *, BinArgs);
+template __global__ void backward_batch_kernel<1, true, false>(const DrawParams *, const GradParams *, const uint32_t *,
+                                                              int, int, uint32_t, uint32_t, uint32_t *,
+                                                              const TriRecord *, BinArgs);
+template __global__ void backward_batch_kernel<4, false, true>(const DrawParams *, const GradParams *, const uint32_t *,
+                                                              int, int, uint32_t, uint32_t, uint32_t *,
+                                                              const TriRecord *, BinArgs);
+template __global__ void backward_batch_kernel<4, true, true>(const DrawParams *, const GradParams *, const uint32_t *,
+                                                              int, int, uint32_t, uint32_t, uint32_t *,
+                                                              const TriRecord *, BinArgs);
+template __global__ void backward_batch_kernel<4, true, false>(const DrawParams *, const GradParams *, const uint32_t *,
+                                                              int, int, uint32_t, uint32_t, uint32_t *,
+                                                              const TriRecord *, BinArgs);
 
 }  // namespace swr
