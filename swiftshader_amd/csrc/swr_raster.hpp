@@ -864,7 +864,13 @@ __global__ __launch_bounds__(256, raster_waves(MS, FCOL, LEVEL, BLEND)) void ras
       __syncthreads();
     } else {
       if (iter) break;
-      t = tileLo + blockIdx.x;
+      // Workgroups go round the 8 XCDs in turn: with four samples, whose planes
+      // outgrow the caches, four neighbouring tiles go to one XCD, so that the
+      // cache lines and records they share meet in one L2 (64-view step 14.84
+      // -> 14.70 ms, 4x frame 576 -> 570 us; with one sample the frame of 50
+      // layers loses 0.5 % to its uneven tiles).
+      const uint32_t grp = blockIdx.x & ~31u, r = blockIdx.x & 31u;
+      t = tileLo + (MS > 1 && grp + 32u <= gridDim.x ? grp + (r & 7u) * 4u + (r >> 3) : blockIdx.x);
     }
     if (t >= tileHi) break;
     int lo = drawLo, hi = drawHi;
