@@ -1305,6 +1305,26 @@ int check_chain(const swr_texture *t, uint32_t texelBytes) {
   return SWR_OK;
 }
 
+// First level of the tail of a chain: the levels from it on are at most
+// kMipTailTexels large (level_count when none is).
+uint32_t mip_tail_first(const swr_texture *t) {
+  uint32_t l = 0;
+  while (l < t->level_count && (uint64_t)t->levels[l].width * t->levels[l].height > kMipTailTexels) l++;
+  return l;
+}
+
+MipTail mip_tail(const swr_texture *t, uint32_t first, uint32_t texelBytes) {
+  MipTail M{};
+  for (uint32_t l = first; l < t->level_count; l++) {
+    const swr_image_level &v = t->levels[l];
+    M.data[M.count] = const_cast<void *>((const void *)v.data);
+    M.width[M.count] = (int)v.width;
+    M.height[M.count] = (int)v.height;
+    M.pitch[M.count++] = (int)(v.row_pitch_bytes / texelBytes);
+  }
+  return M;
+}
+
 }  // namespace
 
 struct swr_batch_plan {
@@ -1773,17 +1793,23 @@ int swr_generate_mips(const swr_texture *tex, void *stream) {
   int r = check_chain(tex, tb);
   if (r != SWR_OK) return r;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  for (uint32_t l = 1; l < tex->level_count; l++) {
+  const uint32_t tail = mip_tail_first(tex);
+  for (uint32_t l = 1; l <= tail && l < tex->level_count; l++) {
     const swr_image_level &a = tex->levels[l - 1], &b = tex->levels[l];
     dim3 grid((b.width + 255) / 256, b.height), block(256);
     if (f)
-      hipLaunchKernelGGL(mip_down_rgba32f_kernel, grid, block, 0, s, (const float4 *)a.data, (int)a.width,
+      hipLaunchKernelGGL(mip_down_kernel<float4>, grid, block, 0, s, (const float4 *)a.data, (int)a.width,
                          (int)a.height, (int)(a.row_pitch_bytes / tb), (float4 *)b.data, (int)b.width, (int)b.height,
                          (int)(b.row_pitch_bytes / tb));
     else
-      hipLaunchKernelGGL(mip_down_rgba8_kernel, grid, block, 0, s, (const uint32_t *)a.data, (int)a.width,
+      hipLaunchKernelGGL(mip_down_kernel<uint32_t>, grid, block, 0, s, (const uint32_t *)a.data, (int)a.width,
                          (int)a.height, (int)(a.row_pitch_bytes / tb), (uint32_t *)b.data, (int)b.width, (int)b.height,
                          (int)(b.row_pitch_bytes / tb));
+  }
+  if (tail + 1 < tex->level_count) {
+    const MipTail M = mip_tail(tex, tail, tb);
+    if (f) hipLaunchKernelGGL(mip_down_tail_kernel<float4>, dim3(1), dim3(kMipTailThreads), 0, s, M);
+    else hipLaunchKernelGGL(mip_down_tail_kernel<uint32_t>, dim3(1), dim3(kMipTailThreads), 0, s, M);
   }
   SWR_HIP_CHECK(hipGetLastError());
   return SWR_OK;
@@ -1795,12 +1821,15 @@ int swr_mip_backward(const swr_texture *grad, void *stream) {
   int r = check_chain(grad, 16);
   if (r != SWR_OK) return r;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  for (uint32_t l = grad->level_count - 1; l >= 1; l--) {
+  const uint32_t tail = mip_tail_first(grad);
+  if (tail + 1 < grad->level_count)
+    hipLaunchKernelGGL(mip_up_tail_kernel, dim3(1), dim3(kMipTailThreads), 0, s, mip_tail(grad, tail, 16));
+  for (uint32_t l = std::min(tail, grad->level_count - 1); l >= 1; l--) {
     const swr_image_level &fine = grad->levels[l - 1], &coarse = grad->levels[l];
     dim3 grid((fine.width + 255) / 256, fine.height), block(256);
-    hipLaunchKernelGGL(mip_up_rgba32f_kernel, grid, block, 0, s, (float4 *)fine.data, (int)fine.width,
-                       (int)fine.height, (int)(fine.row_pitch_bytes / 16), (const float4 *)coarse.data,
-                       (int)coarse.width, (int)coarse.height, (int)(coarse.row_pitch_bytes / 16));
+    hipLaunchKernelGGL(mip_up_kernel, grid, block, 0, s, (float4 *)fine.data, (int)fine.width, (int)fine.height,
+                       (int)(fine.row_pitch_bytes / 16), (const float4 *)coarse.data, (int)coarse.width,
+                       (int)coarse.height, (int)(coarse.row_pitch_bytes / 16));
   }
   SWR_HIP_CHECK(hipGetLastError());
   return SWR_OK;

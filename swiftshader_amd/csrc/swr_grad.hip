@@ -21,7 +21,7 @@
 //                      of the pixel's samples: re-derive the fragment,
 //                      scatter dL/dtexel over the filter footprint, and
 //                      dL/d(colour, uv, x, y, w) of the three vertices.
-//   mip_down_kernel    2x2 box filter, level k -> k+1.
+//   mip_down_kernel    2x2 box filter, level k -> k+1 (mip_down_tail_kernel: the small levels at once).
 //   mip_up_kernel      its adjoint, level k+1 -> k (accumulating).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -1276,22 +1276,18 @@ __global__ __launch_bounds__(kScatterThreads) void tap_scatter_kernel(const TapR
   }
 }
 
-// 2x2 box filter (odd sizes: floor, the second texel clamped).
-__global__ void mip_down_rgba32f_kernel(const float4 *src, int sw, int sh, int sp, float4 *dst, int dw, int dh, int dp) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-  if (x >= dw || y >= dh) return;
+// Texel (x, y) of the level below src: 2x2 box filter (odd sizes: floor, the
+// second texel clamped).
+__device__ __forceinline__ float4 mip_box(const float4 *src, int sw, int sh, int sp, int x, int y) {
   const int x0 = 2 * x < sw - 1 ? 2 * x : sw - 1, x1 = 2 * x + 1 < sw - 1 ? 2 * x + 1 : sw - 1;
   const int y0 = 2 * y < sh - 1 ? 2 * y : sh - 1, y1 = 2 * y + 1 < sh - 1 ? 2 * y + 1 : sh - 1;
   const float4 a = src[x0 + (size_t)y0 * sp], b = src[x1 + (size_t)y0 * sp];
   const float4 c = src[x0 + (size_t)y1 * sp], d = src[x1 + (size_t)y1 * sp];
-  dst[x + (size_t)y * dp] = make_float4(((a.x + b.x) + (c.x + d.x)) * 0.25f, ((a.y + b.y) + (c.y + d.y)) * 0.25f,
-                                        ((a.z + b.z) + (c.z + d.z)) * 0.25f, ((a.w + b.w) + (c.w + d.w)) * 0.25f);
+  return make_float4(((a.x + b.x) + (c.x + d.x)) * 0.25f, ((a.y + b.y) + (c.y + d.y)) * 0.25f,
+                     ((a.z + b.z) + (c.z + d.z)) * 0.25f, ((a.w + b.w) + (c.w + d.w)) * 0.25f);
 }
 
-__global__ void mip_down_rgba8_kernel(const uint32_t *src, int sw, int sh, int sp, uint32_t *dst, int dw, int dh,
-                                      int dp) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-  if (x >= dw || y >= dh) return;
+__device__ __forceinline__ uint32_t mip_box(const uint32_t *src, int sw, int sh, int sp, int x, int y) {
   const int x0 = 2 * x < sw - 1 ? 2 * x : sw - 1, x1 = 2 * x + 1 < sw - 1 ? 2 * x + 1 : sw - 1;
   const int y0 = 2 * y < sh - 1 ? 2 * y : sh - 1, y1 = 2 * y + 1 < sh - 1 ? 2 * y + 1 : sh - 1;
   const uint32_t a = src[x0 + (size_t)y0 * sp], b = src[x1 + (size_t)y0 * sp];
@@ -1303,15 +1299,13 @@ __global__ void mip_down_rgba8_kernel(const uint32_t *src, int sw, int sh, int s
                        ((d >> (8 * k)) & 0xFFu) + 2u;
     o |= (s >> 2) << (8 * k);
   }
-  dst[x + (size_t)y * dp] = o;
+  return o;
 }
 
-// Adjoint of mip_down_rgba32f_kernel: texel (x, y) of the finer level
-// receives 0.25 * (its multiplicity in the box) of its parent's gradient.
-__global__ void mip_up_rgba32f_kernel(float4 *fine, int fw, int fh, int fp, const float4 *coarse, int cw, int ch,
-                                      int cp) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
-  if (x >= fw || y >= fh) return;
+// The adjoint at texel (x, y) of the finer level: it receives 0.25 * (its
+// multiplicity in the box) of its parent's gradient.
+__device__ __forceinline__ void mip_box_adjoint(float4 *fine, int fw, int fh, int fp, const float4 *coarse, int cw, int ch,
+                                                int cp, int x, int y) {
   const int mx = fw == 1 ? 2 : (x < 2 * cw ? 1 : 0);
   const int my = fh == 1 ? 2 : (y < 2 * ch ? 1 : 0);
   if (!mx || !my) return;
@@ -1322,6 +1316,60 @@ __global__ void mip_up_rgba32f_kernel(float4 *fine, int fw, int fh, int fp, cons
   f.y += g.y * s;
   f.z += g.z * s;
   f.w += g.w * s;
+}
+
+template <typename T>
+__global__ void mip_down_kernel(const T *src, int sw, int sh, int sp, T *dst, int dw, int dh, int dp) {
+  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
+  if (x >= dw || y >= dh) return;
+  dst[x + (size_t)y * dp] = mip_box(src, sw, sh, sp, x, y);
+}
+
+__global__ void mip_up_kernel(float4 *fine, int fw, int fh, int fp, const float4 *coarse, int cw, int ch, int cp) {
+  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
+  if (x >= fw || y >= fh) return;
+  mip_box_adjoint(fine, fw, fh, fp, coarse, cw, ch, cp, x, y);
+}
+
+// The small end of a mip chain in one launch: one workgroup takes the levels
+// one after the other, with a barrier between (its own writes are visible to
+// it after one).  A level of up to kMipTailTexels takes it some two
+// microseconds, mostly the latency of its loads, a launch of its own over 4 in
+// a replayed graph (16-view step with a 1024^2 texture, both ways of the
+// chain: 1789 -> 1781 us); larger levels need the chip's bandwidth.
+constexpr uint32_t kMipTailTexels = 4096;  // of the finer level
+constexpr int kMipTailThreads = 1024;
+
+struct MipTail {
+  void *data[kMipLevels];
+  int width[kMipLevels], height[kMipLevels], pitch[kMipLevels];
+  int count;  // levels, the finest first
+};
+
+template <typename T>
+__global__ __launch_bounds__(kMipTailThreads) void mip_down_tail_kernel(MipTail M) {
+  for (int l = 1; l < M.count; l++) {
+    const int w = M.width[l], h = M.height[l];
+    T *dst = reinterpret_cast<T *>(M.data[l]);
+    for (int i = threadIdx.x; i < w * h; i += kMipTailThreads) {
+      const int x = i % w, y = i / w;
+      dst[x + (size_t)y * M.pitch[l]] =
+          mip_box(reinterpret_cast<const T *>(M.data[l - 1]), M.width[l - 1], M.height[l - 1], M.pitch[l - 1], x, y);
+    }
+    __threadfence_block();
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(kMipTailThreads) void mip_up_tail_kernel(MipTail M) {
+  for (int l = M.count - 1; l >= 1; l--) {
+    const int w = M.width[l - 1], h = M.height[l - 1];
+    for (int i = threadIdx.x; i < w * h; i += kMipTailThreads)
+      mip_box_adjoint(reinterpret_cast<float4 *>(M.data[l - 1]), w, h, M.pitch[l - 1],
+                      reinterpret_cast<const float4 *>(M.data[l]), M.width[l], M.height[l], M.pitch[l], i % w, i / w);
+    __threadfence_block();
+    __syncthreads();
+  }
 }
 
 template __global__ void backward_kernel<1>(DrawParams, GradParams, const TriRecord *);
