@@ -882,6 +882,9 @@ __global__ __launch_bounds__(256, raster_waves(MS, FCOL, LEVEL, BLEND)) void ras
     lo = __builtin_amdgcn_readfirstlane(lo);
 #pragma nounroll
     for (int pass = pass0; pass < pass1; pass++) {
+      // The counters of the pass before are summed up (raster_tile's red)
+      // before a wave whose block has nothing left writes this pass's.
+      if (pass > pass0) __syncthreads();
       uint32_t s, e;
       if (pass == 0) {
         s = tileStart[t];
