@@ -582,7 +582,9 @@ int swr_batch_plan_autotune(swr_batch_plan *plan, swr_tuning *best, void *stream
 
 /* Sets the gradient targets of a plan's draws (one swr_grad_desc per
  * planned draw, in the order the draws were given; see swr_grad_desc).  The
- * buffers they name must stay allocated while the plan is used.
+ * buffers they name must stay allocated while the plan is used.  A backward
+ * captured into a HIP graph uses the targets set last before each replay, as
+ * long as the same draws want texture gradients.
  * Synchronises `stream`. */
 int swr_batch_plan_set_grads(swr_batch_plan *plan, const swr_grad_desc *grads, uint32_t count, void *stream);
 

@@ -1339,7 +1339,10 @@ struct swr_batch_plan {
   std::vector<swr_grad_desc> gradDescs;  // caller order
   Scratch gparams, gbase;
   std::vector<uint32_t> bwBase;
-  std::vector<uint8_t> bwAttr;  // per draw: wants gradients of vertex attributes
+  // Per segment and group of draws of one sample count (at most two, which the
+  // layout keeps apart): whether a draw wants gradients of vertex attributes.
+  // gbase holds bwBase and then these.
+  std::vector<uint32_t> bwAttr;
   bool hasGrads = false;
   // Binned texel scatter, per segment (see BinArgs): whether it is used,
   // its bucket count, record capacity and offsets into the plan's tables.
@@ -1621,12 +1624,23 @@ int plan_build_bins(swr_batch_plan *pl, const std::vector<GradParams> &G, int cu
   return SWR_OK;
 }
 
+// Calls f(group, lo, hi) for each run of draws [lo, hi) of segment sg that
+// have one sample count (contiguous: the layout orders draws by variant).
+template <typename F>
+void each_sample_group(const BatchLayout &L, const BatchLayout::Seg &sg, const F &f) {
+  for (int lo = 0, hi, group = 0; lo < sg.count; lo = hi, group++) {
+    for (hi = lo + 1; hi < sg.count && L.P[sg.first + hi].ms == L.P[sg.first + lo].ms;) hi++;
+    f(group, lo, hi);
+  }
+}
+
 int plan_upload_grads(DeviceCtx *c, swr_batch_plan *pl, hipStream_t s) {
   const size_t n = pl->L.P.size();
   std::vector<GradParams> G(n);
   pl->bwBase.assign(n, 0);
-  pl->bwAttr.assign(n, 0);
-  for (const auto &sg : pl->L.segs) {
+  pl->bwAttr.assign(2 * pl->L.segs.size(), 0);
+  for (size_t si = 0; si < pl->L.segs.size(); si++) {
+    const auto &sg = pl->L.segs[si];
     uint32_t base = 0;
     for (int k = 0; k < sg.count; k++) {
       const int i = sg.first + k;
@@ -1635,21 +1649,30 @@ int plan_upload_grads(DeviceCtx *c, swr_batch_plan *pl, hipStream_t s) {
       int r = grad_params(&pl->descs[o], P, &pl->gradDescs[o], G[i]);
       if (r != SWR_OK) return fail(r, "draw %d: %s", o, g_error.c_str());
       pl->bwBase[i] = base;
-      pl->bwAttr[i] = G[i].dPos || G[i].dCol || G[i].dUV;
       base += (uint32_t)(((P.width + 15) / 16) * ((P.height + 15) / 16));
     }
+    each_sample_group(pl->L, sg, [&](int group, int lo, int hi) {
+      for (int i = sg.first + lo; i < sg.first + hi; i++)
+        if (G[i].dPos || G[i].dCol || G[i].dUV) pl->bwAttr[2 * si + group] = 1;
+    });
   }
   if (!n) return SWR_OK;
   SWR_HIP_CHECK(pl->gparams.ensure(sizeof(GradParams) * n));
-  SWR_HIP_CHECK(pl->gbase.ensure(sizeof(uint32_t) * n));
+  SWR_HIP_CHECK(pl->gbase.ensure(sizeof(uint32_t) * (n + pl->bwAttr.size())));
   SWR_HIP_CHECK(hipMemcpyAsync(pl->gparams.ptr, G.data(), sizeof(GradParams) * n, hipMemcpyHostToDevice, s));
   SWR_HIP_CHECK(hipMemcpyAsync(pl->gbase.ptr, pl->bwBase.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, s));
+  SWR_HIP_CHECK(hipMemcpyAsync(pl->gbase.as<uint32_t>() + n, pl->bwAttr.data(), sizeof(uint32_t) * pl->bwAttr.size(),
+                               hipMemcpyHostToDevice, s));
   SWR_HIP_CHECK(hipStreamSynchronize(s));
   return plan_build_bins(pl, G, c->cus, s);
 }
 
 int plan_enqueue_backward(swr_batch_plan *pl, int cus, hipStream_t s) {
   Pipeline &pipe = pl->pipe;
+  // A captured backward runs for the gradient targets set at each replay.
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+  const bool captured = capture != hipStreamCaptureStatusNone;
   for (size_t si = 0; si < pl->L.segs.size(); si++) {
     const auto &sg = pl->L.segs[si];
     const auto &sb = pl->bins.size() > si ? pl->bins[si] : swr_batch_plan::SegBins{};
@@ -1675,33 +1698,31 @@ int plan_enqueue_backward(swr_batch_plan *pl, int cus, hipStream_t s) {
     // each group gets its own work counter (counters[kBackwardSlot + group]).
     uint32_t *ctr = pipe.counters.as<uint32_t>() + kBackwardSlot;
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, ctr, 0u, 2u);
-    int group = 0;
-    int lo = 0;
-    while (lo < sg.count) {
+    const TriRecord *rec = pipe.rec.as<TriRecord>();
+    each_sample_group(pl->L, sg, [&](int group, int lo, int hi) {
       const int ms = pl->L.P[sg.first + lo].ms;
-      int hi = lo + 1;
-      while (hi < sg.count && pl->L.P[sg.first + hi].ms == ms) hi++;
       const uint32_t bLo = pl->bwBase[sg.first + lo];
       const DrawParams &Ph = pl->L.P[sg.first + hi - 1];
       const uint32_t bHi = pl->bwBase[sg.first + hi - 1] + (uint32_t)(((Ph.width + 15) / 16) * ((Ph.height + 15) / 16));
-      if (bHi > bLo) {
-        const bool attr = std::any_of(pl->bwAttr.begin() + sg.first + lo, pl->bwAttr.begin() + sg.first + hi,
-                                      [](uint8_t a) { return a != 0; });
-        const uint32_t wgs = std::min<uint32_t>(bHi - bLo, (uint32_t)(cus * gather_per_cu(ms, sb.on, attr || !sb.on)));
-        const TriRecord *rec = pipe.rec.as<TriRecord>();
-        auto launch = [&](auto *kernel) {
-          hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi, bLo, bHi, ctr + group, rec,
-                             bin);
-        };
-        // Draws that want only the texture's gradient take the kernels without
-        // vertex attributes, whatever their number: they do strictly less.
-        if (!sb.on) launch(ms == 1 ? backward_batch_kernel<1, false, true> : backward_batch_kernel<4, false, true>);
-        else if (attr) launch(ms == 1 ? backward_batch_kernel<1, true, true> : backward_batch_kernel<4, true, true>);
-        else launch(ms == 1 ? backward_batch_kernel<1, true, false> : backward_batch_kernel<4, true, false>);
-      }
-      group++;
-      lo = hi;
-    }
+      if (bHi <= bLo) return;
+      const bool attr = pl->bwAttr[2 * si + group] || !sb.on;
+      // Draws that want only the texture's gradient take the kernels without
+      // vertex attributes, whatever their number: they do strictly less.  When
+      // they are captured, the kernel with attributes is captured beside them
+      // (it leaves at once: a replay of 106 us takes 108, one of 256 us 260),
+      // for targets that are set later.
+      const uint32_t *wants =
+          captured && !attr ? pl->gbase.as<uint32_t>() + pl->L.P.size() + 2 * si + group : nullptr;
+      auto launch = [&](bool a, auto *kernel) {
+        const uint32_t wgs = std::min<uint32_t>(bHi - bLo, (uint32_t)(cus * gather_per_cu(ms, sb.on, a)));
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi, bLo, bHi, ctr + group, rec,
+                           bin, wants);
+      };
+      if (!sb.on) launch(true, ms == 1 ? backward_batch_kernel<1, false, true> : backward_batch_kernel<4, false, true>);
+      else if (attr || wants)
+        launch(true, ms == 1 ? backward_batch_kernel<1, true, true> : backward_batch_kernel<4, true, true>);
+      if (!attr) launch(false, ms == 1 ? backward_batch_kernel<1, true, false> : backward_batch_kernel<4, true, false>);
+    });
     if (sb.on) {
       // The reserved slots sorted by bucket (stable radix sort of (key,
       // slot); unused slots carry a key above every bucket and sort last),

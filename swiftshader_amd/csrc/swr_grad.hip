@@ -912,6 +912,9 @@ __global__ __launch_bounds__(256) void backward_kernel(DrawParams P, GradParams 
 // the same draw.  With BIN there are no texel tables: the draws' texel
 // gradients leave as footprint records (bin), which tap_scatter_kernel
 // scatters.
+// `wants` (NULL: no such choice): whether the launch's draws want gradients of
+// vertex attributes, as swr_batch_plan_set_grads last said; the launch does
+// nothing unless that is ATTR.
 template <int MS, bool BIN, bool ATTR>
 __global__ __launch_bounds__(256, gather_per_cu(MS, BIN, ATTR)) void backward_batch_kernel(
                                                              const DrawParams *__restrict__ params,
@@ -919,7 +922,9 @@ __global__ __launch_bounds__(256, gather_per_cu(MS, BIN, ATTR)) void backward_ba
                                                              const uint32_t *__restrict__ blockBase, int drawLo,
                                                              int drawHi, uint32_t blockLo, uint32_t blockHi,
                                                              uint32_t *__restrict__ counter,
-                                                             const TriRecord *__restrict__ rec, BinArgs bin) {
+                                                             const TriRecord *__restrict__ rec, BinArgs bin,
+                                                             const uint32_t *__restrict__ wants) {
+  if (wants && (*wants != 0) != ATTR) return;
   __shared__ GradLds<BIN> S;
   __shared__ FragQueue Q;
   __shared__ uint32_t sBlock;
@@ -1376,21 +1381,21 @@ template __global__ void backward_kernel<1>(DrawParams, GradParams, const TriRec
 template __global__ void backward_kernel<4>(DrawParams, GradParams, const TriRecord *);
 template __global__ void backward_batch_kernel<1, false, true>(const DrawParams *, const GradParams *, const uint32_t *,
                                                               int, int, uint32_t, uint32_t, uint32_t *,
-                                                              const TriRecord *, BinArgs);
+                                                              const TriRecord *, BinArgs, const uint32_t *);
 template __global__ void backward_batch_kernel<1, true, true>(const DrawParams *, const GradParams *, const uint32_t *,
                                                               int, int, uint32_t, uint32_t, uint32_t *,
-                                                              const TriRecord *, BinArgs);
+                                                              const TriRecord *, BinArgs, const uint32_t *);
 template __global__ void backward_batch_kernel<1, true, false>(const DrawParams *, const GradParams *, const uint32_t *,
                                                               int, int, uint32_t, uint32_t, uint32_t *,
-                                                              const TriRecord *, BinArgs);
+                                                              const TriRecord *, BinArgs, const uint32_t *);
 template __global__ void backward_batch_kernel<4, false, true>(const DrawParams *, const GradParams *, const uint32_t *,
                                                               int, int, uint32_t, uint32_t, uint32_t *,
-                                                              const TriRecord *, BinArgs);
+                                                              const TriRecord *, BinArgs, const uint32_t *);
 template __global__ void backward_batch_kernel<4, true, true>(const DrawParams *, const GradParams *, const uint32_t *,
                                                               int, int, uint32_t, uint32_t, uint32_t *,
-                                                              const TriRecord *, BinArgs);
+                                                              const TriRecord *, BinArgs, const uint32_t *);
 template __global__ void backward_batch_kernel<4, true, false>(const DrawParams *, const GradParams *, const uint32_t *,
                                                               int, int, uint32_t, uint32_t, uint32_t *,
-                                                              const TriRecord *, BinArgs);
+                                                              const TriRecord *, BinArgs, const uint32_t *);
 
 }  // namespace swr
