@@ -1535,10 +1535,29 @@ bool same_tap_target(const DrawParams &A, const GradParams &Ga, const DrawParams
   return true;
 }
 
+// Calls f(group, lo, hi) for each run of draws [lo, hi) of segment sg that
+// have one sample count (contiguous: the layout orders draws by variant).
+template <typename F>
+void each_sample_group(const BatchLayout &L, const BatchLayout::Seg &sg, const F &f) {
+  for (int lo = 0, hi, group = 0; lo < sg.count; lo = hi, group++) {
+    for (hi = lo + 1; hi < sg.count && L.P[sg.first + hi].ms == L.P[sg.first + lo].ms;) hi++;
+    f(group, lo, hi);
+  }
+}
+
+// 16x16-pixel blocks of a draw, as the gather walks it.
+uint32_t gather_blocks(const DrawParams &P) { return (uint32_t)(((P.width + 15) / 16) * ((P.height + 15) / 16)); }
+
+// Workgroups of the gather launch over `blocks` 16x16-pixel blocks.
+uint32_t gather_workgroups(uint32_t blocks, int cus, int ms, bool bin, bool attr) {
+  return std::min<uint32_t>(blocks, (uint32_t)(cus * gather_per_cu(ms, bin, attr)));
+}
+
 // Per segment: the texture groups of its draws, their bucket tables and the
 // record slots: one per sample of every draw with texture gradients (a
-// bound on its fragments) plus the last reservation of every wave the
-// gather can launch (a segment with more groups than kMaxBinGroups, or more
+// bound on its fragments) plus the last reservation of every wave of the
+// segment's gather launches, with or without attribute gradients, so that a
+// captured backward may take either (a segment with more groups than kMaxBinGroups, or more
 // slots than 32-bit indices hold, keeps the texel tables).
 int plan_build_bins(swr_batch_plan *pl, const std::vector<GradParams> &G, int cus, hipStream_t s) {
   pl->bins.assign(pl->L.segs.size(), swr_batch_plan::SegBins{});
@@ -1568,8 +1587,14 @@ int plan_build_bins(swr_batch_plan *pl, const std::vector<GradParams> &G, int cu
       dg[k] = (int8_t)gi;
       cap += (uint64_t)P.width * (uint64_t)P.height * (uint64_t)P.ms;
     }
-    // Up to two gather launches (one per sample count).
-    cap += 2ull * (uint64_t)cus * kGatherSlack;
+    each_sample_group(pl->L, sg, [&](int, int lo, int hi) {
+      uint32_t blocks = 0, slack = 0;
+      for (int i = sg.first + lo; i < sg.first + hi; i++) blocks += gather_blocks(pl->L.P[i]);
+      for (bool attr : {false, true})
+        slack = std::max(slack, gather_workgroups(blocks, cus, pl->L.P[sg.first + lo].ms, true, attr) * 4u *
+                                    bin_reserve(attr));
+      cap += slack;
+    });
     if (!ok || rep.empty() || cap >= (1ull << 31)) continue;
     sb.on = true;
     sb.cap = (uint32_t)cap;
@@ -1624,16 +1649,6 @@ int plan_build_bins(swr_batch_plan *pl, const std::vector<GradParams> &G, int cu
   return SWR_OK;
 }
 
-// Calls f(group, lo, hi) for each run of draws [lo, hi) of segment sg that
-// have one sample count (contiguous: the layout orders draws by variant).
-template <typename F>
-void each_sample_group(const BatchLayout &L, const BatchLayout::Seg &sg, const F &f) {
-  for (int lo = 0, hi, group = 0; lo < sg.count; lo = hi, group++) {
-    for (hi = lo + 1; hi < sg.count && L.P[sg.first + hi].ms == L.P[sg.first + lo].ms;) hi++;
-    f(group, lo, hi);
-  }
-}
-
 int plan_upload_grads(DeviceCtx *c, swr_batch_plan *pl, hipStream_t s) {
   const size_t n = pl->L.P.size();
   std::vector<GradParams> G(n);
@@ -1649,7 +1664,7 @@ int plan_upload_grads(DeviceCtx *c, swr_batch_plan *pl, hipStream_t s) {
       int r = grad_params(&pl->descs[o], P, &pl->gradDescs[o], G[i]);
       if (r != SWR_OK) return fail(r, "draw %d: %s", o, g_error.c_str());
       pl->bwBase[i] = base;
-      base += (uint32_t)(((P.width + 15) / 16) * ((P.height + 15) / 16));
+      base += gather_blocks(P);
     }
     each_sample_group(pl->L, sg, [&](int group, int lo, int hi) {
       for (int i = sg.first + lo; i < sg.first + hi; i++)
@@ -1702,8 +1717,7 @@ int plan_enqueue_backward(swr_batch_plan *pl, int cus, hipStream_t s) {
     each_sample_group(pl->L, sg, [&](int group, int lo, int hi) {
       const int ms = pl->L.P[sg.first + lo].ms;
       const uint32_t bLo = pl->bwBase[sg.first + lo];
-      const DrawParams &Ph = pl->L.P[sg.first + hi - 1];
-      const uint32_t bHi = pl->bwBase[sg.first + hi - 1] + (uint32_t)(((Ph.width + 15) / 16) * ((Ph.height + 15) / 16));
+      const uint32_t bHi = pl->bwBase[sg.first + hi - 1] + gather_blocks(pl->L.P[sg.first + hi - 1]);
       if (bHi <= bLo) return;
       const bool attr = pl->bwAttr[2 * si + group] || !sb.on;
       // Draws that want only the texture's gradient take the kernels without
@@ -1714,9 +1728,8 @@ int plan_enqueue_backward(swr_batch_plan *pl, int cus, hipStream_t s) {
       const uint32_t *wants =
           captured && !attr ? pl->gbase.as<uint32_t>() + pl->L.P.size() + 2 * si + group : nullptr;
       auto launch = [&](bool a, auto *kernel) {
-        const uint32_t wgs = std::min<uint32_t>(bHi - bLo, (uint32_t)(cus * gather_per_cu(ms, sb.on, a)));
-        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, s, params, grads, bb, lo, hi, bLo, bHi, ctr + group, rec,
-                           bin, wants);
+        hipLaunchKernelGGL(kernel, dim3(gather_workgroups(bHi - bLo, cus, ms, sb.on, a)), dim3(256), 0, s, params,
+                           grads, bb, lo, hi, bLo, bHi, ctr + group, rec, bin, wants);
       };
       if (!sb.on) launch(true, ms == 1 ? backward_batch_kernel<1, false, true> : backward_batch_kernel<4, false, true>);
       else if (attr || wants)

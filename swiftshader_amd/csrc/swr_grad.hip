@@ -79,9 +79,6 @@ constexpr uint32_t bin_reserve(bool attr) { return attr ? 512 : 256; }
 // 17.7 -> 18.2 ms), and the texel tables of the kernels without records fill
 // the LDS at two.
 constexpr int gather_per_cu(int ms, bool bin, bool attr) { return !attr ? 5 : ms == 1 && bin ? 3 : 2; }
-// Slots that the last reservations of all of a launch's waves may leave unused, per CU.
-constexpr uint32_t kGatherSlack = 4u * 3u * bin_reserve(true);
-static_assert(4u * 5u * bin_reserve(false) <= kGatherSlack, "slack of the attribute-free kernels");
 constexpr uint32_t kNoBucket = 0xFFFFFFFFu;           // key of a reserved slot left unused
 
 // Footprint of one fragment: texture coordinate, frozen sampling state and
