@@ -34,11 +34,13 @@ __device__ __forceinline__ int32_t rr_trunc_int(float x) {
   if (!(x >= -2147483648.0f && x < 2147483648.0f)) return INT32_MIN;
   return (int32_t)__builtin_truncf(x);
 }
-// 1 / x, correctly rounded, as the division gives it: two Newton steps in
-// fused arithmetic from the hardware's estimate (within one unit in the last
-// place) round correctly (Markstein, IBM J. Res. Dev. 34, 1990), and the fixup
-// restores zeros, infinities and NaN.  Checked against the division over all
-// 2^32 arguments; five instructions instead of eleven.
+// 1 / x, correctly rounded, as the division gives it, in four instructions
+// instead of eleven: one Newton step in fused arithmetic (Markstein, IBM J.
+// Res. Dev. 34, 1990) from the hardware's estimate, which is within one unit in
+// the last place, and the fixup for zeros, infinities and NaN.  One step is
+// not proven to round correctly from every such estimate: it is the sweep of
+// all 2^32 arguments against the division that shows it does
+// (tests/device_numerics.hip).
 __device__ __forceinline__ float rr_rcp(float x) {
   const float r = __builtin_amdgcn_rcpf(x);
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r), x, 1.0f);
@@ -577,8 +579,8 @@ __device__ __forceinline__ float unorm8_to_float(uint32_t b) { return (float)b *
 
 // The four channels clamped to [0, 1], scaled by 255 and rounded to nearest
 // even (a NaN becomes 0), packed R, G, B, A from the low byte.  The hardware's
-// conversion clamps, rounds and packs (checked against the separate steps over
-// all 2^32 arguments).
+// conversion clamps, rounds and packs (tests/device_numerics.hip compares it
+// with the separate steps over all 2^32 arguments).
 __device__ __forceinline__ uint32_t float4_to_unorm8(float4 c) {
   uint32_t v = __builtin_amdgcn_cvt_pk_u8_f32(c.x * 255.0f, 0, 0);
   v = __builtin_amdgcn_cvt_pk_u8_f32(c.y * 255.0f, 1, v);
