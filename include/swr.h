@@ -624,7 +624,9 @@ typedef struct swr_profile {
   uint64_t pairs;    /* (tile, triangle) pairs binned                  */
   uint64_t block_tests;    /* (8x8 block, primitive) coverage evaluations */
   uint64_t block_covers;   /* ... of which covered at least one sample    */
-  uint64_t shaded;         /* fragments shaded (passed all tests)         */
+  uint64_t shaded;         /* fragments that passed all tests and write
+                              colour: a blended draw shades each of them, an
+                              unblended one only the last of each sample     */
 } swr_profile;
 
 /* Enables (1) or disables (0) event recording on the current device. */

@@ -121,7 +121,7 @@ struct DrawParams {
   int primIdPitch;
   long long primIdSlice;
   unsigned long long *occlusion;
-  unsigned long long *stats;  // [block tests, block covers, shaded] or NULL
+  unsigned long long *stats;  // [block tests, block covers, fragments past every test] or NULL
   // Tiling.
   int tileW, tileH, tilesX, tilesY;
   int triBase;  // first record slot of this draw's primitives in its batch
@@ -136,7 +136,8 @@ struct TriRecord {
   int yMin, yMax;   // rows with possible coverage (scissor-clamped)
   int xMin, xMax;   // pixel columns with possible coverage
   int X[3], Y[3];   // 28.4 polygon vertices when n == 3
-  float zlo;        // lower bound of the evaluated depth (bias included) over the bounding box
+  float zlo;        // lower bound of the evaluated depth (bias included): the plane at the polygon's
+                    // vertices, less a margin of its terms' size over the bounding box
   float x0, y0;
   float zA, zB, zC;
   float zBias;      // depth bias added to every sample's depth (0 when off)

@@ -345,7 +345,9 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   // has no side effect (no stencil writes).
   const bool hiz = depthTest && !stencilWrite && (P.depthCompare == 1 || P.depthCompare == 3);
 
-  // Wave totals; nTests, nCovers and nShaded are statistics (profiling only).
+  // Wave totals; nTests, nCovers and nShaded (fragments that passed every test,
+  // whether or not a later one replaces them unshaded) are statistics
+  // (profiling only).
   unsigned long long occl = 0, nTests = 0, nCovers = 0, nShaded = 0;
   // The queue is a ring of two batches; a batch is shaded when it is full
   // (and the last one at the end), so every lane of it has a fragment.
