@@ -159,7 +159,7 @@ __device__ __forceinline__ int lane_cy(int l) { return 2 * (l >> 4) + ((l >> 1) 
 // Blend a shaded colour into the samples of this lane's pixel selected by
 // xMask, then write (PixelRoutine.cpp:1617-2936).
 // srgbLut: srgb_to_linear of every 8-bit code (sRGB targets).
-// FAST: blending, when on, is SRC_ALPHA, ONE_MINUS_SRC_ALPHA, ADD.
+// FAST: the blend is SRC_ALPHA, ONE_MINUS_SRC_ALPHA, ADD.
 template <int MS, bool FCOL, bool XF, bool FAST = false>
 __device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, FCOL, true> &S, float4 s, int xMask,
                                             uint32_t tri, const float *srgbLut) {
@@ -173,13 +173,13 @@ __device__ __forceinline__ void blend_write(const DrawParams &P, PixelState<MS, 
       const uint32_t p = S.cb[FCOL ? 0 : q];
       dst = make_float4(unorm8_to_float(p & 0xFFu), unorm8_to_float((p >> 8) & 0xFFu),
                         unorm8_to_float((p >> 16) & 0xFFu), unorm8_to_float(p >> 24));
-      if ((XF && P.colorSRGB) && P.blendEnable) {  // blended in linear space (PixelRoutine.cpp:1811-1827)
+      if (XF && P.colorSRGB) {  // blended in linear space (PixelRoutine.cpp:1811-1827)
         dst.x = srgbLut[p & 0xFFu];
         dst.y = srgbLut[(p >> 8) & 0xFFu];
         dst.z = srgbLut[(p >> 16) & 0xFFu];
       }
     }
-    float4 o = P.blendEnable ? (FAST ? blend_src_alpha(s, dst) : alpha_blend<XF>(P, s, dst)) : s;
+    float4 o = FAST ? blend_src_alpha(s, dst) : alpha_blend<XF>(P, s, dst);
     if (!FCOL && (XF && P.colorSRGB)) {  // writeColor encodes R, G, B first (PixelRoutine.cpp:1963-1969)
       o.x = linear_to_srgb(o.x);
       o.y = linear_to_srgb(o.y);
