@@ -136,6 +136,26 @@ __device__ __forceinline__ int wave_max_i32(int v) {
   return __builtin_amdgcn_readlane(v, 63);
 }
 
+// The lanes where p holds (all of them must be asked: as __ballot, without its
+// detour through a vector register).
+__device__ __forceinline__ uint64_t lanes_where(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+// The depth compare op as its result where the stored depth is above the
+// fragment's (or either is NaN), equal to it, and below it: every op, with its
+// results for NaN, is a function of stored <= z and stored < z.
+struct DepthPass {
+  bool above, equal, below;
+  __device__ __forceinline__ bool operator()(float stored, float z) const {
+    const bool le = stored <= z, lt = stored < z;
+    return (lt & below) | (le & !lt & equal) | (!le & above);
+  }
+};
+__device__ __forceinline__ DepthPass depth_pass(const DrawParams &P) {
+  const bool inv = P.zInv != 0;
+  const int k = P.zPred;  // le, lt, eq, true
+  return {(k == 3) != inv, (k != 1) != inv, (k != 2) != inv};
+}
+
 // What a wave keeps of its block, per lane one pixel.  With BLEND the colours
 // themselves; without it the primitive that last wrote each sample: an
 // unblended fragment is replaced whole by the next one, so only the last one
@@ -268,6 +288,20 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   const bool depthBias = !SIMPLE && P.depthBias, depthTest = SIMPLE || P.depthTest;
   const bool depthWrite = SIMPLE || P.depthWrite;
   const int colorMask = SIMPLE ? 15 : P.colorMask;
+  // What the candidate loop asks of the draw, loaded here: read in the branches
+  // that use them, the fields cost a scalar load and a wait each per candidate,
+  // and a target of few blocks has one wave per SIMD, which nothing hides them
+  // behind (300x169 pixels, 40,000 blended triangles in display formats with
+  // stencil: 1137 us a draw, 830 with the stencil table and the compares below
+  // as well).  With four samples the common states need the registers: their
+  // depth range is read where it is used (4x frame 566 -> 562 us).
+  constexpr bool KEEP_RANGE = !(SIMPLE && MS > 1);
+  const int msMask = P.msMask, depthCompare = P.depthCompare;
+  const DepthPass zp = depth_pass(P);
+  const float rangeLo = P.depthClampLo, rangeHi = P.depthClampHi;
+  auto range_lo = [&]() __attribute__((always_inline)) { return KEEP_RANGE ? rangeLo : P.depthClampLo; };
+  auto range_hi = [&]() __attribute__((always_inline)) { return KEEP_RANGE ? rangeHi : P.depthClampHi; };
+  const bool depth16 = XF && P.depth16, depthBounds = XF && P.depthBounds, alphaToCoverage = XF && P.alphaToCoverage;
   // Per-wave queue of fragments that passed the tests and await shading,
   // in API order: primitive, owner lane | sample mask << 8, shaded colour.
   constexpr bool QUEUE = BLEND || MS > 1;  // without blending, one pixel is one fragment unless it has samples
@@ -314,11 +348,11 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
       if (P.primId)
         S.id[q] = *reinterpret_cast<const uint32_t *>(P.primId + q * P.primIdSlice + (long long)py * P.primIdPitch +
                                                       4ll * px);
-    if (depthTest || (XF && P.depthBounds))  // D16 holds the float of its integer (readDepth16, PixelRoutine.cpp:466-481)
-      S.zb[q] = (XF && P.depth16) ? (float)*reinterpret_cast<const uint16_t *>(P.depth + q * P.depthSlice +
-                                                                        (long long)py * P.depthPitch + 2ll * px)
-                          : *reinterpret_cast<const float *>(P.depth + q * P.depthSlice +
-                                                             (long long)py * P.depthPitch + 4ll * px);
+    if (depthTest || depthBounds)  // D16 holds the float of its integer (readDepth16, PixelRoutine.cpp:466-481)
+      S.zb[q] = depth16 ? (float)*reinterpret_cast<const uint16_t *>(P.depth + q * P.depthSlice +
+                                                                     (long long)py * P.depthPitch + 2ll * px)
+                        : *reinterpret_cast<const float *>(P.depth + q * P.depthSlice +
+                                                           (long long)py * P.depthPitch + 4ll * px);
     if (stencilActive) S.sb[q] = (uint8_t)P.stencil[q * P.stencilSlice + (long long)py * P.stencilPitch + px];
     if constexpr (BLEND) {
       if constexpr (FCOL)
@@ -330,6 +364,24 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
             *reinterpret_cast<const uint32_t *>(P.color + q * P.colorSlice + (long long)py * P.colorPitch + 4ll * px));
     }
   }
+
+  // What a stencil value becomes: where its test fails in bits 0-7, where the
+  // depth test fails in 8-15 and where both pass in 16-23, write mask applied;
+  // bit 31: the test passes.  For each face one entry a value, so that a
+  // candidate costs a read of LDS instead of the compare and three ops.
+  __shared__ uint32_t stencilTable[SIMPLE ? 1 : 2][SIMPLE ? 1 : 256];
+  if constexpr (!SIMPLE)
+    if (stencilActive) {
+      for (uint32_t i = threadIdx.x; i < 512; i += blockDim.x) {
+        const StencilParams &SP = i < 256 ? P.front : P.back;
+        const uint32_t v = i & 255u, keep = v & ~SP.writeMask, wm = SP.writeMask;
+        stencilTable[i >> 8][v] = (keep | (stencil_apply_op(v, SP.fail) & wm)) |
+                                  (keep | (stencil_apply_op(v, SP.depthFail) & wm)) << 8 |
+                                  (keep | (stencil_apply_op(v, SP.pass) & wm)) << 16 |
+                                  (stencil_compare(SP, v) ? 0x80000000u : 0u);
+      }
+      __syncthreads();
+    }
 
   // The 256 decoded codes of an sRGB target that is blended, so that a blend
   // reads its three channels instead of evaluating three powers.
@@ -343,12 +395,13 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   // by zlo cannot pass LESS (LESS_OR_EQUAL) anywhere in a block whose
   // largest stored depth is <= zlo (< zlo).  Only when a failing fragment
   // has no side effect (no stencil writes).
-  const bool hiz = depthTest && !stencilWrite && (P.depthCompare == 1 || P.depthCompare == 3);
+  const bool hiz = depthTest && !stencilWrite && (depthCompare == 1 || depthCompare == 3);
 
   // Wave totals; nTests, nCovers and nShaded (fragments that passed every test,
   // whether or not a later one replaces them unshaded) are statistics
   // (profiling only).
-  unsigned long long occl = 0, nTests = 0, nCovers = 0, nShaded = 0;
+  unsigned long long occl = 0, nShaded = 0;
+  uint32_t nTests = 0, nCovers = 0;
   // The queue is a ring of two batches; a batch is shaded when it is full
   // (and the last one at the end), so every lane of it has a fragment.
   int qHead = 0, qCount = 0;  // wave-uniform: first entry (0 or 64), entries
@@ -390,7 +443,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   // Queues the fragment of the lanes that `want` it: primitive tri on their
   // pixel's samples xMask.
   auto enqueue = [&](bool want, uint32_t tri, uint32_t xMask) __attribute__((always_inline)) {
-    const uint64_t need = __ballot(want);
+    const uint64_t need = lanes_where(want);
     const int pos = qCount + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
     if (want) {
@@ -422,7 +475,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     return __ballot(nan) ? __builtin_inff() : __int_as_float(m ^ ((m >> 31) & 0x7FFFFFFF));
   };
   auto hidden = [&](float zl, float zmax) __attribute__((always_inline)) {
-    return P.depthCompare == 1 ? zl >= zmax : zl > zmax;
+    return depthCompare == 1 ? zl >= zmax : zl > zmax;
   };
 
   // One batch of candidates, set up one per lane and then read back one at a
@@ -473,8 +526,8 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
                           2.0f * fabsf(zB) * fmaxf(fabsf(ya), fabsf(yb)) + 2.0f * fabsf(zBias);
         zl = fmaxf(__int_as_float(h2.w), m - mag * 0x1p-19f);
         if (!(zl == zl)) zl = -__builtin_inff();
-        zl = fminf(zl, P.depthClampHi);
-        if ((XF && P.depth16)) zl = d16_value(fmaxf(zl, 0.0f));  // the bound in stored units (monotone map)
+        zl = fminf(zl, range_hi());
+        if (depth16) zl = d16_value(fmaxf(zl, 0.0f));  // the bound in stored units (monotone map)
         act = act && !hidden(zl, zmax0);
       }
     }
@@ -548,12 +601,12 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
           cov[q] = span_covers(vtx, n, d, 16 * px + (MS > 1 ? kXf[q] : 0), 16 * py + (MS > 1 ? kYf[q] : 0));
       }
 #pragma unroll
-      for (int q = 0; q < MS; q++) cov[q] = cov[q] && inside && ((P.msMask >> q) & 1);
+      for (int q = 0; q < MS; q++) cov[q] = cov[q] & inside & (((msMask >> q) & 1) != 0);
       nTests++;
       bool anyCov = false;
 #pragma unroll
       for (int q = 0; q < MS; q++) anyCov |= cov[q];
-      if (!__ballot(anyCov)) continue;
+      if (!lanes_where(anyCov)) continue;
       nCovers++;
 
       bool pass[MS];  // samples that pass every test
@@ -569,33 +622,34 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
           const float Dz = c + yy * b;
           // clampDepth; the common state's range is of ordinary floats, for
           // which the hardware's max and min equal the ordered selects.
-          zq[q] = fminf(fmaxf(xx * a + Dz, P.depthClampLo), P.depthClampHi);
+          zq[q] = fminf(fmaxf(xx * a + Dz, range_lo()), range_hi());
         }
-        // The compare op without branches per fragment: one of zb <= z,
-        // zb < z, zb == z or true, inverted for LESS, LESS_OR_EQUAL,
-        // NOT_EQUAL and NEVER; LESS on its own.
-        if (P.depthCompare == 1) {
+        // LESS on its own: one compare.
+        if (depthCompare == 1) {
 #pragma unroll
-          for (int q = 0; q < MS; q++) pass[q] = cov[q] && !(S.zb[q] <= zq[q]);
+          for (int q = 0; q < MS; q++) pass[q] = cov[q] & !(S.zb[q] <= zq[q]);
         } else {
 #pragma unroll
-          for (int q = 0; q < MS; q++) {
-            const bool le = S.zb[q] <= zq[q], lt = S.zb[q] < zq[q], eq = S.zb[q] == zq[q];
-            const bool pr = P.zPred == 0 ? le : (P.zPred == 1 ? lt : (P.zPred == 2 ? eq : true));
-            pass[q] = cov[q] && pr != (P.zInv != 0);
-          }
+          for (int q = 0; q < MS; q++) pass[q] = cov[q] & zp(S.zb[q], zq[q]);
         }
 #pragma unroll
         for (int q = 0; q < MS; q++) {
           S.zb[q] = pass[q] ? zq[q] : S.zb[q];
-          occl += (unsigned)__builtin_popcountll(__ballot(pass[q]));
+          occl += (unsigned)__builtin_popcountll(lanes_where(pass[q]));
         }
       } else {
-        const StencilParams &SP = ((frontLanes >> j) & 1) ? P.front : P.back;
         bool sPass[MS], zPass[MS];
+        uint32_t st[MS];  // stencil table entries; all ones: no stencil test, which passes
 #pragma unroll
-        for (int q = 0; q < MS; q++) sPass[q] = stencilActive ? cov[q] && stencil_compare(SP, S.sb[q]) : cov[q];
-        if (XF && P.alphaToCoverage) {
+        for (int q = 0; q < MS; q++) st[q] = ~0u;
+        if (stencilActive) {
+          const uint32_t *table = stencilTable[(frontLanes >> j) & 1 ? 0 : 1];
+#pragma unroll
+          for (int q = 0; q < MS; q++) st[q] = table[S.sb[q]];
+        }
+#pragma unroll
+        for (int q = 0; q < MS; q++) sPass[q] = cov[q] & ((int)st[q] < 0);
+        if (alphaToCoverage) {
           // The reference shades before the depth test and keeps sample q
           // only where !(alpha < a2c[q]) (alphaTest / alphaToCoverage,
           // PixelProgram.cpp:243-259, PixelRoutine.cpp:317-337, 643-657); the
@@ -606,8 +660,8 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
           if (anyCov) alpha = shade<FCOL, FTEX, XF, FA>(P, rec[tj], px, py, P.color != nullptr).w;
 #pragma unroll
           for (int q = 0; q < MS; q++) {
-            cov[q] = cov[q] && !(alpha < P.a2c[q]);
-            sPass[q] = sPass[q] && cov[q];
+            cov[q] = cov[q] & !(alpha < P.a2c[q]);
+            sPass[q] = sPass[q] & cov[q];
           }
         }
         float zq[MS];
@@ -625,64 +679,53 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
             const float Dz = c + yy * b;
             float z = xx * a + Dz;
             if (depthBias) z = z + zbias;  // PixelRoutine.cpp:141-144, before the clamp
-            z = rr_min(rr_max(z, P.depthClampLo), P.depthClampHi);  // clampDepth
-            if ((XF && P.depth16)) z = d16_value(z);
+            z = rr_min(rr_max(z, range_lo()), range_hi());  // clampDepth
+            if (depth16) z = d16_value(z);
             zq[q] = z;
-            const float zb = S.zb[q];
-            const bool le = zb <= z, lt = zb < z, eq = zb == z;
-            const bool pr = P.zPred == 0 ? le : (P.zPred == 1 ? lt : (P.zPred == 2 ? eq : true));
-            zPass[q] = (stencilActive ? sPass[q] : cov[q]) && pr != (P.zInv != 0);
+            zPass[q] = sPass[q] & zp(S.zb[q], z);
           }
         }
-        if (XF && P.depthBounds) {
+        if (depthBounds) {
           // depthBoundsTest (PixelRoutine.cpp:576-641) on the stored depth, D16
           // as its code / 0xFFFF. With the depth test off the coverage loses
           // the sample while zPass keeps it, so the occlusion count does too.
 #pragma unroll
           for (int q = 0; q < MS; q++) {
-            const float zs = P.depth16 ? S.zb[q] * (1.0f / 65535.0f) : S.zb[q];
-            const bool in = P.depthBoundsMin <= zs && zs <= P.depthBoundsMax;
-            if (depthTest) zPass[q] = zPass[q] && in;
-            else cov[q] = cov[q] && in;
+            const float zs = depth16 ? S.zb[q] * (1.0f / 65535.0f) : S.zb[q];
+            const bool in = (P.depthBoundsMin <= zs) & (zs <= P.depthBoundsMax);
+            if (depthTest) zPass[q] = zPass[q] & in;
+            else cov[q] = cov[q] & in;
           }
         }
         if (stencilWrite) {
 #pragma unroll
           for (int q = 0; q < MS; q++) {
-            const uint32_t bv = S.sb[q];
-            uint32_t nv = stencil_apply_op(bv, SP.pass);
-            const bool zFail = depthTest && sPass[q] && !zPass[q];
-            if (__ballot(zFail)) {
-              const uint32_t v = stencil_apply_op(bv, SP.depthFail);
-              nv = zFail ? v : nv;
-            }
-            if (__ballot(cov[q] && !sPass[q])) {
-              const uint32_t v = stencil_apply_op(bv, SP.fail);
-              nv = sPass[q] ? nv : v;
-            }
-            nv = (nv & SP.writeMask) | (bv & ~SP.writeMask);
-            S.sb[q] = cov[q] ? nv : bv;
+            const uint32_t at = !sPass[q] ? 0u : depthTest & !zPass[q] ? 8u : 16u;
+            S.sb[q] = cov[q] ? st[q] >> at & 255u : S.sb[q];
           }
         }
 #pragma unroll
         for (int q = 0; q < MS; q++) {
           if (depthWrite) S.zb[q] = zPass[q] ? zq[q] : S.zb[q];
-          occl += (unsigned)__builtin_popcountll(__ballot(zPass[q] && sPass[q]));
-          pass[q] = (depthTest ? zPass[q] : cov[q]) && (!stencilActive || sPass[q]);
+          occl += (unsigned)__builtin_popcountll(lanes_where(zPass[q] & sPass[q]));
+          pass[q] = (depthTest ? zPass[q] : cov[q]) & sPass[q];
         }
       }
 
       uint32_t xMask = 0;
 #pragma unroll
       for (int q = 0; q < MS; q++) xMask |= pass[q] ? 1u << q : 0u;
-      const uint64_t need = __ballot(xMask != 0);
+      bool any = false;
+#pragma unroll
+      for (int q = 0; q < MS; q++) any |= pass[q];
+      const uint64_t need = lanes_where(any);
       if (!need) continue;
       if (colorMask) {
         const uint32_t tj = __builtin_amdgcn_readlane(tid, j);
         // Shading is deferred so that it runs with every lane busy: blended
         // fragments queue, others leave their primitive's slot.
         if constexpr (BLEND) {
-          enqueue(xMask != 0, tj, xMask);
+          enqueue(any, tj, xMask);
         } else {
 #pragma unroll
           for (int q = 0; q < MS; q++) S.last[q] = pass[q] ? tj + 1u : S.last[q];
@@ -768,7 +811,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 #pragma unroll
     for (int q = 0; q < MS; q++) {
       if (P.depthWrite) {
-        if ((XF && P.depth16))
+        if (depth16)
           *reinterpret_cast<uint16_t *>(P.depth + q * P.depthSlice + (long long)py * P.depthPitch + 2ll * px) =
               (uint16_t)S.zb[q];
         else
