@@ -470,7 +470,10 @@ int swr_draw(const swr_draw_desc *desc, void *stream);
  * are rendered by the unbinned pass (slower, never dropped).  A draw that
  * leaves room for fewer than 65,536 pairs (about 330,000 primitives)
  * returns SWR_ERROR_UNSUPPORTED.  swr_init(device) locates the device's
- * array; otherwise the first call on that device does. */
+ * array; otherwise the first call on that device does.  The GPU runtime
+ * reserves memory of its own for kernels that spill registers when the first
+ * of them runs (some tens of MiB); a program that cannot have that later runs
+ * one draw of each of its states beforehand. */
 #define SWR_NOALLOC_SCRATCH_BYTES (96u << 20)
 int swr_draw_noalloc(const swr_draw_desc *desc, void *stream);
 

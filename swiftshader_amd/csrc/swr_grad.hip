@@ -71,13 +71,13 @@ constexpr int kMaxBinGroups = 8;
 constexpr uint32_t bin_reserve(bool attr) { return attr ? 512 : 256; }
 // Workgroups of backward_batch_kernel that a CU holds at once (and waves per
 // SIMD, for its registers).  The kernel waits on its fragments' gathers and
-// FP64 chains, so more waves hide more of them as long as their smaller
-// register share holds.  Without attribute gradients (attr) it needs 78 to 95
-// registers and five fit (64-view 4x step 15.8 -> 14.9 ms against the general
-// kernel with two).  With them, records and one sample take three (16-view
-// step 2102 -> 2037 us against two), four samples spill at three (64-view step
-// 17.7 -> 18.2 ms), and the texel tables of the kernels without records fill
-// the LDS at two.
+// FP64 chains, so more waves hide more of them.  Without attribute gradients
+// (attr) it needs 78 to 95 registers and five fit (64-view 4x step 15.8 -> 14.9
+// ms against the general kernel with two).  With them, records and one sample
+// take three: 58 of its registers then spill (168 bytes of scratch a lane) and
+// it is faster all the same (16-view step 2102 -> 2037 us against two, which
+// spill none).  Four samples lose by it (64-view step 17.7 -> 18.2 ms), and the
+// texel tables of the kernels without records fill the LDS at two.
 constexpr int gather_per_cu(int ms, bool bin, bool attr) { return !attr ? 5 : ms == 1 && bin ? 3 : 2; }
 constexpr uint32_t kNoBucket = 0xFFFFFFFFu;           // key of a reserved slot left unused
 
@@ -1345,8 +1345,11 @@ __global__ void mip_up_kernel(float4 *fine, int fw, int fh, int fp, const float4
 // one after the other, with a barrier between (its own writes are visible to
 // it after one).  A level of up to kMipTailTexels takes it some two
 // microseconds, mostly the latency of its loads, a launch of its own over 4 in
-// a replayed graph (16-view step with a 1024^2 texture, both ways of the
-// chain: 1789 -> 1781 us); larger levels need the chip's bandwidth.
+// a replayed graph; larger levels need the chip's bandwidth.  RGBA32F chains, us
+// a call with a launch per level and now (captured: per chain in the graph):
+// 64^2 19 -> 6.8 (12.2 -> 5.2), 256^2 23.4 -> 13.2 (15.9 -> 9.5), 1024^2 28.7 ->
+// 19.7 (21.7 -> 15.6), 2048^2 40.7 -> 28.1 (34.4 -> 29.1); the adjoint at
+// 1024^2 28.7 -> 24.0 (28.0 -> 22.5).
 constexpr uint32_t kMipTailTexels = 4096;  // of the finer level
 constexpr int kMipTailThreads = 1024;
 

@@ -855,6 +855,26 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   }
 }
 
+// Occupancy, in waves per SIMD.  A wave alternates between chains of scalar,
+// LDS and vector work, so another wave pays even where the compiler makes room
+// for it by spilling: up to 52 bytes of scratch a lane in the unblended and up
+// to 68 in the blended kernels of the common states, up to 104 and 160 in the
+// general ones.  At 1280x720 with 30,000 triangles, us a draw here and with one
+// wave less:
+//   one sample, unblended: common states 167 / 170; blended, general: sRGB with
+//   stencil 392 / 413, additive 866 / 971; four samples, unblended: common
+//   256 / 269, general (BGRA) 344 / 370, sRGB 624 / 682; blended: common 548 /
+//   660, sRGB 848 / 930, float colours, whose 16 registers of colour leave them a
+//   wave less, 362 / 425.
+// On targets of a few hundred blocks, which do not fill the waves, the two are
+// within 4 % but for the blended common kernels at 4x (282 / 318).  One wave
+// more: unblended general (BGRA) 195 -> 205 at 6; the blended common kernels lost
+// 7 % at 5 (1080p frame).
+constexpr int raster_waves(int ms, bool floatColor, int level, bool blend) {
+  if (ms == 1) return level == 0 ? 5 : blend ? 4 : 6;
+  return blend ? (floatColor ? 3 : 4) : level == 0 ? 4 : 5;
+}
+
 // A batch of draws: persistent workgroups take global tiles [tileLo, tileHi)
 // from an atomic counter (or, with counter == NULL, workgroup b renders tile
 // tileLo + b once); tile t belongs to the draw d in [drawLo, drawHi) with
@@ -868,20 +888,6 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 // walks its binned list and then those slots, so that one launch does both
 // passes (the tiles of one launch never share pixels, so only the order
 // within a tile matters).
-// Occupancy, in waves per SIMD.  A wave alternates between chains of scalar,
-// LDS and vector work, so more waves pay until registers spill.  With one
-// sample, the unblended kernels of the common states take 6 (16-view step
-// 2050 -> 2015 us against 5, shapes frame 476 -> 469) and the general
-// ones, blended ones included, 5 (sRGB frame 501 -> 468 against 4); the
-// blended ones of the common states 4 (1080p frame 514 us, 549 at 5).  With
-// four, the unblended ones of the common states take 5 (64-view step 18.05 ->
-// 17.56 ms against 4) and the others 4 (4x frame 713 -> 611 against 3), but
-// with float colours to blend, whose 16 registers of colour would spill, 3.
-constexpr int raster_waves(int ms, bool floatColor, int level, bool blend) {
-  if (ms == 1) return level == 0 ? 5 : blend ? 4 : 6;
-  return blend ? (floatColor ? 3 : 4) : level == 0 ? 4 : 5;
-}
-
 template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL, bool BLEND>
 __global__ __launch_bounds__(256, raster_waves(MS, FCOL, LEVEL, BLEND)) void raster_batch_kernel(
                                                            const DrawParams *__restrict__ params,
