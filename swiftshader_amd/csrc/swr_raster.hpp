@@ -270,6 +270,30 @@ __device__ __forceinline__ void store_color(const DrawParams &P, int colorMask, 
 
 constexpr int kQueue = 128;  // deferred-shading queue entries per wave: two batches of 64
 
+// LDS of one wave.  A workgroup has one to four waves (a tile is 8 or 16 pixels
+// a side) and takes one of these for each, dynamically: sized for four, the
+// workgroups of smaller tiles left most of it unused and a CU had five or six of
+// them (1280x720, 30,000 triangles, 8x8 tiles, us a draw: textured and blended
+// 480 -> 339, 4x 1088 -> 559, sRGB with stencil 921 -> 490; 16x8: 317 -> 247,
+// 735 -> 552, 568 -> 424).
+template <int MS, int LEVEL, bool BLEND>
+struct WaveLds {
+  // Without blending, one pixel is one fragment unless it has samples.
+  static constexpr bool kQueued = BLEND || MS > 1;
+  // Chunks of the list that raster_tile loads at a time, and the ring of entries
+  // that wait: at least 63 + 64 * kChunks, a power of two.
+  static constexpr int kChunks = LEVEL == 0 || (MS > 1 && !BLEND) ? 2 : 4;
+  static constexpr uint32_t kRing = 128 * kChunks;
+  int4 cand[3][64];   // a batch of candidates (see raster_tile)
+  int4 candMore[64];  // and the further half planes of polygons
+  float4 qCol[kQueued ? 64 : 1];
+  uint32_t qTri[kQueued ? kQueue : 2];
+  uint32_t qPix[kQueued ? kQueue : 2];
+  uint32_t ring[kRing];
+};
+
+extern __shared__ int4 waveLds[];
+
 // One screen tile of draw P: `bin` is the tile's index in the draw's tile
 // grid, [start, end) its range of the sorted (tile, primitive) list.  The
 // workgroup has one wave per 8x8 block of the tile.
@@ -304,13 +328,12 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   const bool depth16 = XF && P.depth16, depthBounds = XF && P.depthBounds, alphaToCoverage = XF && P.alphaToCoverage;
   // Per-wave queue of fragments that passed the tests and await shading,
   // in API order: primitive, owner lane | sample mask << 8, shaded colour.
-  constexpr bool QUEUE = BLEND || MS > 1;  // without blending, one pixel is one fragment unless it has samples
-  __shared__ uint32_t qTri[QUEUE ? 4 : 1][QUEUE ? kQueue : 1];
-  __shared__ uint32_t qPix[QUEUE ? 4 : 1][QUEUE ? kQueue : 1];
-  __shared__ float4 qCol[QUEUE ? 4 : 1][QUEUE ? 64 : 1];
+  using Lds = WaveLds<MS, LEVEL, BLEND>;
+  constexpr bool QUEUE = Lds::kQueued;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar, as what follows from it: frees up to 14 vector registers
+  Lds &W = reinterpret_cast<Lds *>(waveLds)[wave];
   const int bx = bin % P.tilesX, by = bin / P.tilesX;
   const int bw = P.tileW >> 3;  // 8x8 blocks per tile row
   const int ox = bx * P.tileW + 8 * (wave % bw), oy = by * P.tileH + 8 * (wave / bw);
@@ -413,10 +436,10 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     if constexpr (!QUEUE) return;
     // Shade the queued fragments, one per lane...
     if (lane < qCount) {
-      const uint32_t t = qTri[wave][qHead + lane];
-      const uint32_t pix = qPix[wave][qHead + lane];
+      const uint32_t t = W.qTri[qHead + lane];
+      const uint32_t pix = W.qPix[qHead + lane];
       const int l = (int)(pix & 63u);
-      qCol[wave][lane] = shade<FCOL, FTEX, XF, FA>(P, rec[t], ox + lane_cx(l), oy + lane_cy(l));
+      W.qCol[lane] = shade<FCOL, FTEX, XF, FA>(P, rec[t], ox + lane_cx(l), oy + lane_cy(l));
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -425,12 +448,12 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     while (m) {
       const int k = __builtin_ctzll(m);
       m &= m - 1;
-      const int xMask = MS > 1 ? (int)(qPix[wave][qHead + k] >> 8) : 1;
-      const uint32_t tri = FCOL ? qTri[wave][qHead + k] : 0u;
+      const int xMask = MS > 1 ? (int)(W.qPix[qHead + k] >> 8) : 1;
+      const uint32_t tri = FCOL ? W.qTri[qHead + k] : 0u;
       if constexpr (BLEND)
-        blend_write<MS, FCOL, XF, FAST>(P, S, qCol[wave][k], xMask, tri, srgbLut);
+        blend_write<MS, FCOL, XF, FAST>(P, S, W.qCol[k], xMask, tri, srgbLut);
       else
-        store_color<MS, FCOL, XF>(P, colorMask, px, py, qCol[wave][k], xMask, tri);
+        store_color<MS, FCOL, XF>(P, colorMask, px, py, W.qCol[k], xMask, tri);
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -447,8 +470,8 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     const int pos = qCount + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32),
                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0));
     if (want) {
-      qTri[wave][(qHead + pos) & (kQueue - 1)] = tri;
-      qPix[wave][(qHead + pos) & (kQueue - 1)] = (uint32_t)lane | (xMask << 8);
+      W.qTri[(qHead + pos) & (kQueue - 1)] = tri;
+      W.qPix[(qHead + pos) & (kQueue - 1)] = (uint32_t)lane | (xMask << 8);
       const uint64_t bit = 1ull << (pos & 63);
       mine |= pos < 64 ? bit : 0ull;
       mineNext |= pos < 64 ? 0ull : bit;
@@ -482,8 +505,6 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   // time by the whole wave (a broadcast, which leaves the vector units the
   // arithmetic): half planes 0 to 2 as (f, pk), x0, y0, zA, zB, zC, zBias;
   // half planes 3 and 4 of the polygons that have them.
-  __shared__ int4 cand[4][3][64];
-  __shared__ int4 candMore[4][64];
   int step[MS];  // the pixel's samples from the block's origin, as half_plane's operand
 #pragma unroll
   for (int q = 0; q < MS; q++)
@@ -553,12 +574,12 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
           edge(X.z, Y.z, X.w, Y.w, f[2], pk[2]);
           edge(X.w, Y.w, X4, Y4, m.x, m.y);
           if (n > 4) edge(X4, Y4, X.x, Y.x, m.z, m.w);
-          candMore[wave][lane] = m;
+          W.candMore[lane] = m;
         }
       }
-      cand[wave][0][lane] = make_int4(f[0], pk[0], f[1], pk[1]);
-      cand[wave][1][lane] = make_int4(f[2], pk[2], h3.x, h3.y);
-      cand[wave][2][lane] = make_int4(h3.z, h3.w, h4.x, h4.y);
+      W.cand[0][lane] = make_int4(f[0], pk[0], f[1], pk[1]);
+      W.cand[1][lane] = make_int4(f[2], pk[2], h3.x, h3.y);
+      W.cand[2][lane] = make_int4(h3.z, h3.w, h4.x, h4.y);
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -572,7 +593,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     while (todo) {
       const int j = __builtin_ctzll(todo);
       todo &= todo - 1;
-      const int4 c0 = cand[wave][0][j], c1 = cand[wave][1][j], c2 = cand[wave][2][j];
+      const int4 c0 = W.cand[0][j], c1 = W.cand[1][j], c2 = W.cand[2][j];
       bool cov[MS];
       if (!((spanLanes >> j) & 1)) {
         int in[MS];
@@ -580,7 +601,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
         for (int q = 0; q < MS; q++)
           in[q] = min(min(dot2_i16(c0.y, step[q], c0.x), dot2_i16(c0.w, step[q], c0.z)), dot2_i16(c1.y, step[q], c1.x));
         if ((moreLanes >> j) & 1) {
-          const int4 m = candMore[wave][j];
+          const int4 m = W.candMore[j];
 #pragma unroll
           for (int q = 0; q < MS; q++)
             in[q] = min(min(in[q], dot2_i16(m.y, step[q], m.x)), dot2_i16(m.w, step[q], m.z));
@@ -749,9 +770,8 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
   // chunks are loaded at a time (1080p frame 516 us, 528 with two; the general
   // kernels and the unblended 4x ones take two, for the LDS of their fifth
   // wave per SIMD).
-  constexpr int kChunks = LEVEL == 0 || (MS > 1 && !BLEND) ? 2 : 4;
-  constexpr uint32_t kRing = 128 * kChunks;  // at least 63 + 64 * kChunks; a power of two
-  __shared__ uint32_t ring[4][kRing];
+  constexpr int kChunks = Lds::kChunks;
+  constexpr uint32_t kRing = Lds::kRing;
   uint32_t ringHead = 0, ringCount = 0;  // wave-uniform
   for (uint32_t base = start;;) {
     while (ringCount < 64 && base < end) {
@@ -768,8 +788,8 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
         const bool want = e < end && ((v[u] >> (28 + wave)) & 1u);
         const uint64_t tb = __ballot(want);
         if (want)
-          ring[wave][(ringHead + ringCount +
-                      __builtin_amdgcn_mbcnt_hi((uint32_t)(tb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tb, 0))) &
+          W.ring[(ringHead + ringCount +
+                  __builtin_amdgcn_mbcnt_hi((uint32_t)(tb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tb, 0))) &
                      (kRing - 1)] = v[u] & kSlotMask;
         ringCount += (uint32_t)__builtin_popcountll(tb);
       }
@@ -780,7 +800,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const uint32_t nb = ringCount < 64 ? ringCount : 64;
     const bool act = (uint32_t)lane < nb;
-    const uint32_t t2 = act ? ring[wave][(ringHead + lane) & (kRing - 1)] : 0u;
+    const uint32_t t2 = act ? W.ring[(ringHead + lane) & (kRing - 1)] : 0u;
     ringHead = (ringHead + nb) & (kRing - 1);
     ringCount -= nb;
     process_chunk(act, t2);
@@ -954,7 +974,12 @@ __global__ __launch_bounds__(256, raster_waves(MS, FCOL, LEVEL, BLEND)) void ras
 
 template <int MS, bool FCOL, bool FTEX, bool XF, int LEVEL, bool BLEND>
 void launch_raster_batch(dim3 grid, dim3 block, hipStream_t s, const RasterArgs &a) {
-  hipLaunchKernelGGL((raster_batch_kernel<MS, FCOL, FTEX, XF, LEVEL, BLEND>), grid, block, 0, s, a.params, a.tileBase,
+  // The kernels without a queue gain nothing from more small workgroups a CU,
+  // and long lists lose to them in the caches (16x8 tiles, 30,000 untextured
+  // triangles at 1280x720: 1494 us, 1619 with twice the workgroups).
+  using Lds = WaveLds<MS, LEVEL, BLEND>;
+  const uint32_t lds = (Lds::kQueued ? block.x / 64 : 4) * (uint32_t)sizeof(Lds);
+  hipLaunchKernelGGL((raster_batch_kernel<MS, FCOL, FTEX, XF, LEVEL, BLEND>), grid, block, lds, s, a.params, a.tileBase,
                      a.lo, a.hi, a.tLo, a.tHi, a.counter, a.rec, a.poly, a.bin, a.ts, a.te, a.split, a.segT, a.tail);
 }
 
