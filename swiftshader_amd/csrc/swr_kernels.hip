@@ -211,23 +211,27 @@ struct PolyWork {
   int X[kMaxPolygon], Y[kMaxPolygon];
 };
 
-// Whether polygon X, Y (n >= 3, extents up to 32767) is convex on the 28.4
-// grid, with no repeated vertex: every turn goes the same way or straight on,
-// and the edges change between downward and upward twice (one revolution).
-// The products of 16-bit edges, and the sums of two, fit 32 bits.
-template <int N>
+__device__ __forceinline__ int edge_mul(int a, int b) { return __mul24(a, b); }
+__device__ __forceinline__ long long edge_mul(long long a, long long b) { return a * b; }
+
+// Whether polygon X, Y (n >= 3) is convex on the 28.4 grid, with no repeated
+// vertex: every turn goes the same way or straight on, and the edges change
+// between downward and upward twice (one revolution).  T: int for extents up
+// to 32767 (the products of 16-bit edges, and the sums of two, fit 32 bits),
+// long long for longer ones.
+template <typename T, int N>
 __device__ __forceinline__ bool convex_polygon(const int (&X)[N], const int (&Y)[N], int n) {
   bool left = false, right = false, back = false;
   int changes = 0, dir = 0, firstDir = 0;
-  int dx0 = X[0] - X[n - 1], dy0 = Y[0] - Y[n - 1];
+  T dx0 = X[0] - X[n - 1], dy0 = Y[0] - Y[n - 1];
   for (int i = 0; i < n; i++) {
     const int k = i + 1 < n ? i + 1 : 0;
-    const int dx1 = X[k] - X[i], dy1 = Y[k] - Y[i];
-    const int c = __mul24(dx0, dy1) - __mul24(dy0, dx1);
+    const T dx1 = X[k] - X[i], dy1 = Y[k] - Y[i];
+    const T c = edge_mul(dx0, dy1) - edge_mul(dy0, dx1);
     left |= c > 0;
     right |= c < 0;
     // Straight on, and neither edge of zero length.
-    back |= c == 0 && __mul24(dx0, dx1) + __mul24(dy0, dy1) <= 0;
+    back |= c == 0 && edge_mul(dx0, dx1) + edge_mul(dy0, dy1) <= 0;
     const int s = dy1 > 0 ? 1 : (dy1 < 0 ? -1 : 0);
     changes += s != 0 && firstDir != 0 && s != dir ? 1 : 0;
     firstDir = firstDir ? firstDir : s;
@@ -560,12 +564,14 @@ __device__ __forceinline__ bool setup_one(const DrawParams &P, int t, TriRecord 
   }
   // A triangle is convex; a polygon is when its turns agree.
   const int big = 1 << 20, ext = 32767;
-  bool planes = xLo > -big && xHi < big && yLo > -big && yHi < big && wsub(xHi, xLo) <= ext && wsub(yHi, yLo) <= ext;
+  const bool narrow = wsub(xHi, xLo) <= ext && wsub(yHi, yLo) <= ext;
+  bool planes = xLo > -big && xHi < big && yLo > -big && yHi < big;
   if (planes && n > 3) {
-    if (!POLY) planes = convex_polygon(QX, QY, 4);
-    else planes = n <= kMaxHalfPlanes && convex_polygon(X, Y, n);
+    if (!POLY) planes = narrow ? convex_polygon<int>(QX, QY, 4) : convex_polygon<long long>(QX, QY, 4);
+    else if (n > kMaxHalfPlanes) planes = false;
+    else planes = narrow ? convex_polygon<int>(X, Y, n) : convex_polygon<long long>(X, Y, n);
   }
-  R.nflags = n | (d << 8) | (frontFacing ? 1 << 9 : 0) | (planes ? kRecHalfPlanes : 0);
+  R.nflags = n | (d << 8) | (frontFacing ? 1 << 9 : 0) | (planes ? (narrow ? kRecHalfPlanes : kRecWide) : 0);
   // Tiles are 8 or 16 pixels a side and xMin, yMin >= 0 (scissor-clamped to
   // a render area at x, y >= 0): shifts divide exactly.
   const int sw = __builtin_ctz((uint32_t)P.tileW), sh = __builtin_ctz((uint32_t)P.tileH);

@@ -132,7 +132,7 @@ struct DrawParams {
 // (w plane and attribute planes) is read when fragments are shaded.
 struct TriRecord {
   int nflags;       // bits 0-7: polygon vertex count n (3 unless clipped; 0: culled);
-                    // bit 8: d (winding); bit 9: front facing; bit 10: kRecHalfPlanes
+                    // bit 8: d (winding); bit 9: front facing; bit 10: kRecHalfPlanes; bit 11: kRecWide
   int yMin, yMax;   // rows with possible coverage (scissor-clamped)
   int xMin, xMax;   // pixel columns with possible coverage
   int X[3], Y[3];   // 28.4 polygon vertices when n == 3
@@ -151,6 +151,9 @@ struct TriRecord {
 // (28.4), so that each half plane steps over a block with one 16-bit dot
 // product.
 constexpr int kRecHalfPlanes = 1 << 10;
+// The same with longer edges (below 2^21): half planes in the blocks that no
+// such edge crosses.
+constexpr int kRecWide = 1 << 11;
 constexpr int kMaxHalfPlanes = 5;
 
 static_assert(sizeof(TriRecord) == 160, "TriRecord layout");
