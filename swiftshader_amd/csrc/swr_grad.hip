@@ -72,13 +72,14 @@ constexpr uint32_t bin_reserve(bool attr) { return attr ? 512 : 256; }
 // Workgroups of backward_batch_kernel that a CU holds at once (and waves per
 // SIMD, for its registers).  The kernel waits on its fragments' gathers and
 // FP64 chains, so more waves hide more of them.  Without attribute gradients
-// (attr) it needs 78 to 95 registers and five fit (64-view 4x step 15.8 -> 14.9
-// ms against the general kernel with two).  With them, records and one sample
-// take three: 58 of its registers then spill (168 bytes of scratch a lane) and
-// it is faster all the same (16-view step 2102 -> 2037 us against two, which
-// spill none).  Four samples lose by it (64-view step 17.7 -> 18.2 ms), and the
-// texel tables of the kernels without records fill the LDS at two.
-constexpr int gather_per_cu(int ms, bool bin, bool attr) { return !attr ? 5 : ms == 1 && bin ? 3 : 2; }
+// (attr) it needs 78 to 95 registers; with four samples five waves pay (backward
+// of 32 views of 512x512: 3311 us with two, 3130 with three, 2999), with one
+// sample three (1322, 1245; five 1248).  With attribute gradients, records and
+// one sample take three: 58 of its registers then spill (168 bytes of scratch a
+// lane) and it is faster all the same (2059 -> 1817 us against two, which spill
+// none).  Four samples lose by it (64-view step 17.7 -> 18.2 ms), and the texel
+// tables of the kernels without records fill the LDS at two.
+constexpr int gather_per_cu(int ms, bool bin, bool attr) { return !attr ? (ms == 1 ? 3 : 5) : ms == 1 && bin ? 3 : 2; }
 constexpr uint32_t kNoBucket = 0xFFFFFFFFu;           // key of a reserved slot left unused
 
 // Footprint of one fragment: texture coordinate, frozen sampling state and
