@@ -1261,18 +1261,31 @@ __global__ __launch_bounds__(kScatterThreads) void tap_scatter_kernel(const TapR
           } else {
             // Some taps lie outside the region (all, for an item that adds in
             // float): those go straight to the gradient buffer, the others to
-            // their cells.
+            // their cells.  Mostly all four lie outside; a loop over the taps for
+            // these as well cost 3 % at 16 probes.
+            const int x0 = bin_texel_axis(au.r0, ox, W, addrU == 0), x1 = bin_texel_axis(au.r1, ox, W, addrU == 0);
+            const int y0 = bin_texel_axis(av.r0, oy, H, addrV == 0), y1 = bin_texel_axis(av.r1, oy, H, addrV == 0);
+            // The copy of the second tap's texel that a cell may stand for.
+            const int u1 = addrU == 0 && au.r1 >= W ? au.r1 - W : au.r1, v1 = addrV == 0 && av.r1 >= H ? av.r1 - H : av.r1;
+            const bool ux = (unsigned)au.r0 < (unsigned)side || (unsigned)u1 < (unsigned)side;
+            const bool vy = (unsigned)av.r0 < (unsigned)side || (unsigned)v1 < (unsigned)side;
+            if (!(ux && vy)) {
+              if (g) {
+                add_texel(g, pitch, x0, y0, r.g, (float)w00);
+                add_texel(g, pitch, x1, y0, r.g, (float)w10);
+                add_texel(g, pitch, x0, y1, r.g, (float)w01);
+                add_texel(g, pitch, x1, y1, r.g, (float)w11);
+              }
+              continue;
+            }
 #pragma nounroll
             for (int k = 0; k < 4; k++) {
-              int rx = k & 1 ? au.r1 : au.r0, ry = k & 2 ? av.r1 : av.r0;
-              if (addrU == 0 && rx >= W) rx -= W;  // the copy that a cell may stand for
-              if (addrV == 0 && ry >= H) ry -= H;
+              const int rx = k & 1 ? u1 : au.r0, ry = k & 2 ? v1 : av.r0;
               const double w = k & 2 ? (k & 1 ? w11 : w01) : (k & 1 ? w10 : w00);
               if ((unsigned)rx < (unsigned)side && (unsigned)ry < (unsigned)side)
                 add(Rq + base + ry * side + rx, w);
               else if (g)
-                add_texel(g, pitch, bin_texel_axis(rx, ox, W, addrU == 0), bin_texel_axis(ry, oy, H, addrV == 0), r.g,
-                          (float)w);
+                add_texel(g, pitch, k & 1 ? x1 : x0, k & 2 ? y1 : y0, r.g, (float)w);
             }
           }
         }
