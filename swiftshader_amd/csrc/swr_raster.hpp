@@ -585,19 +585,11 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
       W.cand[0][lane] = make_int4(f[0], pk[0], f[1], pk[1]);
       W.cand[1][lane] = make_int4(f[2], pk[2], h3.x, h3.y);
       W.cand[2][lane] = make_int4(h3.z, h3.w, h4.x, h4.y);
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    uint64_t todo = __ballot(act);
-    uint64_t spanLanes = __ballot(act && !(nflags & kRecHalfPlanes));
-    const uint64_t wideLanes = __ballot(act && (nflags & kRecWide));
-    if (__builtin_expect(wideLanes != 0, 0)) {
-      bool spans = !(nflags & (kRecHalfPlanes | kRecWide));
-      if (act && (nflags & kRecWide)) {
+      if (__builtin_expect((nflags & kRecWide) != 0, 0)) {
         const int *X = reinterpret_cast<const int *>(rec + tid) + offsetof(TriRecord, X) / 4;
-        const int n = nflags & 0xFF;
         if (n != 3) X = poly + (size_t)tid * (2 * kMaxPolygon);
         const int *Y = X + (n == 3 ? 3 : kMaxPolygon);
+        bool crossed = false;
 #pragma nounroll
         for (int i = 0; i < n; i++) {
           int *h = i < 2 ? &W.cand[0][lane].x + 2 * i : i == 2 ? &W.cand[1][lane].x : &W.candMore[lane].x + 2 * (i - 3);
@@ -605,14 +597,15 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
           const int ex = abs(X[k] - X[i]), ey = abs(Y[k] - Y[i]), reach = (ex + ey) * 128;  // below 2^29
           if (h[0] < -reach) act = false;
           else if (h[0] > reach) h[1] = 0;
-          else spans |= max(ex, ey) > 32767;
+          else crossed |= max(ex, ey) > 32767;
         }
+        if (crossed) nflags &= ~kRecWide;
       }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      todo = __ballot(act);
-      spanLanes = __ballot(act && spans);
     }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    uint64_t todo = __ballot(act);
+    const uint64_t spanLanes = __ballot(!(nflags & (kRecHalfPlanes | kRecWide)));
     const uint64_t moreLanes = __ballot((nflags & 0xFF) > 3);
     const uint64_t frontLanes = SIMPLE ? 0ull : __ballot((nflags >> 9) & 1);
     int wrote = 0;
