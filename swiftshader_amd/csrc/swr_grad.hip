@@ -1090,6 +1090,24 @@ __device__ __forceinline__ void add_texel(float *g, int pitch, int x, int y, con
   if (d != 0.0f) gadd(o + 3, d);
 }
 
+// On a wrapping axis of fewer than 8 texels, up to 8 cells stand for one texel
+// (those of axis_cells end at max(dim, kBinHalo0)).  Moves their sums into the
+// first dim cells, so that the flush adds a texel once: every work item adds the
+// texels of the smallest levels, and atomics to one address take turns (8 views
+// of 512x512, a texture of 4x4: backward 420 -> 383 us).
+constexpr int kFoldDim = 8;
+static_assert(kBinHalo0 < kFoldDim && kBinHalo1 < kFoldDim, "cells that a short axis reaches");
+__device__ __forceinline__ void bin_fold(long long *regions, int base, int side, int dim, int step, int across) {
+  for (int i = threadIdx.x; i < side * 4; i += blockDim.x) {
+    long long *c = regions + base + (i & 3) * kBinCells + (i >> 2) * across;
+    for (int r = dim, t = 0; r < kFoldDim; r++, t = t + 1 < dim ? t + 1 : 0) {
+      c[t * step] += c[r * step];
+      c[r * step] = 0;
+    }
+  }
+  __syncthreads();
+}
+
 // Adds the nonzero cells of a region (divided by S: times invS) to the
 // gradient buffer and clears them.
 __device__ __forceinline__ void bin_flush(long long *regions, int base, int side, int ox, int oy, int w, int h,
@@ -1293,6 +1311,11 @@ __global__ __launch_bounds__(kScatterThreads) void tap_scatter_kernel(const TapR
     }
     __syncthreads();
     if (fixed) {
+      // (Uniform.)
+      if (addrU == 0 && W0 < kFoldDim) bin_fold(Rq, 0, kBinR0, W0, 1, kBinR0);
+      if (addrV == 0 && H0 < kFoldDim) bin_fold(Rq, 0, kBinR0, H0, kBinR0, 1);
+      if (addrU == 0 && W1 < kFoldDim) bin_fold(Rq, kR1At, kBinR1, W1, 1, kBinR1);
+      if (addrV == 0 && H1 < kFoldDim) bin_fold(Rq, kR1At, kBinR1, H1, kBinR1, 1);
       bin_flush(Rq, 0, kBinR0, ox0, oy0, W0, H0, addrU == 0, addrV == 0, g0, P0, invS);
       bin_flush(Rq, kR1At, kBinR1, ox1, oy1, W1, H1, addrU == 0, addrV == 0, g1, P1, invS);
     }

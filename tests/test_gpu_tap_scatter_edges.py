@@ -13,11 +13,11 @@ import pytest
 import torch
 
 from grad_cases import G, params_of, view_of
-from swiftshader_amd import abi
+from swiftshader_amd import abi, diff
 from swiftshader_amd.batch import BatchPlan, grad_desc
 from swiftshader_amd.scenes import DrawData, TextureData
 from test_gpu_grad import _t, gpu_forward
-from swiftshader_amd import diff
+from test_gpu_tap_scatter import test_binned_scatter_matches_per_view as matches_per_view
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -95,3 +95,11 @@ def test_a_gradient_that_is_not_finite_stays_in_its_footprint(value):
     assert touched.sum() == 8 and not touched[..., [0, 1, 3]].any()
     assert not np.isfinite(got[touched]).any()
     assert np.abs(got - want)[~touched].max() < 64 * 2.0**-24 * want.max()
+
+
+@pytest.mark.parametrize("mode", [abi.ADDRESS_REPEAT, abi.ADDRESS_CLAMP_TO_EDGE])
+@pytest.mark.parametrize("size", [(1, 3), (3, 5), (5, 6), (7, 2), (6, 8), (8, 7), (9, 4)])
+@pytest.mark.parametrize("aniso", [False, True])
+def test_levels_of_fewer_than_eight_texels(size, mode, aniso):
+    """Several cells of a wrapping level of fewer than 8 texels stand for one texel."""
+    matches_per_view(size, mode, abi.FILTER_LINEAR, aniso, 4 if aniso else 1, size[0] == 5)
