@@ -899,7 +899,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &P, int bin, uint32
 // Occupancy, in waves per SIMD.  A wave alternates between chains of scalar,
 // LDS and vector work, so another wave pays even where the compiler makes room
 // for it by spilling: up to 52 bytes of scratch a lane in the unblended and up
-// to 68 in the blended kernels of the common states, up to 104 and 160 in the
+// to 60 in the blended kernels of the common states, up to 100 and 144 in the
 // general ones.  At 1280x720 with 30,000 triangles, us a draw here and with one
 // wave less:
 //   one sample, unblended: common states 167 / 170; blended, general: sRGB with
